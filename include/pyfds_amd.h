@@ -158,7 +158,8 @@ int fds_run_take(fds_ctx *ctx, double *dst0, double *dst1, double *dst2);
 int fds_prepare_run(fds_ctx *ctx, int64_t start_step, int64_t nsteps, int chunk);
 
 /* Tile shape of the 2D step kernels (autotuner hook): index into the compiled shape table,
- * or -1 for the default.  fds_tile_count reports the table size, fds_tile_shape its entries
+ * or -1 for the default: lossless 2D fields run the fused engine (one-wave strips, up to six
+ * steps per launch, height by fds_set_strip_height), which has no entry in the table.  fds_tile_count reports the table size, fds_tile_shape its entries
  * (tx columns x ty rows).  fds_tile_engine returns 0 for an LDS-tile shape and 1 for a
  * row-streaming shape (a workgroup of tx threads marching down a strip of ty rows); streaming
  * shapes serve the 2D models (lossy acoustics one time step per launch on any of them).
@@ -177,7 +178,8 @@ int fds_tile_engine(int tile_index);
  * start on 16-byte boundaries runs the same tiling with register loads) of a shape.  Shapes
  * with a prefetch depth above 1 serve single lossless fields only. */
 int fds_tile_traits(int tile_index, int *steps, int *nontemporal, int *prefetch, int *lds_ring);
-/* Strip height (rows per workgroup) of a streaming shape; 0 restores the shape's own height.
+/* Strip height (rows per workgroup) of a streaming shape or of the fused engine (at most 512);
+ * 0 restores the shape's own height, or the one chosen from the grid.
  * Ignored by LDS-tile shapes.  For the resident 1D engine the value is the number of cells per
  * thread (1, 2, 4 or 8; 0 = chosen from the line length). */
 int fds_set_strip_height(fds_ctx *ctx, int rows);

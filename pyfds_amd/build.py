@@ -3,7 +3,8 @@
     python -m pyfds_amd.build          # or pyfds_amd.build.build()
 
 Compiles every ``pyfds_amd/csrc/*.hip`` translation unit in parallel with hipcc (the
-streaming kernels' ``fds_stream_tu.hip`` once per numeric form and streaming shape) and links
+streaming kernels' ``fds_stream_tu.hip`` once per numeric form and streaming shape, the
+fused kernels' ``fds_fused_tu.hip`` once per form and stage count) and links
 them into ``pyfds_amd/_lib/libpyfds_amd.so``.  The library is compiled with
 ``-ffp-contract=off`` so the float64 kernels round every product and sum exactly where the
 reference's numpy/scipy code does, and with packed-FP32 instructions disabled.
@@ -27,13 +28,15 @@ FLAGS = ['-O3', '-std=c++17', '--offload-arch=' + ARCH, '-fPIC', '-ffp-contract=
 
 
 STREAM_TU = 'fds_stream_tu.hip'
+FUSED_TU = 'fds_fused_tu.hip'
 
 
-def _num_stream_shapes():
+def _constant(name):
+    """An integer constant of the kernel tables' header."""
     with open(os.path.join(CSRC, 'fds_kernels.h')) as f:
-        m = re.search(r'kNumStream\s*=\s*(\d+)', f.read())
+        m = re.search(name + r'\s*=\s*(\d+)', f.read())
     if not m:
-        raise RuntimeError('kNumStream not found in fds_kernels.h')
+        raise RuntimeError(name + ' not found in fds_kernels.h')
     return int(m.group(1))
 
 
@@ -57,15 +60,18 @@ def build(verbose=True):
     objdir = os.path.join(HERE, '_build')
     os.makedirs(objdir, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
-    srcs = sorted(f for f in os.listdir(CSRC) if f.endswith('.hip') and f != STREAM_TU)
-    # (source, object, defines): the streaming kernels once per form and shape
+    srcs = sorted(f for f in os.listdir(CSRC) if f.endswith('.hip') and f not in (STREAM_TU, FUSED_TU))
+    # (source, object, defines)
     units = [(f, f[:-4] + '.o', ()) for f in srcs]
     for form in range(3):
-        for shape in range(_num_stream_shapes()):
+        for shape in range(_constant('kNumStream')):
             units.append((STREAM_TU, 'fds_stream_f%d_s%d.o' % (form, shape),
                           ('FDS_FORM=%d' % form, 'FDS_SHAPE=%d' % shape)))
+        for stages in range(1, _constant('kFusedMax') + 1):
+            units.append((FUSED_TU, 'fds_fused_f%d_s%d.o' % (form, stages),
+                          ('FDS_FORM=%d' % form, 'FDS_STAGES=%d' % stages)))
     # longest first: the streaming units dominate
-    units.sort(key=lambda u: u[0] != STREAM_TU)
+    units.sort(key=lambda u: u[0] not in (STREAM_TU, FUSED_TU))
     jobs = {}
     with cf.ThreadPoolExecutor(max_workers=min(os.cpu_count() or 8, 16, len(units))) as pool:
         for f, o, d in units:

@@ -190,6 +190,14 @@ struct fds_ctx {
   int ghost = 0;          // ghost columns per side of a streaming tile (fuse - 1; lossy: 1)
   int ghost_rows = 0;     // ghost rows per side of a streaming strip (fuse - 1; lossy: 0)
   int sx = 0;             // x stride of the tiles (tx - 2*ghost)
+  bool fused = false;     // fused engine in use (a row-streaming engine: streaming is set too)
+  bool coupled = false;   // stepped one step per launch by a coupling (until the next commit)
+  bool fused_over = false;   // the event lists do not fit the fused engine's tile classes
+  DevBuf fev_slot, fev_words, fev_cls_ptr, fev_cls, fev_points,
+      fev_point_rows, fev_tiles;     // its event tables (fds::FusedEv)
+  int fev_rows = 0, fev_nslots = 0;
+  DevBuf pal_idx, pal;    // material classes of the cells and their coefficients
+  int npal = 0;           // classes, the zero class included (0: none known)
   bool line = false;      // resident 1D engine in use (one workgroup, many steps per launch)
   int line_var = 0;       // its variant: index into fds::kLineCpt
   int line_threads = 0;   // its workgroup size
@@ -370,6 +378,15 @@ bool can_stream(const fds_ctx *c) {
 
 bool can_stream_batch(const fds_ctx *c) { return can_stream(c) && !c->lossy; }
 
+// The fused engine covers the lossless 2D models whose arrays a buffer descriptor spans (32-bit
+// byte offsets, rows past either end included).
+bool can_fuse(const fds_ctx *c) {
+  const bool lossy = c->lossy && c->family == kAcoustic;
+  const int64_t reach = c->n + (fds::kFusedStrip + 4 * fds::kFusedMax) * c->nx + 1024;
+  return can_stream(c) && !lossy && !c->fused_over &&
+         reach * (int64_t)c->elem < (int64_t)1 << 32;
+}
+
 // Resident 1D engine variant for n cells: `cpt` cells per thread if given, else the fewest
 // cells per thread that fit (the most threads: a step is bound by the one CU's issue rate, so
 // spreading the line over more waves wins; measured on 2000 cells: 0.59 us per step with 2
@@ -383,8 +400,44 @@ int line_variant(int64_t n, int cpt, int fam) {
   return -1;
 }
 
+// Layout of the fused engine: stages per launch and strip height.
+//
+// Stages: a launch's time grows slowly with them (2048^2 FP64 acoustics: 36 us at 4, 42 us at 6),
+// so all kFusedMax, except on small grids, where a launch is bound by the latency of one strip
+// and the iterations it takes: 401 x 301 FP64 2.5 us a step at 4 stages, 2.6 at 6; from 800 x 600
+// on 6 are ahead (FP64 3.0 and 2.9).  One where something follows every step.
+//
+// Height: short strips make enough waves to fill the chip, tall ones waste fewer ghost rows
+// (2S a strip).  About 24 strips a CU are two rounds of resident waves, and measured best or
+// within 3 % of it from 1024 x 1536 (4-6 rows) over 2048^2 (12) to 4096 x 3000 (24-48).
+int choose_fused(fds_ctx *c) {
+  const bool each = c->lbc_w1 || c->flow || c->coupled;
+  const int S = each ? 1 : c->n < (1 << 18) ? 4 : fds::kFusedMax;
+  const int64_t sx = 64 - 2 * S, across = (c->nx + sx - 1) / sx;
+  const int64_t want = (across * c->ny + 12 * (int64_t)c->num_cu) / (24 * (int64_t)c->num_cu);
+  const int H = c->strip_rows > 0 ? std::min(c->strip_rows, fds::kFusedStrip)
+                                  : (int)std::min<int64_t>(std::max<int64_t>(want, 4), 64);
+  c->fused = c->streaming = true;
+  c->fuse = S;
+  c->ghost = S;
+  c->ghost_rows = S - 1;
+  c->tx = 64;
+  c->ty = H;
+  c->sx = 64 - 2 * S;
+  c->shape = fds::kDefaultLossless2D;
+  c->tiles_x = (int)((c->nx + c->sx - 1) / c->sx);
+  c->tiles_y = (int)((c->ny + c->ty - 1) / c->ty);
+  const int64_t nt = (int64_t)c->tiles_x * c->tiles_y;
+  if (nt > (int64_t)std::numeric_limits<int32_t>::max() / 2)
+    return fail(FDS_E_ARG, "grid too large for the tile index (%lld tiles)", (long long)nt);
+  c->ntiles = (int)nt;
+  c->events_dirty = true;
+  return 0;
+}
+
 int choose_tiles(fds_ctx *c) {
   c->streaming = false;
+  c->fused = false;
   c->line = false;
   c->fuse = 1;
   c->ghost = 0;
@@ -446,6 +499,7 @@ int choose_tiles(fds_ctx *c) {
     c->ty = 1;
     c->shape = 0;
   } else {
+    if (c->tile < 0 && can_fuse(c)) return choose_fused(c);
     int t = c->tile;
     if (t < 0) t = (c->ny == 1) ? fds::kTileRow : (c->lossy ? fds::kDefaultLossy2D
                                                              : fds::kDefaultLossless2D);
@@ -555,8 +609,109 @@ void build_line_heads(const Comp &cp, const Events &ev, const Events &oe, int nt
   }
 }
 
+// Event tables of the fused engine (fds::FusedEv) from the components' boundary event lists
+// `bev` and output event lists `oev`.  Boundary programs become classes: a tile's distinct
+// programs, each a chain of entries.  Returns 1 when some tile has more entries than the kernels
+// hold (the caller then leaves the fused engine).
+int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
+  const int rows = c->ty + 2 * c->fuse, g = c->ghost_rows + 1;
+  std::vector<int32_t> slot(c->ntiles, -1), cls_ptr(1, 0), tiles;
+  std::vector<uint32_t> words;
+  std::vector<fds::FusedClass> cls;
+  std::vector<fds::FusedPoint> points;
+  std::vector<int32_t> point_rows;
+  // distinct programs of each component, by their entries
+  std::vector<int32_t> prog[3];
+  std::vector<std::pair<int32_t, int32_t>> first[3];   // entries of a distinct program
+  for (int k = 0; k < 3; ++k) {
+    const Comp &cp = c->comp[k];
+    std::map<std::vector<int64_t>, int32_t> seen;
+    std::vector<int64_t> key;
+    for (size_t u = 0; u < cp.cells.size(); ++u) {
+      key.clear();
+      for (int32_t e = cp.ptr[u]; e < cp.ptr[u + 1]; ++e) {
+        int64_t bits;
+        std::memcpy(&bits, &cp.a[e], 8);
+        key.insert(key.end(), {bits, cp.off[e], cp.stride[e]});
+      }
+      const auto it = seen.emplace(key, (int32_t)first[k].size());
+      if (it.second) first[k].push_back({cp.ptr[u], cp.ptr[u + 1]});
+      prog[k].push_back(it.first->second);
+    }
+  }
+  int nslots = 0;
+  std::map<std::pair<int32_t, int32_t>, int32_t> local;   // (component, program) -> entry
+  for (int t = 0; t < c->ntiles; ++t) {
+    bool any = false;
+    for (int k = 0; k < 3; ++k)
+      any = any || bev[k].ptr[t + 1] > bev[k].ptr[t] || oev[k].ptr[t + 1] > oev[k].ptr[t];
+    if (!any) continue;
+    slot[t] = nslots++;
+    tiles.push_back(t);
+    words.resize((size_t)nslots * rows * 64, 0u);
+    uint32_t *w = words.data() + (size_t)(nslots - 1) * rows * 64;
+    local.clear();
+    const size_t base = cls.size();
+    for (int k = 0; k < 3; ++k) {
+      const Region R = region_of(c, k);
+      for (int32_t e = bev[k].ptr[t]; e < bev[k].ptr[t + 1]; ++e) {
+        const int r = bev[k].pos[e] / R.w + R.rmin + g, col = bev[k].pos[e] % R.w + R.cmin;
+        if (r < 0 || r >= rows || col < 0 || col >= 64) continue;
+        const int32_t p = prog[k][bev[k].id[e]];
+        const auto it = local.emplace(std::make_pair(k, p), (int32_t)(cls.size() - base + 1));
+        if (it.second) {
+          const auto [e0, e1] = first[k][p];
+          for (int32_t q = e0; q < e1; ++q)
+            cls.push_back(fds::FusedClass{c->comp[k].a[q], c->comp[k].off[q],
+                                          c->comp[k].stride[q], k,
+                                          q + 1 < e1 ? (int32_t)(cls.size() - base + 2) : 0});
+          if (cls.size() - base >= (size_t)fds::kFusedClasses) return 1;
+        }
+        w[r * 64 + col] |= (uint32_t)it.first->second << (8 * k);
+      }
+      // recorded points: owned cells, the list is sorted by row
+      int32_t e = oev[k].ptr[t];
+      for (int r = 0; r <= c->ty; ++r) {
+        point_rows.push_back((int32_t)points.size());
+        for (; e < oev[k].ptr[t + 1] && oev[k].pos[e] / R.w + R.rmin == r; ++e) {
+          const int col = oev[k].pos[e] % R.w + R.cmin;
+          points.push_back(fds::FusedPoint{col, oev[k].id[e]});
+          w[(r + g) * 64 + col] |= fds::kFusedRecord << k;
+        }
+      }
+    }
+    cls_ptr.push_back((int32_t)cls.size());
+  }
+  c->fev_rows = rows;
+  c->fev_nslots = nslots;
+  HIP_TRY(upload(c->fev_tiles, tiles, c->stream));
+  HIP_TRY(upload(c->fev_slot, slot, c->stream));
+  HIP_TRY(upload(c->fev_words, words, c->stream));
+  HIP_TRY(upload(c->fev_cls_ptr, cls_ptr, c->stream));
+  HIP_TRY(upload(c->fev_cls, cls, c->stream));
+  HIP_TRY(upload(c->fev_points, points, c->stream));
+  HIP_TRY(upload(c->fev_point_rows, point_rows, c->stream));
+  return 0;
+}
+
 int rebuild_events(fds_ctx *c) {
   if (!c->events_dirty) return 0;
+  if (c->fused) {
+    Events bev[3], oev[3];
+    for (int k = 0; k < 3; ++k) {
+      build_bound_events(c, k, bev[k]);
+      build_output_events(c, k, oev[k]);
+    }
+    const int rc = build_fused_events(c, bev, oev);
+    if (rc < 0) return rc;
+    if (rc == 0) {
+      c->events_dirty = false;
+      touch(c);
+      return 0;
+    }
+    c->fused_over = true;    // until the boundaries change
+    if (int rc2 = choose_tiles(c)) return rc2;
+  }
   std::vector<int32_t> zp(c->ntiles + 1, 0);
   HIP_TRY(upload(c->zero_ptr, zp, c->stream));
   for (int k = 0; k < 3; ++k) {
@@ -647,12 +802,29 @@ void fill_args(const fds_ctx *c, fds::StepArgs<T> &a, int parity) {
   a.flags = (c->iso_b ? fds::kFlagIsoB : 0) | (c->iso_k ? fds::kFlagIsoK : 0);
   a.strip_h = c->ty;
   a.ghost = c->ghost;
+  a.ghost_rows = c->ghost_rows;
+  a.sx = c->sx;
+  if (c->fused) {
+    a.fev = fds::FusedEv{c->fev_slot.as<const int32_t>(), c->fev_tiles.as<const int32_t>(),
+                         c->fev_words.as<const uint32_t>(),
+                         c->fev_cls_ptr.as<const int32_t>(),
+                         c->fev_cls.as<const fds::FusedClass>(),
+                         c->fev_points.as<const fds::FusedPoint>(),
+                         c->fev_point_rows.as<const int32_t>(), c->fev_rows, c->fev_nslots};
+    a.pal_idx = c->pal_idx.as<const uint8_t>();
+    a.pal = c->pal.as<const T>();
+    a.npal = c->npal;
+  }
 }
 
 // ring_ok: the arrays suit an LDS-ring shape's 16-byte row loads (else its register-path twin
 // runs, same bits).
 fds::LaunchFn pick_launch(const fds_ctx *c, int stages, bool ring_ok = true) {
   const int t = c->shape;
+  if (c->fused) {
+    const int v = c->axi ? 1 : (c->iso_b && c->iso_k) ? 2 : 0;
+    return c->ks->fused[c->family == kThermal ? 1 : 0][c->npal > 0 ? 1 : 0][v][stages - 1];
+  }
   if (c->streaming && c->lossy) {
     // variant: axial-symmetric, isotropic (B, K and M y slots alias the x ones), plain
     const int v = c->axi ? 1 : (c->iso_b && c->iso_k && !c->coef_set[FDS_C_MY]) ? 2 : 0;
@@ -786,7 +958,7 @@ int launch_step(fds_ctx *c, int parity, int k, bool store, int stages) {
   a.k = k;
   if (store) a.flags |= fds::kFlagStore;
   bool ring_ok = true;
-  if (c->streaming && fds::kStreamShapes[c->shape - fds::kNumTiles][5]) {
+  if (c->streaming && !c->fused && fds::kStreamShapes[c->shape - fds::kNumTiles][5]) {
     // LDS-ring kernels load 16-byte chunks of rows: rows must start on 16-byte boundaries and
     // every array they read must be 16-byte aligned (whole device allocations are); otherwise
     // the register-path kernel of the same tiling runs
@@ -795,7 +967,7 @@ int launch_step(fds_ctx *c, int parity, int k, bool store, int stages) {
       ring_ok = ring_ok && ((uintptr_t)a.in[k] & 15) == 0 && ((uintptr_t)a.cin[k] & 15) == 0;
     for (int q = 0; q < FDS_NUM_COEFF; ++q) ring_ok = ring_ok && ((uintptr_t)a.coef[q] & 15) == 0;
   }
-  const int nb = fds::xcd_grid(c->ntiles);
+  const int nb = fds::xcd_grid(c->ntiles) + (c->fused ? fds::xcd_grid(c->fev_nslots) : 0);
   pick_launch(c, stages, ring_ok)(&a, nb, lds_bytes(c), c->stream);
   HIP_TRY(hipGetLastError());
   if (c->flow) {
@@ -923,6 +1095,76 @@ int get_graph(fds_ctx *c, int chunk, int parity, hipGraphExec_t *out) {
   // the graph's device-side copy now, not on its first launch inside a run
   HIP_TRY(hipGraphUpload(ex, c->stream));
   *out = ex;
+  return 0;
+}
+
+// Material classes.  Cells with the same coefficients (slots 0-3, by their bits) are one class;
+// a field whose cells form fewer than kPalMax classes gets an array of class numbers, one byte a
+// cell, and a table of the classes' coefficients.  Pass q compares every cell without a class to
+// the first such cell (`first[q]`, found by the pass before), gives the equal ones class q + 1
+// and finds the first cell left.
+template <typename T>
+__global__ __launch_bounds__(256) void k_pal_pass(const T *c0, const T *c1, const T *c2,
+                                                  const T *c3, int64_t n, uint8_t *idx, T *pal,
+                                                  unsigned *first, int q) {
+  using B = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
+  const unsigned f = first[q];
+  if (f == ~0u) return;
+  const T *c[4] = {c0, c1, c2, c3};
+  B b[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) b[k] = __builtin_bit_cast(B, c[k][f]);
+  // table columns: x factor of the backward and of the forward difference, then the y factors
+  if (blockIdx.x == 0 && threadIdx.x < 4)
+    pal[(q + 1) * 4 + threadIdx.x] = c[(threadIdx.x & 1) ? threadIdx.x >> 1 : 2 + (threadIdx.x >> 1)][f];
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  unsigned left = ~0u;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
+    if (q > 0 && idx[i]) continue;
+    bool eq = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) eq = eq && __builtin_bit_cast(B, c[k][i]) == b[k];
+    if (eq) idx[i] = (uint8_t)(q + 1);
+    else {
+      if (q == 0) idx[i] = 0;
+      if (left == ~0u) left = (unsigned)i;
+    }
+  }
+  for (int d = 32; d > 0; d >>= 1) left = min(left, (unsigned)__shfl_xor((int)left, d));
+  if ((threadIdx.x & 63) == 0 && left != ~0u) atomicMin(first + q + 1, left);
+}
+
+template <typename T>
+int find_classes(fds_ctx *c) {
+  c->npal = 0;
+  const T *cf[4];
+  for (int k = 0; k < 4; ++k)
+    cf[k] = c->coef_set[k] ? c->coef[k].as<const T>() : c->coef[k - 1].as<const T>();
+  DevBuf first;
+  HIP_TRY(c->pal_idx.ensure(c->n));
+  HIP_TRY(c->pal.ensure(fds::kPalMax * 4 * sizeof(T)));
+  std::vector<unsigned> f(fds::kPalMax + 1, ~0u);
+  f[0] = 0;
+  HIP_TRY(upload(first, f, c->stream));
+  HIP_TRY(hipMemsetAsync(c->pal.p, 0, fds::kPalMax * 4 * sizeof(T), c->stream));
+  const unsigned nb = (unsigned)std::min<int64_t>((c->n + 1023) / 1024, 2048);
+  const int most = fds::kPalMax - 1;
+  for (int q = 0; q < most;) {
+    const int q1 = std::min(q + 4, most);
+    for (; q < q1; ++q)
+      hipLaunchKernelGGL(k_pal_pass<T>, dim3(nb), dim3(256), 0, c->stream, cf[0], cf[1], cf[2],
+                         cf[3], c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(),
+                         first.as<unsigned>(), q);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(f.data(), first.p, f.size() * sizeof(unsigned), hipMemcpyDeviceToHost,
+                           c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (f[q] == ~0u) {
+      while (q > 1 && f[q - 1] == ~0u) --q;
+      c->npal = q + 1;
+      return 0;
+    }
+  }
   return 0;
 }
 
@@ -1144,6 +1386,7 @@ int fds_commit(fds_ctx *c) {
   } else {
     if (!c->coef_set[FDS_C_RHO0]) return fail(FDS_E_STATE, "static density must be set");
   }
+  c->coupled = false;
   c->iso_b = !c->one_d && !c->coef_set[FDS_C_BY];   // (thermal: QY)
   c->iso_k = !c->one_d && !c->coef_set[FDS_C_KY];   // (thermal: GY)
   if (c->family != kNonlinear) {
@@ -1155,6 +1398,10 @@ int fds_commit(fds_ctx *c) {
       c->tile = -1;
       if (int rc = choose_tiles(c)) return rc;
     }
+  }
+  c->npal = 0;
+  if (c->fused) {
+    if (int rc = c->elem == 8 ? find_classes<double>(c) : find_classes<float>(c)) return rc;
   }
   c->committed = true;
   touch(c);
@@ -1239,6 +1486,10 @@ int fds_set_boundaries(fds_ctx *c, int comp, int64_t ncell, const int64_t *cells
   HIP_TRY(upload(cp.d_off, cp.off, c->stream));
   HIP_TRY(upload(cp.d_stride, cp.stride, c->stream));
   HIP_TRY(upload(cp.d_table, cp.table, c->stream));
+  if (c->fused_over) {
+    c->fused_over = false;
+    if (int rc = choose_tiles(c)) return rc;
+  }
   c->events_dirty = true;
   touch(c);
   return 0;
@@ -1723,6 +1974,7 @@ int fds_set_flow(fds_ctx *c, const int64_t *period, int64_t nrows) {
   if (int rc = check_idle(c)) return rc;
   if (!period || nrows == 0) {
     c->flow = false;
+    if (int rc = choose_tiles(c)) return rc;
     touch(c);
     return 0;
   }
@@ -1734,6 +1986,7 @@ int fds_set_flow(fds_ctx *c, const int64_t *period, int64_t nrows) {
   HIP_TRY(upload(c->flow_period, p, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->flow = true;
+  if (int rc = choose_tiles(c)) return rc;
   touch(c);
   return 0;
 }
@@ -1743,6 +1996,7 @@ int fds_set_learned_boundary(fds_ctx *c, const uint16_t *w1, const uint16_t *w2,
   if (int rc = check_idle(c)) return rc;
   if (!w1) {
     c->lbc_w1 = c->lbc_w2 = nullptr;
+    if (int rc = choose_tiles(c)) return rc;
     touch(c);
     return 0;
   }
@@ -1760,6 +2014,7 @@ int fds_set_learned_boundary(fds_ctx *c, const uint16_t *w1, const uint16_t *w2,
   c->lbc_w2 = w2;
   c->lbc_layer = layer;
   for (int k = 0; k < 3; ++k) c->lbc_cs[k] = comp_scale[k];
+  if (int rc = choose_tiles(c)) return rc;
   touch(c);
   return 0;
 }

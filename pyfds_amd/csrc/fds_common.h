@@ -33,6 +33,39 @@ struct OutView {
   int32_t m;
 };
 
+// Fused kernels: one boundary class of a tile, x = a*x + table[off + step*stride] of component
+// comp, then entry `next` of the tile's list (1-based; 0: last).
+struct FusedClass {
+  double a;
+  int64_t off, stride;
+  int32_t comp, next;
+};
+
+// Fused kernels: one recorded point of a strip (lane of its column, output slot).
+struct FusedPoint {
+  int32_t col, id;
+};
+
+constexpr int kPalMax = 64;                 // material classes, class 0 = outside the array
+constexpr int kFusedClasses = 64;           // classes per tile, entry 0 = none
+constexpr uint32_t kFusedRecord = 1u << 24; // word bit of a recorded point of component 0
+
+// Fused kernels: the tiles' events.  slot[tile] >= 0: the tile has a word per cell of its rows
+// (words[slot][row][lane]: the class of component k in bits 8k .. 8k+7, kFusedRecord << k for
+// a recorded point), classes cls[cls_ptr[slot] .. cls_ptr[slot + 1]) and recorded points
+// points[point_rows[slot][k][r] .. point_rows[slot][k][r + 1]) of component k in row r.
+struct FusedEv {
+  const int32_t *slot;
+  const int32_t *tiles;     // tile of each slot
+  const uint32_t *words;
+  const int32_t *cls_ptr;
+  const FusedClass *cls;
+  const FusedPoint *points;
+  const int32_t *point_rows;
+  int32_t rows;             // word rows per tile
+  int32_t nslots;           // tiles with events
+};
+
 template <typename T>
 struct StepArgs {
   int32_t nx, ny;
@@ -53,6 +86,12 @@ struct StepArgs {
   int32_t steps;        // resident 1D kernels: steps to run in this launch
   int32_t strip_h;      // row-streaming kernels: rows per strip
   int32_t ghost;        // row-streaming kernels: ghost columns / rows per side (fused steps - 1)
+  int32_t ghost_rows;   // fused kernels: ghost rows above a strip the event tables cover
+  int32_t sx;           // fused kernels: columns a strip owns
+  FusedEv fev;
+  const uint8_t *pal_idx;   // fused kernels: material class of each cell (1 ..; nullptr: none)
+  const T *pal;             // and the classes' coefficients [class][4] (class 0: zeros)
+  int32_t npal;
   const void *lhead[3]; // resident 1D kernels: per-thread first boundary cell (LineEvHead)
   const void *ohead[3]; // resident 1D kernels: per-thread first recorded point (LineOutHead)
 };
@@ -119,10 +158,10 @@ __device__ __forceinline__ double out_value(T x, T c) {
 // 32 bits, no LDS round trip, no barrier): lane i receives lane i-1's value (lane 0 gets zero)
 // or lane i+1's value (lane 63 gets zero).  Called with all 64 lanes active.
 __device__ __forceinline__ int dpp_from_left(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);   // wave_shr:1
+  return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true);   // wave_shr:1
 }
 __device__ __forceinline__ int dpp_from_right(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, false);   // wave_shl:1
+  return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true);   // wave_shl:1
 }
 __device__ __forceinline__ float wave_from_left(float v) {
   return __int_as_float(dpp_from_left(__float_as_int(v)));

@@ -11,7 +11,8 @@ constexpr int kNumTiles = 6;
 constexpr int kTileShapes[kNumTiles][2] = {
     {64, 16}, {64, 8}, {128, 8}, {256, 4}, {128, 4}, {256, 1}};
 constexpr int kDefaultTile2D = 1;       // default of the tile engine (lossy models)
-constexpr int kDefaultLossless2D = kNumTiles + 8;   // lossless 2D: streaming 64 x 16, 2 steps
+constexpr int kDefaultLossless2D = kNumTiles + 8;   // lossless 2D where the fused engine does
+                                                    // not apply: streaming 64 x 16, 2 steps
 constexpr int kDefaultLossy2D = kNumTiles + 7;      // lossy 2D: streaming 64 x 16, one step
 constexpr int kTileRow = 5;
 
@@ -79,6 +80,11 @@ struct BatchLaunch {
 };
 using BatchFn = void (*)(const BatchLaunch &b, int nblocks, size_t lds_bytes, hipStream_t s);
 
+// Fused engine (fds_fused2d.h): most stages per launch, tallest strip.
+constexpr int kFusedMax = 6;
+constexpr int kFusedStrip = 512;
+#define FDS_FUSED_STAGES(X) X(1) X(2) X(3) X(4) X(5) X(6)
+
 struct KernelSet {
   LaunchFn acoustic[kNumTiles][2][2];   // [tile][axi][lossy]
   LaunchFn thermal[kNumTiles][2];       // [tile][axi]
@@ -91,6 +97,9 @@ struct KernelSet {
   // persistent variant: a resident grid takes tiles from a work queue (grid chosen inside)
   BatchFn stream_batch_wq[kNumStream][kMaxStages];
   LaunchFn stream_lossy[kNumStream][3];         // lossy acoustics, one step: [shape][variant]
+  // fused engine (one-wave strips): [acoustic, thermal][coefficients per cell, per material
+  // class][plain, axi, isotropic][stages - 1]
+  LaunchFn fused[2][2][3][kFusedMax];
   // resident 1D engine: [cells per thread][acoustic, lossy acoustic, thermal, nonlinear]
   LineFn line[4][4];
   // ThermoAcoustic1D on the resident engine: [cells per thread][lossless, lossy acoustics]

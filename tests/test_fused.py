@@ -1,0 +1,118 @@
+"""The fused engine (default of the lossless 2D models) where it can go wrong: grids at the
+edges of its strips (64 - 2S owned columns, partial strips), rows narrower than a wave, runs
+that end in launches of fewer steps, materials with and without classes, boundary classes with
+several entries and more classes than a tile holds.  FP64 against the oracle bit for bit, the
+FP32 forms against the LDS-tile engine's bits."""
+import numpy as np
+import pytest
+
+import pyfds_amd
+import scenes
+
+pytestmark = pytest.mark.gpu
+
+STEPS = 23      # three launches of six stages and one of five; six of four, one of three
+
+
+def _scene(model, nx, ny, steps=STEPS, medium='block', boundaries='plain', seed=0, ratio=1.0):
+    rng = np.random.default_rng(seed)
+    n = nx * ny
+    thermal = model.startswith('Thermal')
+    dx = 1e-3 if thermal else 1e-4
+    kwargs = dict(x_samples=nx, x_delta=dx, y_samples=ny, y_delta=dx * ratio, t_samples=steps)
+    if thermal:
+        kind, base = 'ThermalMaterial', dict(heat_capacity=4000.0, density=1000.0,
+                                             thermal_conductivity=0.6)
+        kwargs['t_delta'] = 0.1 * dx ** 2 * 4e6 / 50.0
+        main, other = 'temperature', ('heat_flux_x', 'heat_flux_y')
+    else:
+        kind, base = 'AcousticMaterial', dict(scenes.WATER)
+        kwargs['t_delta'] = 0.4 * dx / 5900.0
+        main, other = 'pressure', ('velocity_x', 'velocity_y')
+
+    def material(i):
+        if thermal:
+            return kind, dict(base, thermal_conductivity=1.0 + i % 50)
+        return kind, dict(base, sound_velocity=1000.0 + 7.0 * i, density=900.0 + 3.0 * i)
+
+    if medium == 'block':
+        cells = np.flatnonzero(rng.random(n) < 0.3)
+        regions = [(cells, material(11))] if cells.size else []
+    else:               # one material a row: more classes than the kernels hold (64) if ny > 63
+        regions = [(np.arange(r * nx, (r + 1) * nx), material(r)) for r in range(ny)]
+    signal = rng.standard_normal(steps)
+    point = [int(rng.integers(n))]
+    bounds = {main: [dict(indices=point, value=signal, additive=True)]}
+    if boundaries != 'plain':
+        x, y = np.arange(nx), np.arange(ny)
+        bounds[other[0]] = [dict(indices=np.concatenate([y * nx, y * nx + nx - 1]), value=0.0,
+                                 additive=False)]
+        bounds[other[1]] = [dict(indices=np.concatenate([x, x + (ny - 1) * nx]), value=0.25,
+                                 additive=False)]
+        # chains of entries: the same cells again, and a repeated index
+        bounds[main] += [dict(indices=point * 2, value=0.5, additive=True),
+                         dict(indices=[0, n - 1, point[0]], value=signal[::-1].copy(),
+                              additive=True)]
+    if boundaries == 'many':      # a signal a point, two rows of them: more than a tile holds
+        k = 2 * nx
+        bounds[main].append(dict(indices=list(range(k)),
+                                 value=[rng.standard_normal(steps) for _ in range(k)],
+                                 additive=True))
+    outs = [int(v) for v in rng.integers(0, n, size=6)]
+    return dict(name='fused', model=model, kwargs=kwargs, material=(kind, base), regions=regions,
+                init={main: rng.standard_normal(n)}, boundaries=bounds,
+                outputs={main: [outs, list(range(min(n, 130)))], other[0]: [outs],
+                         other[1]: [outs]},
+                plan=[('simulate', steps - 10), ('simulate', 7), ('simulate', 3)])
+
+
+def _run(scene, **attrs):
+    fld = scenes.build_field(pyfds_amd, pyfds_amd.regions, scene)
+    for k, v in attrs.items():
+        setattr(fld, k, v)
+    scenes.run_plan(fld, scene)
+    res = scenes.collect(fld, scene)
+    group = fld._runner().lib.fds_steps_per_launch(fld._runner().ctx)
+    fld._runner().close()
+    return res, group
+
+
+CASES = [
+    ('Acoustic2D', 52, 40, 'block', 'plain', 1.0, 0),      # one column block (4 stages: 56)
+    ('Acoustic2D', 57, 9, 'block', 'walls', 1.0, 0),       # one column more; partial strip
+    ('Acoustic2D', 113, 70, 'rows', 'walls', 1.25, 7),     # coefficients cell by cell
+    ('Acoustic2D', 1, 50, 'block', 'plain', 1.0, 0),
+    ('Acoustic2D', 3, 33, 'block', 'walls', 1.0, 5),
+    ('Acoustic2D', 200, 2, 'block', 'plain', 1.25, 0),
+    ('Acoustic2D', 520, 510, 'block', 'walls', 1.0, 0),    # six stages a launch
+    ('Acoustic2D', 130, 60, 'block', 'many', 1.0, 16),     # leaves the engine
+    ('Acoustic3DAxi', 105, 66, 'rows', 'walls', 1.0, 4),
+    ('Acoustic3DAxi', 521, 511, 'block', 'plain', 1.0, 0),
+    ('Thermal2D', 64, 31, 'block', 'walls', 1.0, 0),
+    ('Thermal2D', 530, 500, 'rows', 'walls', 1.25, 0),
+    ('Thermal3DAxi', 71, 65, 'rows', 'plain', 1.0, 9),
+    ('Thermal3DAxi', 517, 513, 'block', 'walls', 1.0, 0),
+]
+
+
+@pytest.mark.parametrize('model,nx,ny,medium,boundaries,ratio,strip', CASES)
+def test_fp64_matches_oracle_bitwise(model, nx, ny, medium, boundaries, ratio, strip):
+    scene = _scene(model, nx, ny, medium=medium, boundaries=boundaries, ratio=ratio)
+    print('fused', model, nx, ny, medium, boundaries, flush=True)
+    ref = scenes.run_oracle(scene)
+    got, group = _run(scene, strip_height=strip)
+    assert group == (2 if boundaries == 'many' else 6 if nx * ny >= 1 << 18 else 4)
+    for k in ref:
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+@pytest.mark.parametrize('form', ['fp32', 'fp32_kahan'])
+@pytest.mark.parametrize('case', [2, 6, 8, 11, 13])
+def test_fp32_forms_equal_tile_engine(case, form):
+    model, nx, ny, medium, boundaries, ratio, strip = CASES[case]
+    scene = _scene(model, nx, ny, medium=medium, boundaries=boundaries, ratio=ratio, seed=3)
+    print('fused', form, model, nx, ny, flush=True)
+    a, _ = _run(scene, form=form, tile=1)
+    b, _ = _run(scene, form=form, strip_height=strip)
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
