@@ -378,13 +378,15 @@ bool can_stream(const fds_ctx *c) {
 
 bool can_stream_batch(const fds_ctx *c) { return can_stream(c) && !c->lossy; }
 
-// The fused engine covers the lossless 2D models whose arrays a buffer descriptor spans (32-bit
-// byte offsets, rows past either end included).
-bool can_fuse(const fds_ctx *c) {
-  const bool lossy = c->lossy && c->family == kAcoustic;
+// The fused engines cover the 2D models whose arrays a buffer descriptor spans (32-bit byte
+// offsets, rows past either end included), lossy ones if their material classes are known.
+bool fuse_reach(const fds_ctx *c) {
   const int64_t reach = c->n + (fds::kFusedStrip + 4 * fds::kFusedMax) * c->nx + 1024;
-  return can_stream(c) && !lossy && !c->fused_over &&
-         reach * (int64_t)c->elem < (int64_t)1 << 32;
+  return can_stream(c) && reach * (int64_t)c->elem < (int64_t)1 << 32;
+}
+
+bool can_fuse(const fds_ctx *c) {
+  return fuse_reach(c) && !c->fused_over && (!(c->lossy && c->family == kAcoustic) || c->npal > 0);
 }
 
 // Resident 1D engine variant for n cells: `cpt` cells per thread if given, else the fewest
@@ -407,23 +409,34 @@ int line_variant(int64_t n, int cpt, int fam) {
 // and the iterations it takes: 401 x 301 FP64 2.5 us a step at 4 stages, 2.6 at 6; from 800 x 600
 // on 6 are ahead (FP64 3.0 and 2.9).  One where something follows every step.
 //
+// Lossy acoustics: a stage holds 15 values a column, so three stages (2000 x 1500 FP64 11 us a
+// step at 3, 14 at 2; 3000^2 38 at 3 and 4), four for large fields of the FP32 forms (3000^2 FP32
+// 13.4 at 4, 15.0 at 3), and with the radius' coefficients on top two (2000 x 1500 FP64 15.8 at
+// 2, 15.6 at 3, 301 x 901 5.4 and 5.7), three for large ones (3000^2 FP64 53 at 2, 46 at 3).
+//
 // Height: short strips make enough waves to fill the chip, tall ones waste fewer ghost rows
-// (2S a strip).  About 24 strips a CU are two rounds of resident waves, and measured best or
-// within 3 % of it from 1024 x 1536 (4-6 rows) over 2048^2 (12) to 4096 x 3000 (24-48).
+// (2S a strip, lossy 3S).  About 24 strips a CU (lossy: 16) are two rounds of resident waves, and
+// measured best or within 3 % of it (lossy 5 %) from 1024 x 1536 (4-6 rows) over 2048^2 (12) to
+// 4096 x 3000 (24-48).
 int choose_fused(fds_ctx *c) {
   const bool each = c->lbc_w1 || c->flow || c->coupled;
-  const int S = each ? 1 : c->n < (1 << 18) ? 4 : fds::kFusedMax;
-  const int64_t sx = 64 - 2 * S, across = (c->nx + sx - 1) / sx;
-  const int64_t want = (across * c->ny + 12 * (int64_t)c->num_cu) / (24 * (int64_t)c->num_cu);
+  const bool lossy = c->lossy && c->family == kAcoustic;
+  int S = c->n < (1 << 18) ? 4 : fds::kFusedMax;
+  if (lossy && c->axi) S = c->n < (1 << 22) ? 2 : 3;
+  else if (lossy) S = c->elem == 4 && c->n >= (1 << 20) ? fds::kFusedLossyMax : 3;
+  if (each) S = 1;
+  const int64_t sx = 64 - 2 * S - (lossy ? 1 : 0), across = (c->nx + sx - 1) / sx;
+  const int64_t strips = (lossy ? 16 : 24) * (int64_t)c->num_cu;
+  const int64_t want = (across * c->ny + strips / 2) / strips;
   const int H = c->strip_rows > 0 ? std::min(c->strip_rows, fds::kFusedStrip)
                                   : (int)std::min<int64_t>(std::max<int64_t>(want, 4), 64);
   c->fused = c->streaming = true;
   c->fuse = S;
   c->ghost = S;
-  c->ghost_rows = S - 1;
+  c->ghost_rows = lossy ? 2 * S - 1 : S - 1;
   c->tx = 64;
   c->ty = H;
-  c->sx = 64 - 2 * S;
+  c->sx = (int)sx;
   c->shape = fds::kDefaultLossless2D;
   c->tiles_x = (int)((c->nx + c->sx - 1) / c->sx);
   c->tiles_y = (int)((c->ny + c->ty - 1) / c->ty);
@@ -614,7 +627,7 @@ void build_line_heads(const Comp &cp, const Events &ev, const Events &oe, int nt
 // programs, each a chain of entries.  Returns 1 when some tile has more entries than the kernels
 // hold (the caller then leaves the fused engine).
 int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
-  const int rows = c->ty + 2 * c->fuse, g = c->ghost_rows + 1;
+  const int g = c->ghost_rows + 1, rows = c->ty + 2 * g;
   std::vector<int32_t> slot(c->ntiles, -1), cls_ptr(1, 0), tiles;
   std::vector<uint32_t> words;
   std::vector<fds::FusedClass> cls;
@@ -821,6 +834,9 @@ void fill_args(const fds_ctx *c, fds::StepArgs<T> &a, int parity) {
 // runs, same bits).
 fds::LaunchFn pick_launch(const fds_ctx *c, int stages, bool ring_ok = true) {
   const int t = c->shape;
+  if (c->fused && c->lossy && c->family == kAcoustic)
+    return c->ks->fused_lossy[c->axi ? 1 : (c->iso_b && c->iso_k && !c->coef_set[FDS_C_MY]) ? 2 : 0]
+                             [stages - 1];
   if (c->fused) {
     const int v = c->axi ? 1 : (c->iso_b && c->iso_k) ? 2 : 0;
     return c->ks->fused[c->family == kThermal ? 1 : 0][c->npal > 0 ? 1 : 0][v][stages - 1];
@@ -1098,34 +1114,38 @@ int get_graph(fds_ctx *c, int chunk, int parity, hipGraphExec_t *out) {
   return 0;
 }
 
-// Material classes.  Cells with the same coefficients (slots 0-3, by their bits) are one class;
-// a field whose cells form fewer than kPalMax classes gets an array of class numbers, one byte a
-// cell, and a table of the classes' coefficients.  Pass q compares every cell without a class to
-// the first such cell (`first[q]`, found by the pass before), gives the equal ones class q + 1
-// and finds the first cell left.
+// Material classes.  Cells with the same coefficients (by their bits) are one class; a field whose
+// cells form fewer than kPalMax classes gets an array of class numbers, one byte a cell, and a
+// table of the classes' coefficients.  Pass q compares every cell without a class to the first
+// such cell (`first[q]`, found by the pass before), gives the equal ones class q + 1 and finds
+// the first cell left.
 template <typename T>
-__global__ __launch_bounds__(256) void k_pal_pass(const T *c0, const T *c1, const T *c2,
-                                                  const T *c3, int64_t n, uint8_t *idx, T *pal,
+struct PalCoefs {
+  const T *c[fds::kPalSlots];   // in the table's order
+};
+
+template <typename T, int NC>
+__global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uint8_t *idx, T *pal,
                                                   unsigned *first, int q) {
   using B = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
   const unsigned f = first[q];
   if (f == ~0u) return;
-  const T *c[4] = {c0, c1, c2, c3};
-  B b[4];
+  B b[NC];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) b[k] = __builtin_bit_cast(B, c[k][f]);
-  // table columns: x factor of the backward and of the forward difference, then the y factors
-  if (blockIdx.x == 0 && threadIdx.x < 4)
-    pal[(q + 1) * 4 + threadIdx.x] = c[(threadIdx.x & 1) ? threadIdx.x >> 1 : 2 + (threadIdx.x >> 1)][f];
+  for (int k = 0; k < NC; ++k) {
+    b[k] = __builtin_bit_cast(B, pc.c[k][f]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) pal[(q + 1) * fds::kPalSlots + k] = pc.c[k][f];
+  }
   const int64_t stride = (int64_t)gridDim.x * 256;
   unsigned left = ~0u;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
     if (q > 0 && idx[i]) continue;
     bool eq = true;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) eq = eq && __builtin_bit_cast(B, c[k][i]) == b[k];
-    if (eq) idx[i] = (uint8_t)(q + 1);
-    else {
+    for (int k = 0; k < NC; ++k) eq = eq && __builtin_bit_cast(B, pc.c[k][i]) == b[k];
+    if (eq) {
+      idx[i] = (uint8_t)(q + 1);
+    } else {
       if (q == 0) idx[i] = 0;
       if (left == ~0u) left = (unsigned)i;
     }
@@ -1136,24 +1156,28 @@ __global__ __launch_bounds__(256) void k_pal_pass(const T *c0, const T *c1, cons
 
 template <typename T>
 int find_classes(fds_ctx *c) {
-  c->npal = 0;
-  const T *cf[4];
-  for (int k = 0; k < 4; ++k)
-    cf[k] = c->coef_set[k] ? c->coef[k].as<const T>() : c->coef[k - 1].as<const T>();
+  const bool lossy = c->lossy && c->family == kAcoustic;
+  const auto slot = [&](int k, int alias) {
+    return c->coef_set[k] ? c->coef[k].as<const T>()
+                          : alias >= 0 ? c->coef[alias].as<const T>() : c->zeros.as<const T>();
+  };
+  // (thermal: Q, G in the places of B, K)
+  const PalCoefs<T> pc{{slot(2, -1), slot(0, -1), slot(3, 2), slot(1, 0), slot(4, -1), slot(5, 4),
+                        slot(6, -1), slot(7, -1)}};
   DevBuf first;
   HIP_TRY(c->pal_idx.ensure(c->n));
-  HIP_TRY(c->pal.ensure(fds::kPalMax * 4 * sizeof(T)));
+  HIP_TRY(c->pal.ensure(fds::kPalMax * fds::kPalSlots * sizeof(T)));
   std::vector<unsigned> f(fds::kPalMax + 1, ~0u);
   f[0] = 0;
   HIP_TRY(upload(first, f, c->stream));
-  HIP_TRY(hipMemsetAsync(c->pal.p, 0, fds::kPalMax * 4 * sizeof(T), c->stream));
+  HIP_TRY(hipMemsetAsync(c->pal.p, 0, fds::kPalMax * fds::kPalSlots * sizeof(T), c->stream));
   const unsigned nb = (unsigned)std::min<int64_t>((c->n + 1023) / 1024, 2048);
   const int most = fds::kPalMax - 1;
   for (int q = 0; q < most;) {
     const int q1 = std::min(q + 4, most);
     for (; q < q1; ++q)
-      hipLaunchKernelGGL(k_pal_pass<T>, dim3(nb), dim3(256), 0, c->stream, cf[0], cf[1], cf[2],
-                         cf[3], c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(),
+      hipLaunchKernelGGL((lossy ? k_pal_pass<T, 8> : k_pal_pass<T, 4>), dim3(nb), dim3(256), 0,
+                         c->stream, pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(),
                          first.as<unsigned>(), q);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(f.data(), first.p, f.size() * sizeof(unsigned), hipMemcpyDeviceToHost,
@@ -1166,6 +1190,13 @@ int find_classes(fds_ctx *c) {
     }
   }
   return 0;
+}
+
+// The material classes of a field that may run on the fused engines.
+int ready_classes(fds_ctx *c) {
+  c->npal = 0;
+  if (c->tile >= 0 || c->family == kNonlinear || !fuse_reach(c)) return 0;
+  return c->elem == 8 ? find_classes<double>(c) : find_classes<float>(c);
 }
 
 int check_ctx(fds_ctx *c) {
@@ -1390,7 +1421,8 @@ int fds_commit(fds_ctx *c) {
   c->iso_b = !c->one_d && !c->coef_set[FDS_C_BY];   // (thermal: QY)
   c->iso_k = !c->one_d && !c->coef_set[FDS_C_KY];   // (thermal: GY)
   if (c->family != kNonlinear) {
-    // the engine depends on the lossy flag just derived
+    // the engine depends on the lossy flag just derived and on the material classes
+    if (int rc = ready_classes(c)) return rc;
     if (int rc = choose_tiles(c)) return rc;
     const size_t lds = lds_bytes(c);
     if (lds > 65536) {
@@ -1398,10 +1430,6 @@ int fds_commit(fds_ctx *c) {
       c->tile = -1;
       if (int rc = choose_tiles(c)) return rc;
     }
-  }
-  c->npal = 0;
-  if (c->fused) {
-    if (int rc = c->elem == 8 ? find_classes<double>(c) : find_classes<float>(c)) return rc;
   }
   c->committed = true;
   touch(c);
@@ -1515,6 +1543,8 @@ int fds_set_tile(fds_ctx *c, int t) {
     return fail(FDS_E_ARG, "tile index %d out of range", t);
   const int old = c->tile;
   c->tile = t;
+  if (c->committed && t < 0 && old >= 0 && !c->coupled)
+    if (int rc = ready_classes(c)) return rc;
   if (int rc = choose_tiles(c)) return rc;
   if (c->committed && lds_bytes(c) > 65536) {
     c->tile = old;

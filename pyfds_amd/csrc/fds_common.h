@@ -46,6 +46,7 @@ struct FusedPoint {
   int32_t col, id;
 };
 
+constexpr int kPalSlots = 8;               // coefficients of a material class
 constexpr int kPalMax = 64;                 // material classes, class 0 = outside the array
 constexpr int kFusedClasses = 64;           // classes per tile, entry 0 = none
 constexpr uint32_t kFusedRecord = 1u << 24; // word bit of a recorded point of component 0
@@ -90,7 +91,9 @@ struct StepArgs {
   int32_t sx;           // fused kernels: columns a strip owns
   FusedEv fev;
   const uint8_t *pal_idx;   // fused kernels: material class of each cell (1 ..; nullptr: none)
-  const T *pal;             // and the classes' coefficients [class][4] (class 0: zeros)
+  const T *pal;             // and the classes' coefficients [class][kPalSlots]
+                            // (class 0: zeros): x factors of the backward and forward
+                            // difference, the y ones, Mx, My, Mc, Mt
   int32_t npal;
   const void *lhead[3]; // resident 1D kernels: per-thread first boundary cell (LineEvHead)
   const void *ohead[3]; // resident 1D kernels: per-thread first recorded point (LineOutHead)

@@ -180,12 +180,12 @@ __device__ __forceinline__ void fused_terms(const FusedEvents &E, int s, uint32_
 }
 
 // Recorded points of row r of the strip at stage s: lane q takes the row's point q (its value
-// comes from the lane of its column).
-template <typename T, bool KAHAN>
+// comes from the lane of its column; components K0 .. K1 - 1).
+template <typename T, bool KAHAN, int K0 = 0, int K1 = 3>
 __device__ __forceinline__ void fused_record(const FusedEvents &E, int s, int r, T p, T cp, T vx,
                                              T cvx, T vy, T cvy) {
   const int t = threadIdx.x;
-  for (int k = 0; k < 3; ++k) {
+  for (int k = K0; k < K1; ++k) {
     const T x = k == 0 ? p : k == 1 ? vx : vy, c = k == 0 ? cp : k == 1 ? cvx : cvy;
     const int e0 = E.rows[k * E.stride + r], e1 = E.rows[k * E.stride + r + 1];
     for (int e = e0; e < e1; e += 64) {
@@ -195,6 +195,49 @@ __device__ __forceinline__ void fused_record(const FusedEvents &E, int s, int r,
       if (in) E.out[k].buf[(E.row + s) * E.out[k].m + q.id] = out_value<T, KAHAN>(xv, cv);
     }
   }
+}
+
+// The events of the tile in word slot `slot`; its classes go to LDS, lane q evaluates entry q for
+// every stage.
+template <int S, typename T>
+__device__ __forceinline__ FusedEvents fused_events(const StepArgs<T> &a, int slot, int64_t step,
+                                                    int64_t row,
+                                                    FusedTerm (&term)[S][kFusedClasses],
+                                                    uint8_t (&next)[kFusedClasses]) {
+  const FusedEv &fe = a.fev;
+  const int t = threadIdx.x, stride = a.strip_h + 1;
+  FusedEvents E;
+  E.term = &term[0][0];
+  E.next = next;
+  E.out = a.outp;
+  E.point = fe.points;
+  E.stride = stride;
+  E.rows = fe.point_rows + (int64_t)slot * 3 * stride;
+  E.row = row;
+  const int e0 = fe.cls_ptr[slot], e1 = fe.cls_ptr[slot + 1];
+  bool chained = false;
+  if (t == 0) {
+    next[0] = 0;
+    for (int s = 0; s < S; ++s) term[s][0] = FusedTerm{1.0, 0.0};
+  }
+  for (int q = t; q < e1 - e0; q += 64) {
+    const FusedClass cl = fe.cls[e0 + q];
+    next[q + 1] = (uint8_t)cl.next;
+    chained = chained || cl.next != 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      term[s][q + 1] = FusedTerm{cl.a, a.prog[cl.comp].table[cl.off + (step + s) * cl.stride]};
+  }
+  E.chained = __any(chained);
+  __syncthreads();
+  return E;
+}
+
+// What the row with event words w holds.
+__device__ __forceinline__ uint32_t fused_row_flags(uint32_t w) {
+  if (!__any(w != 0)) return 0;
+  return (__any(fused_class<0>(w) != 0) ? 1u : 0u) | (__any(fused_class<1>(w) != 0) ? 2u : 0u) |
+         (__any(fused_class<2>(w) != 0) ? 4u : 0u) | (__any((w >> 24) != 0) ? kRowRecord : 0u);
 }
 
 // One stage of the lossless acoustic step: takes row r in x, leaves row r - 1 of the next time
@@ -318,7 +361,7 @@ __device__ __forceinline__ void fused_strip(const StepArgs<T> &a, int tile, int 
     if (t < a.npal) {
       constexpr int NC = FusedLds<T, ISO, S>::NC;
 #pragma unroll
-      for (int q = 0; q < NC; ++q) L.pal[t][q] = a.pal[t * 4 + q];
+      for (int q = 0; q < NC; ++q) L.pal[t][q] = a.pal[t * kPalSlots + q];
     }
     __syncthreads();
   }
@@ -330,34 +373,7 @@ __device__ __forceinline__ void fused_strip(const StepArgs<T> &a, int tile, int 
                                       (int64_t)a.fev.rows * 64)
                            : buf_rsrc((const uint32_t *)a.in[0], 0);
   FusedEvents E{};
-  if constexpr (EV) {
-    const FusedEv &fe = a.fev;
-    E.term = &L.term[0][0];
-    E.next = L.next;
-    E.out = a.outp;
-    E.point = fe.points;
-    E.stride = H + 1;
-    E.rows = fe.point_rows + (int64_t)slot * 3 * (H + 1);
-    E.row = row;
-    // this tile's classes: lane q evaluates entry q for every stage
-    const int e0 = fe.cls_ptr[slot], e1 = fe.cls_ptr[slot + 1];
-    bool chained = false;
-    if (t == 0) {
-      L.next[0] = 0;
-      for (int s = 0; s < S; ++s) L.term[s][0] = FusedTerm{1.0, 0.0};
-    }
-    for (int q = t; q < e1 - e0; q += 64) {
-      const FusedClass cl = fe.cls[e0 + q];
-      L.next[q + 1] = (uint8_t)cl.next;
-      chained = chained || cl.next != 0;
-#pragma unroll
-      for (int s = 0; s < S; ++s)
-        L.term[s][q + 1] =
-            FusedTerm{cl.a, a.prog[cl.comp].table[cl.off + (step + s) * cl.stride]};
-    }
-    E.chained = __any(chained);
-    __syncthreads();
-  }
+  if constexpr (EV) E = fused_events<S>(a, slot, step, row, L.term, L.next);
 
   struct Slot {
     FuRow<T> x;
@@ -438,14 +454,8 @@ __device__ __forceinline__ void fused_strip(const StepArgs<T> &a, int tile, int 
     }
     if constexpr (EV) {
       wc[0] = in[W].w;
-      ac[0] = 0;
-      if (__any(wc[0] != 0)) {
-        ac[0] = (__any(fused_class<0>(wc[0]) != 0) ? 1u : 0u) |
-                (__any(fused_class<1>(wc[0]) != 0) ? 2u : 0u) |
-                (__any(fused_class<2>(wc[0]) != 0) ? 4u : 0u) |
-                (__any((wc[0] >> 24) != 0) ? kRowRecord : 0u);
-        busy = S;
-      }
+      ac[0] = fused_row_flags(wc[0]);
+      if (ac[0]) busy = S;
     }
     auto stages = [&](auto EVc) __attribute__((always_inline)) {
       constexpr bool E1 = decltype(EVc)::value;

@@ -2,6 +2,7 @@
 // once per form (FDS_FORM 0: float64, 1: float32, 2: float32 + Kahan) and stage count
 // (FDS_STAGES), so they compile in parallel.
 #include "fds_fused2d.h"
+#include "fds_fused_lossy.h"
 #include "fds_kernels.h"
 
 #if !defined(FDS_FORM) || !defined(FDS_STAGES)
@@ -34,6 +35,7 @@ constexpr bool K = FDS_KAHAN;
 // Rows of loads in flight: 3 keep the memory busy at two or three waves per SIMD; 2 and 5
 // measured within 3 % (5 takes the registers of one more wave).
 constexpr int kRowsAhead = 3;
+constexpr int kLossyRowsAhead = 2;   // (a stage holds more: 1 and 2 take the same registers)
 
 template <int S, bool THERMAL, bool AXI, bool ISO, bool PAL>
 __global__ __launch_bounds__(64) void k_fused(StepArgs<T> a) {
@@ -44,6 +46,18 @@ __global__ __launch_bounds__(64) void k_fused(StepArgs<T> a) {
 template <int S, bool THERMAL, bool AXI, bool ISO, bool PAL>
 void launch_fused(const void *args, int nblocks, size_t, hipStream_t s) {
   hipLaunchKernelGGL((k_fused<S, THERMAL, AXI, ISO, PAL>), dim3(nblocks), dim3(64), 0, s,
+                     *static_cast<const StepArgs<T> *>(args));
+}
+
+template <int S, bool AXI, bool ISO>
+__global__ __launch_bounds__(64) void k_fused_lossy(StepArgs<T> a) {
+  __shared__ LossyFusedLds<T, ISO, S> L;
+  fused_lossy_tile<T, K, AXI, ISO, S, kLossyRowsAhead>(a, a.dyn[0] + a.k, a.dyn[1] + a.k, L);
+}
+
+template <int S, bool AXI, bool ISO>
+void launch_fused_lossy(const void *args, int nblocks, size_t, hipStream_t s) {
+  hipLaunchKernelGGL((k_fused_lossy<S, AXI, ISO>), dim3(nblocks), dim3(64), 0, s,
                      *static_cast<const StepArgs<T> *>(args));
 }
 
@@ -62,6 +76,11 @@ void FDS_CAT(fill_fused_, FDS_STAGES)(KernelSet &ks) {
   fill_family<S, false, true>(ks);
   fill_family<S, true, false>(ks);
   fill_family<S, true, true>(ks);
+  if constexpr (S <= kFusedLossyMax) {
+    ks.fused_lossy[0][S - 1] = launch_fused_lossy<S, false, false>;
+    ks.fused_lossy[1][S - 1] = launch_fused_lossy<S, true, false>;
+    ks.fused_lossy[2][S - 1] = launch_fused_lossy<S, false, true>;
+  }
 }
 
 }  // namespace FDS_FORM_NS

@@ -82,6 +82,7 @@ using BatchFn = void (*)(const BatchLaunch &b, int nblocks, size_t lds_bytes, hi
 
 // Fused engine (fds_fused2d.h): most stages per launch, tallest strip.
 constexpr int kFusedMax = 6;
+constexpr int kFusedLossyMax = 4;  // lossy acoustics
 constexpr int kFusedStrip = 512;
 #define FDS_FUSED_STAGES(X) X(1) X(2) X(3) X(4) X(5) X(6)
 
@@ -100,6 +101,7 @@ struct KernelSet {
   // fused engine (one-wave strips): [acoustic, thermal][coefficients per cell, per material
   // class][plain, axi, isotropic][stages - 1]
   LaunchFn fused[2][2][3][kFusedMax];
+  LaunchFn fused_lossy[3][kFusedLossyMax];   // lossy acoustics: [variant][stages - 1]
   // resident 1D engine: [cells per thread][acoustic, lossy acoustic, thermal, nonlinear]
   LineFn line[4][4];
   // ThermoAcoustic1D on the resident engine: [cells per thread][lossless, lossy acoustics]

@@ -1,4 +1,4 @@
-"""The fused engine (default of the lossless 2D models) where it can go wrong: grids at the
+"""The fused engines (default of the 2D models) where it can go wrong: grids at the
 edges of its strips (64 - 2S owned columns, partial strips), rows narrower than a wave, runs
 that end in launches of fewer steps, materials with and without classes, boundary classes with
 several entries and more classes than a tile holds.  FP64 against the oracle bit for bit, the
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 STEPS = 23      # three launches of six stages and one of five; six of four, one of three
 
 
-def _scene(model, nx, ny, steps=STEPS, medium='block', boundaries='plain', seed=0, ratio=1.0):
+def _scene(model, nx, ny, steps=STEPS, medium='block', boundaries='plain', seed=0, ratio=1.0,
+           mu=0.0):
     rng = np.random.default_rng(seed)
     n = nx * ny
     thermal = model.startswith('Thermal')
@@ -26,7 +27,7 @@ def _scene(model, nx, ny, steps=STEPS, medium='block', boundaries='plain', seed=
         kwargs['t_delta'] = 0.1 * dx ** 2 * 4e6 / 50.0
         main, other = 'temperature', ('heat_flux_x', 'heat_flux_y')
     else:
-        kind, base = 'AcousticMaterial', dict(scenes.WATER)
+        kind, base = 'AcousticMaterial', dict(scenes.WATER, absorption_coef=mu)
         kwargs['t_delta'] = 0.4 * dx / 5900.0
         main, other = 'pressure', ('velocity_x', 'velocity_y')
 
@@ -112,6 +113,48 @@ def test_fp32_forms_equal_tile_engine(case, form):
     model, nx, ny, medium, boundaries, ratio, strip = CASES[case]
     scene = _scene(model, nx, ny, medium=medium, boundaries=boundaries, ratio=ratio, seed=3)
     print('fused', form, model, nx, ny, flush=True)
+    a, _ = _run(scene, form=form, tile=1)
+    b, _ = _run(scene, form=form, strip_height=strip)
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+# lossy: one, two or three stages a launch, one more ghost column on the right, twice the ghost
+# rows below
+LOSSY = [
+    ('Acoustic2D', 57, 40, 'block', 'plain', 1.0, 0),
+    ('Acoustic2D', 58, 9, 'block', 'walls', 1.0, 0),
+    ('Acoustic2D', 115, 70, 'block', 'walls', 1.25, 7),
+    ('Acoustic2D', 1, 50, 'block', 'plain', 1.0, 0),
+    ('Acoustic2D', 2, 33, 'block', 'walls', 1.0, 5),
+    ('Acoustic2D', 200, 2, 'block', 'plain', 1.25, 0),
+    ('Acoustic2D', 90, 71, 'rows', 'walls', 1.0, 0),       # too many classes: one step a launch
+    ('Acoustic2D', 130, 60, 'block', 'many', 1.0, 16),     # leaves the engine
+    ('Acoustic3DAxi', 106, 66, 'block', 'walls', 1.0, 4),
+    ('Acoustic3DAxi', 171, 90, 'block', 'walls', 1.25, 0),
+    ('Acoustic3DAxi', 64, 40, 'rows', 'plain', 1.0, 0),    # forty classes
+    ('Acoustic2D', 530, 500, 'block', 'walls', 1.0, 0),
+]
+
+
+@pytest.mark.parametrize('model,nx,ny,medium,boundaries,ratio,strip', LOSSY)
+def test_fp64_lossy_matches_oracle_bitwise(model, nx, ny, medium, boundaries, ratio, strip):
+    scene = _scene(model, nx, ny, medium=medium, boundaries=boundaries, ratio=ratio, mu=0.3)
+    print('fused lossy', model, nx, ny, medium, boundaries, flush=True)
+    ref = scenes.run_oracle(scene)
+    got, group = _run(scene, strip_height=strip)
+    assert (group > 1) == (boundaries != 'many' and (medium, ny) != ('rows', 71))
+    for k in ref:
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+@pytest.mark.parametrize('form', ['fp32', 'fp32_kahan'])
+@pytest.mark.parametrize('case', [2, 4, 9, 11])
+def test_fp32_lossy_forms_equal_tile_engine(case, form):
+    model, nx, ny, medium, boundaries, ratio, strip = LOSSY[case]
+    scene = _scene(model, nx, ny, medium=medium, boundaries=boundaries, ratio=ratio, seed=3,
+                   mu=0.3)
+    print('fused lossy', form, model, nx, ny, flush=True)
     a, _ = _run(scene, form=form, tile=1)
     b, _ = _run(scene, form=form, strip_height=strip)
     for k in a:
