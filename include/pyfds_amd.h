@@ -165,7 +165,7 @@ int fds_prepare_run(fds_ctx *ctx, int64_t start_step, int64_t nsteps, int chunk)
  * shapes serve the 2D models (lossy acoustics one time step per launch on any of them).
  * 1D models (Acoustic1D, Thermal1D, IdealGas1D, Acoustic2ndOrder1D) of up to 2^24 cells
  * default (-1) to the resident 1D engine: workgroups keep the line in registers for many steps
- * per launch (one workgroup up to 512 cells, segments beyond; see fds_set_line_shape); any tile
+ * per launch (one wave up to 64 cells, one-wave segments beyond; see fds_set_line_shape); any tile
  * index (and longer lines) puts them on the LDS-tile kernels (one launch per step; nonlinear models on their 256-cell tiles
  * whatever the index). */
 int fds_set_tile(fds_ctx *ctx, int tile_index);

@@ -456,17 +456,16 @@ int choose_tiles(fds_ctx *c) {
   c->ghost = 0;
   c->ghost_rows = 0;
   if ((c->one_d || c->family == kNonlinear) && c->tile < 0 && c->n <= fds::kLineMaxResident) {
-    // segmented lines take up to kLineMaxResident cells; one segment must hold the whole
-    // line.  Automatic
-    // layout: one segment up to kLineSegmentAbove cells, else segments of the default shape
+    // automatic layout (no line shape set): one wave, else segments by line_layout
     int cfg_threads = c->line_cfg_threads, cfg_ghost = c->line_cfg_ghost, cpt_req = c->strip_rows;
     if (cfg_threads < 0) {
       cfg_threads = 0;
-      if (c->strip_rows <= 0 && c->n > fds::kLineSegmentAbove) {
-        const bool lng = c->n > fds::kLineSegLongAbove;
-        cfg_threads = fds::kLineSegThreads;
-        cfg_ghost = lng ? fds::kLineSegLongGhost : fds::kLineSegGhost;
-        cpt_req = lng ? fds::kLineSegLongCpt : fds::kLineSegCpt;
+      if (c->strip_rows <= 0 && c->n > fds::kLineWave) {
+        const fds::LineLayout l = fds::line_layout(
+            c->n, c->lossy && c->family == kAcoustic, c->family == kNonlinear);
+        cfg_threads = fds::kLineWave;
+        cfg_ghost = l.ghost;
+        cpt_req = l.cpt;
       }
     }
     int v = -1;

@@ -45,18 +45,36 @@ constexpr int kCoupleMaxThreads[kNumLineCpt] = {1024, 512, 512, 256};
 // the nonlinear models hold three components and call pow_cr / expm1 / log1p
 constexpr int kNlLineMaxThreads[kNumLineCpt] = {512, 512, 512, 256};
 constexpr int kLineSteps = 2048;                   // time steps per launch at most
-// default layout: one workgroup up to kLineSegmentAbove cells; longer lines in one-wave
-// segments (DPP neighbour exchange, no barriers) of 64 threads x 2 cells with 48 ghost cells
-// per side: 32 owned cells, 47 steps per launch.  Measured on Acoustic1D, 2000 cells: 0.30 us
-// per step, against 0.42 for 128-thread segments with LDS exchange and 0.64 for one
-// workgroup (one CU's issue rate bounds a single workgroup).  A step of a one-wave segment
-// costs ~0.27 us of dependent latency and a launch ~2.8 us, so more ghost cells (more steps
-// per launch) pay until the redundant ghost work matters; lines past kLineSegLongAbove cells,
-// which fill the GPU, use 4 cells per thread and 64 ghost cells (half the redundancy).
+// Default layout: one wave holds a line of up to 64 cells; longer lines are cut into one-wave
+// segments (DPP neighbour exchange, no barriers).  A step of a segment costs its dependent
+// latency (Acoustic1D FP64 about 0.19 us with one cell a lane, 0.35 with two) and a launch 3-4 us,
+// so few cells a lane and many ghost cells (ghost - 1 steps per launch) win as long as the
+// redundant ghost work has idle CUs to run on; longer lines need fewer ghosts, then more cells
+// a lane.  us a step, (cells a lane, ghost cells), FP64:
+//   Acoustic1D 2000 cells (1, 28) 0.34, (2, 48) 0.40; 60000 cells (2, 32) 0.41, (4, 64) 0.44
+//   lossy 24001 cells (1, 20) 0.46, (4, 64) 0.65; 200000 cells (2, 32) 0.75, (4, 64) 0.79
+//   IdealGas1D, whose step is the power's latency: 24001 cells (1, 20) 1.87, (4, 64) 5.2;
+//   60000 cells (1, 16) 1.96; 600000 cells (2, 24) 4.7, (1, 16) 5.0, (4, 64) 7.0
+struct LineLayout {
+  int cpt, ghost;
+};
+
+inline LineLayout line_layout(int64_t n, bool viscous, bool nonlinear) {
+  if (n <= 16384) return {1, 28};
+  // (the per-thread event tables grow with the segments: none of the short ones past 2^21 cells)
+  if (nonlinear)
+    return n <= 32768 ? LineLayout{1, 20} : n <= 131072 ? LineLayout{1, 16}
+           : n <= (1 << 21) ? LineLayout{2, 24} : LineLayout{4, 64};
+  if (viscous) return n <= 32768 ? LineLayout{1, 20} : n <= 262144 ? LineLayout{2, 32}
+                                                                  : LineLayout{4, 64};
+  return n <= 131072 ? LineLayout{2, 32} : LineLayout{4, 64};
+}
+
+// Layout of coupled pairs (two fields in one kernel): one workgroup up to kLineSegmentAbove
+// cells, else one-wave segments of 2 cells a lane with 48 ghost cells.
+constexpr int kLineWave = 64;
 constexpr int kLineSegmentAbove = 512;
 constexpr int kLineSegCpt = 2, kLineSegThreads = 64, kLineSegGhost = 48;
-constexpr int kLineSegLongAbove = 16384;
-constexpr int kLineSegLongCpt = 4, kLineSegLongGhost = 64;
 // longest line on the resident engine: its per-thread event tables hold one entry per thread
 // of every segment (half a line's cells); longer lines step on the LDS-tile kernels
 constexpr int64_t kLineMaxResident = int64_t(1) << 24;
@@ -85,6 +103,7 @@ __device__ __forceinline__ int line_base(const StepArgs<T> &a) {
 // general path, which re-reads the thread's list.
 struct LineBound {
   int info;          // bits 0-7: cached cell's register slot (0xff: none); bit 8: general path
+  bool any;          // some lane of the wave has a cell (uniform: most waves skip apply)
   int32_t idx;       // table index of the value of the step after the next to apply
   int32_t stride;
   double a, val, val2;   // x = a*x + val this step; val2 the next step's value
@@ -101,6 +120,7 @@ struct LineBound {
     a = h.a;
     idx = (int32_t)(h.off + step0 * (int64_t)h.stride);
     const bool on = (info & 0xff) != 0xff;
+    any = __any(info != 0xff);
     val = on ? pg.table[idx] : 0.0;
     val2 = (on && stride != 0 && steps > 1) ? pg.table[idx + stride] : val;
   }
@@ -110,6 +130,7 @@ struct LineBound {
   template <typename T, bool KAHAN, int CPT>
   __device__ __forceinline__ void apply(const EvView &ev, const ProgView &pg, int64_t step,
                                         int rem, T (&x)[CPT], T (&c)[CPT]) {
+    if (!any) return;
     const int sl = slot();
     if (sl != 0xff) {
       // the slot is tested against each register position (compile-time index) so that the
@@ -146,16 +167,19 @@ struct LineBound {
 // output slot).  The first point is cached in registers; further points re-read the list.
 struct LineRecord {
   int info, id;      // info: bits 0-7 first point's register slot (0xff: none), bit 8: more
+  bool any;          // some lane of the wave has a point (uniform)
 
   __device__ __forceinline__ void init(const void *heads, int t) {
     const LineOutHead h = static_cast<const LineOutHead *>(heads)[t];
     info = h.info;
     id = h.id;
+    any = __any((info & 0xff) != 0xff);
   }
 
   template <typename T, bool KAHAN, int CPT>
   __device__ __forceinline__ void write(const OutView &o, int64_t row, const T (&x)[CPT],
                                         const T (&c)[CPT]) const {
+    if (!any) return;
     const int sl = info & 0xff;
     if (sl == 0xff) return;
     double *dst = o.buf + row * o.m;
