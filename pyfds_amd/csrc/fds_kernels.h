@@ -77,6 +77,10 @@ struct BatchLaunch {
   int nq;
   int spl;
   int num_cu;
+  // fused launches: the tiles with events (instance, event slot), launched first
+  const int32_t *ev_inst;
+  const int32_t *ev_slot;
+  int nev;
 };
 using BatchFn = void (*)(const BatchLaunch &b, int nblocks, size_t lds_bytes, hipStream_t s);
 
@@ -101,6 +105,8 @@ struct KernelSet {
   // fused engine (one-wave strips): [acoustic, thermal][coefficients per cell, per material
   // class][plain, axi, isotropic][stages - 1]
   LaunchFn fused[2][2][3][kFusedMax];
+  // batches on the fused engine: [acoustic plain/axi isotropic only, any lossless model]
+  BatchFn fused_batch[2][kFusedMax];
   LaunchFn fused_lossy[3][kFusedLossyMax];   // lossy acoustics: [variant][stages - 1]
   // resident 1D engine: [cells per thread][acoustic, lossy acoustic, thermal, nonlinear]
   LineFn line[4][4];

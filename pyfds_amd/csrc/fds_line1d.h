@@ -95,8 +95,8 @@ __device__ __forceinline__ int line_base(const StepArgs<T> &a) {
   return blockIdx.x * a.strip_h - a.ghost;
 }
 
-// A thread's boundary cells of one component.  Lists are CSR over threads: entries
-// ev.ptr[t]..ev.ptr[t+1]-1, ev.pos = register slot, ev.id = unique boundary cell.  The first
+// A thread's boundary cells of one component: entries e0 .. e1 - 1 of the event list (from the
+// thread's head), ev.pos = register slot, ev.id = unique boundary cell.  The first
 // cell, when its program has a single entry (the usual case), is cached in registers; a
 // constant value (stride 0) is loaded once, a signal's values two steps ahead (a step of a
 // segment is shorter than a cache round trip).  Any other cell of the thread takes the
@@ -107,6 +107,7 @@ struct LineBound {
   int32_t idx;       // table index of the value of the step after the next to apply
   int32_t stride;
   double a, val, val2;   // x = a*x + val this step; val2 the next step's value
+  int e0, e1;        // the general path's entries
 
   __device__ __forceinline__ int slot() const { return info & 0xff; }
 
@@ -118,6 +119,8 @@ struct LineBound {
     info = h.info;
     stride = h.stride;
     a = h.a;
+    e0 = h.e0;
+    e1 = h.e1;
     idx = (int32_t)(h.off + step0 * (int64_t)h.stride);
     const bool on = (info & 0xff) != 0xff;
     any = __any(info != 0xff);
@@ -151,9 +154,7 @@ struct LineBound {
       }
     }
     if (info & 0x100) {
-      const int t = line_thread();
-      const int e1 = ev.ptr[t + 1];
-      for (int e = ev.ptr[t] + (sl != 0xff ? 1 : 0); e < e1; ++e) {
+      for (int e = e0; e < e1; ++e) {
         const int s = ev.pos[e], u = ev.id[e];
 #pragma unroll
         for (int m = 0; m < CPT; ++m)
@@ -163,16 +164,19 @@ struct LineBound {
   }
 };
 
-// A thread's recorded points of one component (CSR over threads like LineBound; ev.id = the
-// output slot).  The first point is cached in registers; further points re-read the list.
+// A thread's recorded points of one component (ev.id = the output slot).  The first point is
+// cached in registers; further points re-read the list.
 struct LineRecord {
   int info, id;      // info: bits 0-7 first point's register slot (0xff: none), bit 8: more
+  int e0, e1;        // the further points
   bool any;          // some lane of the wave has a point (uniform)
 
   __device__ __forceinline__ void init(const void *heads, int t) {
     const LineOutHead h = static_cast<const LineOutHead *>(heads)[t];
     info = h.info;
     id = h.id;
+    e0 = h.e0;
+    e1 = h.e1;
     any = __any((info & 0xff) != 0xff);
   }
 
@@ -187,9 +191,7 @@ struct LineRecord {
     for (int m = 0; m < CPT; ++m)
       if (sl == m) dst[id] = out_value<T, KAHAN>(x[m], c[m]);
     if (info & 0x100) {
-      const int t = line_thread();
-      const int e1 = o.ev.ptr[t + 1];
-      for (int e = o.ev.ptr[t] + 1; e < e1; ++e) {
+      for (int e = e0; e < e1; ++e) {
         const int s = o.ev.pos[e], i = o.ev.id[e];
 #pragma unroll
         for (int m = 0; m < CPT; ++m)

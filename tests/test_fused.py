@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import pyfds_amd
+import pyfds_amd.batch
 import scenes
 
 pytestmark = pytest.mark.gpu
@@ -159,3 +160,48 @@ def test_fp32_lossy_forms_equal_tile_engine(case, form):
     b, _ = _run(scene, form=form, strip_height=strip)
     for k in a:
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+def _batch_scenes(models):
+    sizes = [(130, 61), (57, 200), (300, 40), (3, 70), (515, 520)]
+    return [_scene(m, *sizes[i], medium='block', boundaries='walls' if i % 2 else 'plain',
+                   ratio=r, seed=i) for i, (m, r) in enumerate(models)]
+
+
+@pytest.mark.parametrize('models', [
+    [('Acoustic2D', 1.0), ('Acoustic3DAxi', 1.0), ('Acoustic3DAxi', 1.25), ('Acoustic2D', 1.0),
+     ('Acoustic2D', 1.0)],
+    [('Acoustic2D', 1.25), ('Thermal2D', 1.0), ('Thermal3DAxi', 1.0), ('Thermal2D', 1.25)]])
+def test_fp64_batch_matches_oracle_bitwise(models):
+    """Batches on the fused engine: six and four stages a launch, remainders in one launch; then
+    a boundary list that no longer fits it, which moves the batch to its streaming shape."""
+    built = [(sc, scenes.build_field(pyfds_amd, pyfds_amd.regions, sc))
+             for sc in _batch_scenes(models)]
+    fields = [f for _, f in built]
+    batch = pyfds_amd.batch.BatchRunner(fields, chunk=8)
+    for n in (13, 7):
+        batch.simulate(n)
+    group = batch.lib.fds_batch_steps_per_launch(batch.handle)
+    assert group == (6 if sum(f.num_points for f in fields) >= 1 << 18 else 4)
+    more = [dict(indices=list(range(250)), value=[np.full(STEPS, 0.1 * i) for i in range(250)],
+                 additive=True)]
+    main = next(iter(built[0][0]['boundaries']))
+    getattr(fields[0], main).add_boundary(pyfds_amd.regions.Region(more[0]['indices']),
+                                          value=more[0]['value'], additive=True)
+    batch.simulate(3)
+    assert batch.lib.fds_batch_steps_per_launch(batch.handle) == 2
+    for i, (sc, fld) in enumerate(built):
+        print('member', i, sc['model'], flush=True)
+        o = scenes.build_oracle(sc)
+        o.simulate(20)
+        if i == 0:
+            o.boundaries[main] = o.boundaries[main] + more
+        o.simulate(3)
+        got = scenes.collect(fld, sc)
+        for comp in scenes.COMPONENTS[sc['model']]:
+            np.testing.assert_array_equal(got['values/' + comp], o.components[comp],
+                                          err_msg='%d %s' % (i, comp))
+            for k, out in enumerate(o.outputs[comp]):
+                np.testing.assert_array_equal(got['signals/%s/%d' % (comp, k)],
+                                              np.array(out['signals'], dtype=float),
+                                              err_msg='%d %s' % (i, comp))
