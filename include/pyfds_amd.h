@@ -342,6 +342,24 @@ int fds_lbc_gather(const float *frames, const int32_t *run, const int32_t *step,
                    int D, int G, int L, const float *comp_scale, void *stream);
 int fds_lbc_band_rms(const float *frames, float *rms, int F, int D, int G, int L, void *stream);
 
+/* `iters` iterations of the training (gather, both convolutions, loss, their gradients, Adam, bf16
+ * copies) of the network above, enqueued on `stream` in three launches each.  frames, comp_scale, T,
+ * D, G, L as for fds_lbc_gather; run, step, side, scale: [iters][B]; layers: the two layers'
+ * float32 weights and moments, their bf16 copies wb ([4][Co][5][Ci]) and wt ([4][Ci][5][Co]);
+ * wch [48]; work: fds_lbc_train_workspace(B, G) bytes, 16-byte aligned; loss: B * ceil(G / 64)
+ * partial sums of the last iteration's loss over positions [0, G) (sides 0, 1) or [L, G - L).
+ * Adam's step counts from first_step (1 for the first ever). */
+typedef struct {
+  float *w, *m, *v;
+  uint16_t *wb, *wt;
+} fds_lbc_layer;
+int fds_lbc_train_workspace(int B, int G, int64_t *bytes);
+int fds_lbc_train(const float *frames, const int32_t *run, const int32_t *step,
+                  const int32_t *side, const float *scale, const float *wch,
+                  const fds_lbc_layer *layers, void *work, float *loss, int iters, int B, int T,
+                  int D, int G, int L, const float *comp_scale, float lr, float b1, float b2,
+                  float eps, int first_step, void *stream);
+
 /* Diagnostics in float64 on the device: over a wx x wy window at (ax0, ay0) of context a and
  * (bx0, by0) of context b, num = sum (a - b)^2 and den = sum b^2 of the current states. */
 int fds_window_sq_diff(fds_ctx *a, int comp_a, fds_ctx *b, int comp_b, int wx, int wy, int ax0,

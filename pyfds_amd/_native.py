@@ -30,11 +30,17 @@ EXPORTS = ('fds_create', 'fds_destroy', 'fds_set_scalars', 'fds_set_coeff', 'fds
            'fds_set_learned_boundary',
            'fds_lbc_conv_fwd', 'fds_lbc_conv_bwd_data', 'fds_lbc_conv_bwd_weight',
            'fds_lbc_reduce_weight', 'fds_lbc_mse', 'fds_lbc_adam', 'fds_lbc_pack',
-           'fds_lbc_gather', 'fds_lbc_band_rms', 'fds_window_sq_diff', 'fds_window_sq_diff_static',
+           'fds_lbc_gather', 'fds_lbc_band_rms', 'fds_lbc_train', 'fds_lbc_train_workspace',
+           'fds_window_sq_diff', 'fds_window_sq_diff_static',
            'fds_output_device_ptr',
            'fds_set_nonfinite_check', 'fds_coupling_create', 'fds_coupling_set_material',
            'fds_coupling_set_scalars', 'fds_coupling_state', 'fds_coupling_run',
            'fds_coupling_destroy', 'fds_get_coeff', 'fds_last_error', 'fds_version')
+
+
+class LbcLayer(ct.Structure):
+    """``fds_lbc_layer``: device pointers of one layer's weights, moments and bf16 copies."""
+    _fields_ = [(n, ct.c_void_p) for n in ('w', 'm', 'v', 'wb', 'wt')]
 
 
 class NativeError(RuntimeError):
@@ -122,6 +128,9 @@ def load():
         'fds_lbc_mse': (ct.c_int, [_p] * 7 + [ct.c_int] * 4 + [ct.c_float, _p]),
         'fds_lbc_adam': (ct.c_int, [_p] * 4 + [ct.c_int] + [ct.c_float] * 4 + [ct.c_int, _p]),
         'fds_lbc_pack': (ct.c_int, [_p] * 3 + [ct.c_int] * 4 + [_p]),
+        'fds_lbc_train_workspace': (ct.c_int, [ct.c_int] * 2 + [_p]),
+        'fds_lbc_train': (ct.c_int, [_p] * 9 + [ct.c_int] * 6 + [_p] + [ct.c_float] * 4
+                          + [ct.c_int, _p]),
         'fds_lbc_gather': (ct.c_int, [_p] * 7 + [ct.c_int] * 5 + [_p, _p]),
         'fds_lbc_band_rms': (ct.c_int, [_p, _p] + [ct.c_int] * 4 + [_p]),
         'fds_window_sq_diff': (ct.c_int, [_p, ct.c_int, _p, ct.c_int] + [ct.c_int] * 6

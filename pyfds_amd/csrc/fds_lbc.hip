@@ -14,23 +14,10 @@
 
 #include "../../include/pyfds_amd.h"
 #include "fds_lbc.h"
+#include "fds_lbc_dev.h"
 
 namespace fds {
 namespace {
-
-typedef short s4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);   // round to nearest even
-  return (uint16_t)(u >> 16);
-}
-
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
-__device__ __forceinline__ s4 ld4(const uint16_t *p) { return *reinterpret_cast<const s4 *>(p); }
 
 __device__ __forceinline__ s4 ld4_strided(const uint16_t *p, int stride, int n_valid) {
   s4 r;
@@ -39,10 +26,6 @@ __device__ __forceinline__ s4 ld4_strided(const uint16_t *p, int stride, int n_v
   r[2] = n_valid > 2 ? (short)p[2 * stride] : (short)0;
   r[3] = n_valid > 3 ? (short)p[3 * stride] : (short)0;
   return r;
-}
-
-__device__ __forceinline__ f4 mfma(s4 a, s4 b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------- training kernels
@@ -239,6 +222,316 @@ __global__ __launch_bounds__(256) void k_gather(const float *__restrict__ frames
   for (int c = 0; c < 3; ++c)
     for (int d = 0; d < kLbcDepth; ++d)
       to[c * kLbcDepth + d] = frames[(((f0 * 3 + c) * 4 + s) * D + d) * G + a] * cs[c] * sc;
+}
+
+// ---------------------------------------------------------------- fused training iteration
+// Three launches per iteration.  One kernel per operation, enqueued one by one with six sample
+// lists copied in between, was bound by the host and by those copies: 20 iterations of 32 samples
+// on 1056 positions 6.9 ms, so 1.6 ms.
+//   k_train_grads    gather, both convolutions, loss and the gradient at the hidden layer of a
+//                    segment of a sample, in LDS;
+//   k_train_weights  the weight gradients of one sample, one 16 x 16 tile for all taps a wave;
+//   k_train_update   sum over the samples, Adam, and the bf16 copies of the weights.
+// Sums run in the order of the separate kernels (k_conv_fwd, ...): the same bits.
+// Between the first two, x, the hidden layer and both gradients stand channel-major
+// ([B][C][pitch] bf16, position p at kPad + p, zeros around), so that the reduction over the
+// positions reads whole vectors.
+constexpr int kPad = 4;
+constexpr int kTrainSeg = 64;     // positions a workgroup of k_train_grads hands on
+constexpr int kChunk = 8;         // 16-position products of k_train_weights in flight
+
+struct TrainStep {
+  const float *frames, *scale, *wch;
+  const int32_t *run, *step, *side;
+  const uint16_t *w1b, *w2b, *w2t;
+  uint16_t *x, *h, *dy, *dh;
+  float *part1, *part2, *loss;
+  int T, D, G, L, pitch;
+  float cs[3], norm;
+};
+
+__host__ __device__ inline int train_pitch(int G) { return (G + 127) / 128 * 128 + 2 * kPad; }
+
+// Zeros around the rows of the four channel-major arrays (k_train_grads writes the rest).
+__global__ __launch_bounds__(64) void k_train_pads(uint16_t *rows, int G, int pitch) {
+  uint16_t *r = rows + (size_t)blockIdx.x * pitch;
+  if (threadIdx.x < kPad) r[threadIdx.x] = 0;
+  for (int i = kPad + G + threadIdx.x; i < pitch; i += 64) r[i] = 0;
+}
+
+// Bound by latency: a chain of loads, three products and three barriers; 64 positions a
+// workgroup give 544 of them for 32 samples of 1056 positions (two a CU), and the 12 rows
+// computed twice on the way cost a fifth.  The weights stay in registers: a wave keeps one
+// column of 16 output channels for all its rows.
+__global__ __launch_bounds__(256) void k_train_grads(TrainStep A) {
+  constexpr int R = kLbcTaps / 2;
+  constexpr int NT = 5;                            // row tiles of the hidden layer and of dy
+  constexpr int NR = 16 * NT, NXR = NR + 2 * R;    // rows; input rows the tiles read
+  constexpr int SX = kLbcCin + 4, SH = kLbcHidden + 4, SY = kLbcCout + 4;  // (LDS banks)
+  static_assert(kTrainSeg + 8 * R <= NR, "hidden rows cover the segment and its reach");
+  // row 0 of the hidden layer and of dy is position a0 - 2R, of the input a0 - 3R; hid has R
+  // rows more on both sides, which only rows of dy that nothing reads look at
+  __shared__ __attribute__((aligned(16))) uint16_t xin[NXR * SX];
+  __shared__ __attribute__((aligned(16))) uint16_t hid[(NR + 2 * R) * SH];
+  __shared__ __attribute__((aligned(16))) uint16_t dyl[NR * SY];
+  __shared__ float red[4];
+  const int G = A.G, L = A.L, b = blockIdx.y, a0 = blockIdx.x * kTrainSeg;
+  const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63, m = l & 15, g = l >> 4;
+  const int s = A.side[b];
+  const size_t f0 = (size_t)A.run[b] * A.T + A.step[b];
+  const float sc = A.scale[b];
+  constexpr int N1 = kLbcTaps * (kLbcCin / 16), N2 = kLbcTaps * (kLbcHidden / 16),
+                NB = kLbcTaps * (kLbcCout / 16);
+
+  // inputs, targets and the weights of both layers, all in flight together
+  constexpr int NI = kLbcCin * NXR, II = (NI + 255) / 256;
+  float rx[II];
+#pragma unroll
+  for (int i = 0; i < II; ++i) {
+    const int e = tid + 256 * i, row = e % NXR, ci = e / NXR, a = a0 - 3 * R + row;
+    rx[i] = 0.f;
+    if (e < NI && a >= L && a < G - L) {
+      const int h = ci / 24, c = (ci % 24) / kLbcBand, j = ci % kLbcBand;
+      rx[i] = A.frames[((((f0 - h) * 3 + c) * 4 + s) * A.D + L + j) * G + a];
+    }
+  }
+  // layer 2: waves 0-2 take a column of channels each (a component), rows of tiles 0-3; wave 3
+  // the last tile of all three
+  float tg[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int nt = wave < 3 ? wave : i, mt = wave < 3 ? i : NT - 1;
+    const int a = a0 - 2 * R + 16 * mt + 4 * g;
+    const bool job = wave < 3 || i < 3;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      tg[i][v] = 0.f;
+      if (job && a + v >= 0 && a + v < G)
+        tg[i][v] = A.frames[(((f0 * 3 + nt) * 4 + s) * A.D + m) * G + a + v];
+    }
+  }
+  s4 b1[N1], b2[N2];
+  const uint16_t *g1 = A.w1b + (size_t)s * kLbcHidden * kLbcTaps * kLbcCin;
+  const uint16_t *g2 = A.w2b + (size_t)s * kLbcCout * kLbcTaps * kLbcHidden;
+  const auto load2 = [&](int nt) {
+#pragma unroll
+    for (int i = 0; i < N2; ++i)
+      b2[i] = ld4(g2 + ((16 * nt + m) * kLbcTaps + i / 2) * kLbcHidden + 16 * (i % 2) + 4 * g);
+  };
+#pragma unroll
+  for (int i = 0; i < N1; ++i)
+    b1[i] = ld4(g1 + ((16 * (wave & 1) + m) * kLbcTaps + i / 3) * kLbcCin + 16 * (i % 3) + 4 * g);
+  load2(wave < 3 ? wave : 0);
+
+#pragma unroll
+  for (int i = 0; i < II; ++i) {
+    const int e = tid + 256 * i, row = e % NXR, ci = e / NXR, a = a0 - 3 * R + row;
+    if (e >= NI) continue;
+    const int c = (ci % 24) / kLbcBand;
+    const uint16_t v = f2bf(rx[i] * (c == 0 ? A.cs[0] : c == 1 ? A.cs[1] : A.cs[2]) * sc);
+    xin[row * SX + ci] = v;
+    if (a >= a0 && a < a0 + kTrainSeg && a < G)
+      A.x[((size_t)b * kLbcCin + ci) * A.pitch + kPad + a] = v;
+  }
+  for (int e = tid; e < R * SH; e += 256) {
+    hid[e] = 0;
+    hid[(NR + R) * SH + e] = 0;
+  }
+  __syncthreads();
+
+  // layer 1
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int nt = wave & 1, mt = (wave >> 1) + 2 * i;
+    if (mt >= NT) break;
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+      acc = mfma(ld4(xin + (16 * mt + m + j / 3) * SX + 16 * (j % 3) + 4 * g), b1[j], acc);
+    s4 o;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int hp = 16 * mt + 4 * g + v, a = a0 - 2 * R + hp;
+      o[v] = a >= 0 && a < G ? (short)f2bf(acc[v]) : (short)0;
+      hid[(hp + R) * SH + 16 * nt + m] = (uint16_t)o[v];
+    }
+    const int a = a0 - 2 * R + 16 * mt + 4 * g;
+    if (a >= a0 && a < a0 + kTrainSeg)
+      *reinterpret_cast<s4 *>(A.h + ((size_t)b * kLbcHidden + 16 * nt + m) * A.pitch + kPad + a) = o;
+  }
+  __syncthreads();
+
+  // layer 2, the loss and its gradient; the weights of the way back are under way meanwhile
+  s4 bb[NB];
+  const uint16_t *gt = A.w2t + (size_t)s * kLbcHidden * kLbcTaps * kLbcCout;
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    bb[i] = ld4(gt + ((16 * (wave & 1) + m) * kLbcTaps + i / 3) * kLbcCout + 16 * (i % 3) + 4 * g);
+  const int lo = s < 2 ? 0 : L, hi = s < 2 ? G : G - L;
+  float lsum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int nt = wave < 3 ? wave : i, mt = wave < 3 ? i : NT - 1;
+    if (wave == 3) {
+      if (i == 3) break;
+      if (i > 0) load2(nt);
+    }
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < N2; ++j)
+      acc = mfma(ld4(hid + (16 * mt + m + j / 2) * SH + 16 * (j % 2) + 4 * g), b2[j], acc);
+    const float wc = A.wch[16 * nt + m], cs = nt == 0 ? A.cs[0] : nt == 1 ? A.cs[1] : A.cs[2];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int hp = 16 * mt + 4 * g + v, p = a0 - 2 * R + hp;
+      float d = 0.f;
+      if (p >= lo && p < hi) {
+        const float e = acc[v] - tg[i][v] * cs * sc;
+        if (p >= a0 && p < a0 + kTrainSeg) lsum += wc * e * e;
+        d = 2.f * wc * e * A.norm;
+      }
+      dyl[hp * SY + 16 * nt + m] = f2bf(d);
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+  if (l == 0) red[wave] = lsum;
+  __syncthreads();
+  if (tid == 0)
+    A.loss[(size_t)b * gridDim.x + blockIdx.x] = (red[0] + red[1] + red[2] + red[3]) * A.norm;
+
+  // dy and the gradient at the hidden layer, channel-major (rows past the strip are zeros)
+#pragma unroll
+  for (int i = 0; i < kLbcCout * kTrainSeg / 4 / 256; ++i) {
+    const int e = tid + 256 * i, ch = e / (kTrainSeg / 4), q = e % (kTrainSeg / 4) * 4;
+    s4 o;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = (short)dyl[(2 * R + q + v) * SY + ch];
+    *reinterpret_cast<s4 *>(A.dy + ((size_t)b * kLbcCout + ch) * A.pitch + kPad + a0 + q) = o;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int nt = wave & 1, mt = (wave >> 1) * 2 + i;
+    f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      acc = mfma(ld4(dyl + (16 * mt + m + 3 * R - j / 3) * SY + 16 * (j % 3) + 4 * g), bb[j], acc);
+    const int a = a0 + 16 * mt + 4 * g;
+    s4 o;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = a + v < G ? (short)f2bf(acc[v]) : (short)0;
+    *reinterpret_cast<s4 *>(A.dh + ((size_t)b * kLbcHidden + 16 * nt + m) * A.pitch + kPad + a) = o;
+  }
+}
+
+// part[b][co][k][ci] = sum_p d[b, p, co] * in[b, p + k - R, ci] of both layers: one wave takes
+// a 16 x 16 tile for all taps over the whole strip, so that the sum keeps its order and the
+// taps are independent products.  A lane's four positions of the five taps lie in 16 bytes.
+// Bound by the memory's latency over the positions, hence kChunk products' operands ahead.
+__global__ __launch_bounds__(64) void k_train_weights(TrainStep A) {
+  typedef uint32_t u4a __attribute__((ext_vector_type(4), aligned(4)));
+  const int tile = blockIdx.x % 6, b = blockIdx.y;
+  const bool first = blockIdx.x < 6;
+  const int Co = first ? kLbcHidden : kLbcCout, Ci = first ? kLbcCin : kLbcHidden;
+  const int nci = Ci / 16, co0 = tile / nci * 16, ci0 = tile % nci * 16;
+  const int l = threadIdx.x, m = l & 15, g = l >> 4;
+  const uint16_t *ra = (first ? A.dh : A.dy) + ((size_t)b * Co + co0 + m) * A.pitch + kPad + 4 * g;
+  const uint16_t *rb = (first ? A.x : A.h) + ((size_t)b * Ci + ci0 + m) * A.pitch + kPad + 4 * g -
+                       kLbcTaps / 2;
+  struct Operands {
+    s4 a[kChunk];
+    u4a b[kChunk];
+  };
+  const auto load = [&](Operands &o, int c) {
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      o.a[i] = ld4(ra + 16 * (kChunk * c + i));
+      o.b[i] = *reinterpret_cast<const u4a *>(rb + 16 * (kChunk * c + i));
+    }
+  };
+  f4 acc[kLbcTaps] = {};
+  const auto multiply = [&](const Operands &o) {
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      const u4a w = o.b[i];
+      const uint32_t o0 = __builtin_amdgcn_alignbit(w[1], w[0], 16),
+                     o1 = __builtin_amdgcn_alignbit(w[2], w[1], 16),
+                     o2 = __builtin_amdgcn_alignbit(w[3], w[2], 16);
+      const uint32_t v[kLbcTaps][2] = {{w[0], w[1]}, {o0, o1}, {w[1], w[2]}, {o1, o2}, {w[2], w[3]}};
+#pragma unroll
+      for (int k = 0; k < kLbcTaps; ++k) {
+        s4 bv;
+        __builtin_memcpy(&bv, v[k], 8);
+        acc[k] = mfma(o.a[i], bv, acc[k]);
+      }
+    }
+  };
+  const int chunks = (A.G + 16 * kChunk - 1) / (16 * kChunk);
+  Operands even, odd;
+  load(even, 0);
+  for (int c = 0; c < chunks; c += 2) {     // (loads past the end read the last chunk again)
+    load(odd, min(c + 1, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(even);
+    if (c + 1 >= chunks) break;
+    load(even, min(c + 2, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(odd);
+  }
+  float *pb = (first ? A.part1 : A.part2) + (size_t)b * Co * kLbcTaps * Ci;
+#pragma unroll
+  for (int k = 0; k < kLbcTaps; ++k)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      pb[((size_t)(co0 + 4 * g + v) * kLbcTaps + k) * Ci + ci0 + m] = acc[k][v];
+}
+
+struct TrainLayer {
+  float *w, *m1, *m2;
+  uint16_t *wb, *wt;
+  const float *part;
+  int Co, Ci;
+};
+
+// One weight a thread: its samples' gradients in order (four loads in flight), Adam, the copies.
+__global__ __launch_bounds__(256) void k_train_update(TrainLayer first, TrainLayer second,
+                                                      const int32_t *__restrict__ side, int B,
+                                                      float lr, float b1, float b2, float eps,
+                                                      float c1, float c2) {
+  const TrainLayer &Y = blockIdx.z == 0 ? first : second;
+  const int n = Y.Co * kLbcTaps * Y.Ci, i = blockIdx.x * 256 + threadIdx.x;
+  const int s = blockIdx.y, l = threadIdx.x & 63;
+  const int at = min(i, n - 1);
+  float gi = 0.f;
+  for (int b0 = 0; b0 < B; b0 += 64) {
+    uint64_t mine = __ballot(b0 + l < B && side[min(b0 + l, B - 1)] == s);
+    while (mine) {
+      float v[4];
+      int got = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (!mine) break;
+        const int b = b0 + __builtin_ctzll(mine);
+        mine &= mine - 1;
+        v[j] = Y.part[(size_t)b * n + at];
+        got = j + 1;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < got) gi += v[j];
+    }
+  }
+  if (i >= n) return;
+  const size_t q = (size_t)s * n + i;
+  const float a = b1 * Y.m1[q] + (1.f - b1) * gi;
+  const float v = b2 * Y.m2[q] + (1.f - b2) * gi * gi;
+  Y.m1[q] = a;
+  Y.m2[q] = v;
+  const float w = Y.w[q] - lr * (a / c1) / (sqrtf(v / c2) + eps);
+  Y.w[q] = w;
+  const int ci = i % Y.Ci, k = i / Y.Ci % kLbcTaps, co = i / (Y.Ci * kLbcTaps);
+  const uint16_t h = f2bf(w);
+  Y.wb[q] = h;
+  Y.wt[(((size_t)s * Y.Ci + ci) * kLbcTaps + k) * Y.Co + co] = h;
 }
 
 // RMS of the pressure band of every frame and side: rms[f][s]
@@ -507,6 +800,63 @@ int fds_lbc_gather(const float *frames, const int32_t *run, const int32_t *step,
   hipLaunchKernelGGL(fds::k_gather, dim3((G + 255) / 256, B), dim3(256), 0, as_stream(stream),
                      frames, run, step, side, scale, x, t, T, D, G, L, comp_scale[0],
                      comp_scale[1], comp_scale[2]);
+  return last_launch();
+}
+
+int fds_lbc_train_workspace(int B, int G, int64_t *bytes) {
+  if (B < 1 || B > 65535 || G < 1) return FDS_E_ARG;
+  const int64_t rows = (int64_t)B * 2 * (fds::kLbcCin + fds::kLbcHidden);
+  const int64_t part = (int64_t)B * 2 * fds::kLbcCin * fds::kLbcTaps * fds::kLbcHidden;
+  *bytes = rows * fds::train_pitch(G) * 2 + part * 4;
+  return 0;
+}
+
+int fds_lbc_train(const float *frames, const int32_t *run, const int32_t *step,
+                  const int32_t *side, const float *scale, const float *wch,
+                  const fds_lbc_layer *layers, void *work, float *loss, int iters, int B, int T,
+                  int D, int G, int L, const float *comp_scale, float lr, float b1, float b2,
+                  float eps, int first_step, void *stream) {
+  if (iters < 1 || B < 1 || B > 65535 || T < 2 || G < 2 * L + 1 || L != fds::kLbcDepth ||
+      D < L + fds::kLbcBand || first_step < 1)
+    return FDS_E_ARG;
+  const hipStream_t q = as_stream(stream);
+  const int segs = (G + fds::kTrainSeg - 1) / fds::kTrainSeg;
+  constexpr int n = fds::kLbcCin * fds::kLbcTaps * fds::kLbcHidden;
+  fds::TrainStep a{};
+  a.frames = frames;
+  a.wch = wch;
+  a.w1b = layers[0].wb;
+  a.w2b = layers[1].wb;
+  a.w2t = layers[1].wt;
+  a.T = T, a.D = D, a.G = G, a.L = L;
+  a.pitch = fds::train_pitch(G);
+  for (int c = 0; c < 3; ++c) a.cs[c] = comp_scale[c];
+  a.norm = (float)(1.0 / ((double)B * G * 4.0));
+  a.part1 = static_cast<float *>(work);
+  a.part2 = a.part1 + (size_t)B * n;
+  a.x = reinterpret_cast<uint16_t *>(a.part2 + (size_t)B * n);
+  a.h = a.x + (size_t)B * fds::kLbcCin * a.pitch;
+  a.dy = a.h + (size_t)B * fds::kLbcHidden * a.pitch;
+  a.dh = a.dy + (size_t)B * fds::kLbcCout * a.pitch;
+  a.loss = loss;
+  const fds::TrainLayer y[2] = {
+      {layers[0].w, layers[0].m, layers[0].v, layers[0].wb, layers[0].wt, a.part1,
+       fds::kLbcHidden, fds::kLbcCin},
+      {layers[1].w, layers[1].m, layers[1].v, layers[1].wb, layers[1].wt, a.part2,
+       fds::kLbcCout, fds::kLbcHidden}};
+  hipLaunchKernelGGL(fds::k_train_pads, dim3(B * 2 * (fds::kLbcCin + fds::kLbcHidden)), dim3(64),
+                     0, q, a.x, G, a.pitch);
+  for (int it = 0; it < iters; ++it) {
+    a.run = run + (size_t)it * B;
+    a.step = step + (size_t)it * B;
+    a.side = side + (size_t)it * B;
+    a.scale = scale + (size_t)it * B;
+    const float t = (float)(first_step + it), c1 = 1.f - powf(b1, t), c2 = 1.f - powf(b2, t);
+    hipLaunchKernelGGL(fds::k_train_grads, dim3(segs, B), dim3(256), 0, q, a);
+    hipLaunchKernelGGL(fds::k_train_weights, dim3(12, B), dim3(64), 0, q, a);
+    hipLaunchKernelGGL(fds::k_train_update, dim3((n + 255) / 256, 4, 2), dim3(256), 0, q, y[0],
+                       y[1], a.side, B, lr, b1, b2, eps, c1, c2);
+  }
   return last_launch();
 }
 

@@ -36,6 +36,8 @@ from . import regions
 
 LAYER, BAND, CIN, HIDDEN, COUT, TAPS = 16, 8, 48, 32, 48, 5
 DEPTH_REC = LAYER + BAND
+SEGMENT = 64           # positions per partial sum of the training loss
+CALL_ITERS = 256       # training iterations enqueued at once, at most (bounds their sample lists)
 
 
 def lbc_cell(side, d, a, g):
@@ -201,19 +203,11 @@ class LearnedBoundary:
         return arr.shape
 
     # ------------------------------------------------------------------ training
-    def _forward(self, x, side, B):
-        t = self.torch
-        P = self.G
-        h = t.empty((B, P, HIDDEN), dtype=t.float32, device=self.dev)
-        hb = t.empty((B, P, HIDDEN), dtype=t.int16, device=self.dev)
-        y = t.empty((B, P, COUT), dtype=t.float32, device=self.dev)
-        nat.check(self.lib.fds_lbc_conv_fwd(self._p(x), self._p(self.w1b), self._p(side),
-                                            self._p(h), self._p(hb), B, P, CIN, HIDDEN, TAPS,
-                                            self._stream()))
-        nat.check(self.lib.fds_lbc_conv_fwd(self._p(hb), self._p(self.w2b), self._p(side),
-                                            self._p(y), None, B, P, HIDDEN, COUT, TAPS,
-                                            self._stream()))
-        return hb, y
+    def _layers(self):
+        """The two layers as ``fds_lbc_layer`` pairs (pointers of the tensors as they are now)."""
+        rows = ((self.w1, self.opt[0], self.opt[1], self.w1b, self.w1t),
+                (self.w2, self.opt[2], self.opt[3], self.w2b, self.w2t))
+        return (nat.LbcLayer * 2)(*[nat.LbcLayer(*[t.data_ptr() for t in row]) for row in rows])
 
     def train(self, iters=1500, batch=32, lr=2e-3, seed=0, log_every=0):
         t = self.torch
@@ -223,60 +217,36 @@ class LearnedBoundary:
                 if self.rms[r, s, side] > 0.02 * self.rms[r].max()]
         cand = np.array(cand, dtype=np.int64)
         B, P = batch, self.G
-        x = t.empty((B, P, CIN), dtype=t.int16, device=self.dev)
-        tgt = t.empty((B, P, COUT), dtype=t.float32, device=self.dev)
-        dyb = t.empty((B, P, COUT), dtype=t.int16, device=self.dev)
-        dh = t.empty((B, P, HIDDEN), dtype=t.float32, device=self.dev)
-        dhb = t.empty((B, P, HIDDEN), dtype=t.int16, device=self.dev)
-        part1 = t.empty((B, HIDDEN, TAPS, CIN), dtype=t.float32, device=self.dev)
-        part2 = t.empty((B, COUT, TAPS, HIDDEN), dtype=t.float32, device=self.dev)
-        g1 = t.empty_like(self.w1)
-        g2 = t.empty_like(self.w2)
+        size = ct.c_int64()
+        if iters > 0:
+            nat.check(self.lib.fds_lbc_train_workspace(B, P, ct.byref(size)))
+        work = t.empty(size.value, dtype=t.uint8, device=self.dev)
+        loss = t.empty(B * -(-P // SEGMENT), dtype=t.float32, device=self.dev)
         wch = np.where(np.arange(COUT) % LAYER >= LAYER - 4, 1.0, 0.05).astype(np.float32)
         wch_d = t.from_numpy(wch).to(self.dev)
-        nblk = 256
-        loss_part = t.empty(nblk, dtype=t.float32, device=self.dev)
         cs = self.cs.ctypes.data_as(ct.c_void_p)
         history = []
-        for it in range(iters):
-            pick = cand[rng.integers(0, len(cand), size=B)]
-            run = t.from_numpy(pick[:, 0].astype(np.int32)).to(self.dev)
-            step = t.from_numpy(pick[:, 1].astype(np.int32)).to(self.dev)
-            side = t.from_numpy(pick[:, 2].astype(np.int32)).to(self.dev)
-            scale = t.from_numpy((1.0 / self.rms[pick[:, 0], pick[:, 1], pick[:, 2]])
-                                 .astype(np.float32)).to(self.dev)
-            lo = t.from_numpy(np.where(pick[:, 2] < 2, 0, LAYER).astype(np.int32)).to(self.dev)
-            hi = t.from_numpy(np.where(pick[:, 2] < 2, P, P - LAYER).astype(np.int32)).to(self.dev)
-            nat.check(self.lib.fds_lbc_gather(self._p(self.frames), self._p(run), self._p(step),
-                                              self._p(side), self._p(scale), self._p(x),
-                                              self._p(tgt), B, self.T, DEPTH_REC, P, LAYER, cs,
-                                              self._stream()))
-            hb, y = self._forward(x, side, B)
-            norm = 1.0 / (B * P * 4.0)
-            nat.check(self.lib.fds_lbc_mse(self._p(y), self._p(tgt), self._p(lo), self._p(hi),
-                                           self._p(wch_d), self._p(dyb), self._p(loss_part),
-                                           nblk, B, P, COUT, norm, self._stream()))
-            # layer 2 weights, then back through layer 2, then layer 1 weights
-            nat.check(self.lib.fds_lbc_conv_bwd_weight(self._p(dyb), self._p(hb), self._p(part2),
-                                                       B, P, HIDDEN, COUT, TAPS, self._stream()))
-            nat.check(self.lib.fds_lbc_reduce_weight(self._p(part2), self._p(side), self._p(g2),
-                                                     B, 4, COUT * TAPS * HIDDEN, self._stream()))
-            nat.check(self.lib.fds_lbc_conv_bwd_data(self._p(dyb), self._p(self.w2t),
-                                                     self._p(side), self._p(dh), self._p(dhb),
-                                                     B, P, HIDDEN, COUT, TAPS, self._stream()))
-            nat.check(self.lib.fds_lbc_conv_bwd_weight(self._p(dhb), self._p(x), self._p(part1),
-                                                       B, P, CIN, HIDDEN, TAPS, self._stream()))
-            nat.check(self.lib.fds_lbc_reduce_weight(self._p(part1), self._p(side), self._p(g1),
-                                                     B, 4, HIDDEN * TAPS * CIN, self._stream()))
-            self.adam_step += 1
-            for w, g, m1, m2 in ((self.w1, g1, self.opt[0], self.opt[1]),
-                                 (self.w2, g2, self.opt[2], self.opt[3])):
-                nat.check(self.lib.fds_lbc_adam(self._p(w), self._p(m1), self._p(m2), self._p(g),
-                                                w.numel(), lr, 0.9, 0.999, 1e-8, self.adam_step,
-                                                self._stream()))
-            self._pack()
-            if log_every and (it % log_every == 0 or it == iters - 1):
-                history.append((it, float(loss_part.sum().item())))
+        it = 0
+        while it < iters:
+            # one call enqueues all iterations up to the next logged one
+            n = min(iters - it, CALL_ITERS)
+            if log_every:
+                n = next((k for k in range(1, n) if (it + k - 1) % log_every == 0), n)
+            pick = np.stack([cand[rng.integers(0, len(cand), size=B)] for _ in range(n)])
+            scale = 1.0 / self.rms[pick[..., 0], pick[..., 1], pick[..., 2]]
+            lists = np.empty((4, n, B), np.int32)
+            lists[:3] = np.moveaxis(pick, -1, 0)
+            lists[3] = scale.astype(np.float32).view(np.int32)
+            run, step, side, scale = t.from_numpy(lists).to(self.dev)
+            nat.check(self.lib.fds_lbc_train(self._p(self.frames), self._p(run), self._p(step),
+                                             self._p(side), self._p(scale), self._p(wch_d),
+                                             self._layers(), self._p(work), self._p(loss), n, B,
+                                             self.T, DEPTH_REC, P, LAYER, cs, lr, 0.9, 0.999,
+                                             1e-8, self.adam_step + 1, self._stream()))
+            self.adam_step += n
+            it += n
+            if log_every and ((it - 1) % log_every == 0 or it == iters):
+                history.append((it - 1, float(loss.sum().item())))
         self.torch.cuda.synchronize(self.dev)
         return history
 

@@ -223,6 +223,85 @@ def test_mfma_training_kernels_match_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('g, B, iters', [(33, 1, 1), (64, 3, 2), (65, 70, 2), (129, 5, 3),
+                                         (190, 32, 2)])
+def test_training_iterations_equal_the_single_kernels(g, B, iters):
+    """fds_lbc_train against the kernels of one operation each, which the oracle checks above:
+    the same sums in the same order, so the same bits; the loss is summed in another order
+    (a few hundred float32 terms: 1e-5).  Strips shorter than a segment, of whole segments and
+    with remainders; sides without a sample; more samples than lanes."""
+    torch = _torch()
+    lib = nat.load()
+    rng = np.random.default_rng(g)
+    T, D, L, K, Ci, Ch, Co = 6, 24, 16, 5, 48, 32, 48
+    frames = torch.from_numpy(rng.standard_normal((2 * T, 3, 4, D, g)).astype(np.float32)).cuda()
+    pick = [rng.integers(lo, hi, (iters, B)).astype(np.int32)
+            for lo, hi in ((0, 2), (1, T), (0, 4 if B > 3 else 2))]
+    scale = rng.uniform(0.5, 2.0, (iters, B)).astype(np.float32)
+    run, step, side, scale = (torch.from_numpy(a).cuda() for a in pick + [scale])
+    wch = torch.from_numpy(rng.random(Co).astype(np.float32)).cuda()
+    cs = np.array([1.0, 2.0, 0.5], np.float32)
+    s = ct.c_void_p(torch.cuda.current_stream().cuda_stream)
+    p = lambda t: ct.c_void_p(t.data_ptr())
+
+    def layers():
+        gen = torch.Generator().manual_seed(g)
+        out = []
+        for co, ci in ((Ch, Ci), (Co, Ch)):
+            w = (torch.randn(4, co, K, ci, generator=gen) * 0.1).cuda()
+            wb = torch.empty(w.shape, dtype=torch.int16, device='cuda')
+            wt = torch.empty((4, ci, K, co), dtype=torch.int16, device='cuda')
+            nat.check(lib.fds_lbc_pack(p(w), p(wb), p(wt), 4, co, K, ci, s))
+            out.append([w, torch.zeros_like(w), torch.zeros_like(w), wb, wt])
+        return out
+
+    got = layers()
+    size = ct.c_int64()
+    nat.check(lib.fds_lbc_train_workspace(B, g, ct.byref(size)))
+    work = torch.full((size.value,), 0xff, dtype=torch.uint8, device='cuda')
+    loss = torch.empty(B * -(-g // 64), dtype=torch.float32, device='cuda')
+    arg = (nat.LbcLayer * 2)(*[nat.LbcLayer(*[t.data_ptr() for t in row]) for row in got])
+    nat.check(lib.fds_lbc_train(p(frames), p(run), p(step), p(side), p(scale), p(wch), arg,
+                                p(work), p(loss), iters, B, T, D, g, L,
+                                cs.ctypes.data_as(ct.c_void_p), 1e-2, 0.9, 0.999, 1e-8, 3, s))
+    want = layers()
+    new = lambda dt, *shape: torch.empty(shape, dtype=dt, device='cuda')
+    f4, i2 = torch.float32, torch.int16
+    x, tgt = new(i2, B, g, Ci), new(f4, B, g, Co)
+    h, hb, y, dyb = new(f4, B, g, Ch), new(i2, B, g, Ch), new(f4, B, g, Co), new(i2, B, g, Co)
+    dh, dhb = new(f4, B, g, Ch), new(i2, B, g, Ch)
+    lp = new(f4, 64)
+    (w1, m1, v1, w1b, w1t), (w2, m2, v2, w2b, w2t) = want
+    part1, part2 = new(f4, B, Ch, K, Ci), new(f4, B, Co, K, Ch)
+    g1, g2 = torch.empty_like(w1), torch.empty_like(w2)
+    for i in range(iters):
+        sd = side[i]
+        edge = torch.where(sd < 2, 0, L).int()
+        lo, hi = edge, (g - edge).int()
+        nat.check(lib.fds_lbc_gather(p(frames), p(run[i]), p(step[i]), p(sd), p(scale[i]), p(x),
+                                     p(tgt), B, T, D, g, L, cs.ctypes.data_as(ct.c_void_p), s))
+        nat.check(lib.fds_lbc_conv_fwd(p(x), p(w1b), p(sd), p(h), p(hb), B, g, Ci, Ch, K, s))
+        nat.check(lib.fds_lbc_conv_fwd(p(hb), p(w2b), p(sd), p(y), None, B, g, Ch, Co, K, s))
+        nat.check(lib.fds_lbc_mse(p(y), p(tgt), p(lo), p(hi), p(wch), p(dyb), p(lp), 64, B, g, Co,
+                                  1.0 / (B * g * 4.0), s))
+        nat.check(lib.fds_lbc_conv_bwd_weight(p(dyb), p(hb), p(part2), B, g, Ch, Co, K, s))
+        nat.check(lib.fds_lbc_reduce_weight(p(part2), p(sd), p(g2), B, 4, Co * K * Ch, s))
+        nat.check(lib.fds_lbc_conv_bwd_data(p(dyb), p(w2t), p(sd), p(dh), p(dhb), B, g, Ch, Co, K,
+                                            s))
+        nat.check(lib.fds_lbc_conv_bwd_weight(p(dhb), p(x), p(part1), B, g, Ci, Ch, K, s))
+        nat.check(lib.fds_lbc_reduce_weight(p(part1), p(sd), p(g1), B, 4, Ch * K * Ci, s))
+        for (w, m, v, wb, wt), gr, co, ci in ((want[0], g1, Ch, Ci), (want[1], g2, Co, Ch)):
+            nat.check(lib.fds_lbc_adam(p(w), p(m), p(v), p(gr), w.numel(), 1e-2, 0.9, 0.999, 1e-8,
+                                       3 + i, s))
+            nat.check(lib.fds_lbc_pack(p(w), p(wb), p(wt), 4, co, K, ci, s))
+    torch.cuda.synchronize()
+    for a, b, layer in zip(got, want, (1, 2)):
+        for u, v, name in zip(a, b, ('w', 'm', 'v', 'wb', 'wt')):
+            assert torch.equal(u, v), (layer, name, (u != v).sum().item())
+    assert np.isclose(loss.sum().item(), lp.sum().item(), rtol=1e-5)
+
+
+@pytest.mark.gpu
 def test_fused_inference_writes_oracle_layer():
     """One step of a 64 x 64 FP32 grid with the learned layer: the layer cells equal the
     network evaluated by the oracle on the band rows (bf16 inputs and hidden activations
