@@ -212,10 +212,9 @@ class LearnedBoundary:
     def train(self, iters=1500, batch=32, lr=2e-3, seed=0, log_every=0):
         t = self.torch
         rng = np.random.default_rng(seed)
-        runs, T, _ = self.rms.shape
-        cand = [(r, s, side) for r in range(runs) for s in range(1, T) for side in range(4)
-                if self.rms[r, s, side] > 0.02 * self.rms[r].max()]
-        cand = np.array(cand, dtype=np.int64)
+        T = self.rms.shape[1]
+        loud = self.rms > 0.02 * self.rms.max(axis=(1, 2), keepdims=True)
+        cand = np.argwhere(loud[:, 1:T]) + (0, 1, 0)      # (run, step, side), steps from 1 on
         B, P = batch, self.G
         size = ct.c_int64()
         if iters > 0:
