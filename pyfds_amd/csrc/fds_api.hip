@@ -737,7 +737,7 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
         point_rows.push_back((int32_t)points.size());
         for (; e < oev[k].ptr[t + 1] && oev[k].pos[e] / R.w + R.rmin == r; ++e) {
           const int col = oev[k].pos[e] % R.w + R.cmin;
-          points.push_back(fds::FusedPoint{col, oev[k].id[e]});
+          points.push_back(fds::FusedPoint{(uint32_t)(col | k << 6 | r << 8), oev[k].id[e]});
           w[(r + g) * 64 + col] |= fds::kFusedRecord << k;
         }
       }

@@ -43,7 +43,8 @@ struct FusedClass {
 
 // Fused kernels: one recorded point of a strip (lane of its column, output slot).
 struct FusedPoint {
-  int32_t col, id;
+  uint32_t where;   // column | component << 6 | row << 8
+  int32_t id;
 };
 
 constexpr int kPalSlots = 8;               // coefficients of a material class

@@ -124,14 +124,17 @@ struct FusedEvents {
   const OutView *out;
   const FusedPoint *point;
   bool chained;             // some class has a next entry
+  bool few;                 // the tile has at most 64 recorded points, one a lane:
+  uint32_t where;           // this lane's (FusedPoint; none: all bits)
+  int32_t id;
   const int32_t *rows;      // first point of (component, row of the strip), rows + 1 a component
   int stride;
   int64_t row;              // output row of stage 0
 };
 
 // What a row's event words hold (bits of a uniform mask): boundary cells of component k
-// (1 << k), recorded points.
-constexpr uint32_t kRowRecord = 8u;
+// (1 << k), its recorded points (8 << k).
+constexpr uint32_t kRowRecord = 0x38u;
 
 // Entry of component K's boundary class in event word w.
 template <int K>
@@ -179,20 +182,38 @@ __device__ __forceinline__ void fused_terms(const FusedEvents &E, int s, uint32_
   }
 }
 
-// Recorded points of row r of the strip at stage s: lane q takes the row's point q (its value
-// comes from the lane of its column; components K0 .. K1 - 1).
+// Recorded points of row r of the strip at stage s (components K0 .. K1 - 1; `any`: what the row
+// holds).  A point's value comes from the lane of its column.  The points of the usual tile are in
+// its lanes' registers; lists are read only for more than 64 of them.  (With lists for all, a row
+// with a point cost three dependent lookups a stage, and the addresses of all stages 30 registers
+// that every tile paid for in occupancy: 1056^2 FP32 with a source and four points 19.2 us a
+// launch of six steps then, 17.6 so; 4096^2 Thermal2D Kahan 16.5 us a step and 13.5.)
 template <typename T, bool KAHAN, int K0 = 0, int K1 = 3>
-__device__ __forceinline__ void fused_record(const FusedEvents &E, int s, int r, T p, T cp, T vx,
-                                             T cvx, T vy, T cvy) {
+__device__ __forceinline__ void fused_record(const FusedEvents &E, int s, int r, uint32_t any, T p,
+                                             T cp, T vx, T cvx, T vy, T cvy) {
   const int t = threadIdx.x;
+#pragma unroll
   for (int k = K0; k < K1; ++k) {
+    if (!(any & (8u << k))) continue;
     const T x = k == 0 ? p : k == 1 ? vx : vy, c = k == 0 ? cp : k == 1 ? cvx : cvy;
+    int64_t row = E.row;
+    __asm__ volatile("" : "+v"(row));     // (else the addresses of all stages stay in registers)
+    double *buf = E.out[k].buf + (row + s) * E.out[k].m;
+    if (E.few) {
+      const int col = E.where & 63;
+      const T xv = __shfl(x, col), cv = KAHAN ? __shfl(c, col) : T(0);
+      int32_t id = E.id;
+      __asm__ volatile("" : "+v"(id));
+      if (E.where >> 6 == (uint32_t)(k | r << 2)) buf[id] = out_value<T, KAHAN>(xv, cv);
+      continue;
+    }
     const int e0 = E.rows[k * E.stride + r], e1 = E.rows[k * E.stride + r + 1];
     for (int e = e0; e < e1; e += 64) {
       const bool in = e + t < e1;
       const FusedPoint q = E.point[in ? e + t : e0];
-      const T xv = __shfl(x, q.col), cv = KAHAN ? __shfl(c, q.col) : T(0);
-      if (in) E.out[k].buf[(E.row + s) * E.out[k].m + q.id] = out_value<T, KAHAN>(xv, cv);
+      const int col = q.where & 63;
+      const T xv = __shfl(x, col), cv = KAHAN ? __shfl(c, col) : T(0);
+      if (in) buf[q.id] = out_value<T, KAHAN>(xv, cv);
     }
   }
 }
@@ -214,6 +235,14 @@ __device__ __forceinline__ FusedEvents fused_events(const StepArgs<T> &a, int sl
   E.stride = stride;
   E.rows = fe.point_rows + (int64_t)slot * 3 * stride;
   E.row = row;
+  const int p0 = E.rows[0], np = E.rows[3 * stride - 1] - p0;
+  E.few = np <= 64;
+  E.where = ~0u;
+  E.id = 0;
+  if (E.few && t < np) {
+    E.where = fe.points[p0 + t].where;
+    E.id = fe.points[p0 + t].id;
+  }
   const int e0 = fe.cls_ptr[slot], e1 = fe.cls_ptr[slot + 1];
   bool chained = false;
   if (t == 0) {
@@ -237,7 +266,8 @@ __device__ __forceinline__ FusedEvents fused_events(const StepArgs<T> &a, int sl
 __device__ __forceinline__ uint32_t fused_row_flags(uint32_t w) {
   if (!__any(w != 0)) return 0;
   return (__any(fused_class<0>(w) != 0) ? 1u : 0u) | (__any(fused_class<1>(w) != 0) ? 2u : 0u) |
-         (__any(fused_class<2>(w) != 0) ? 4u : 0u) | (__any((w >> 24) != 0) ? kRowRecord : 0u);
+         (__any(fused_class<2>(w) != 0) ? 4u : 0u) | (__any(w & kFusedRecord) ? 8u : 0u) |
+         (__any(w & kFusedRecord << 1) ? 16u : 0u) | (__any(w & kFusedRecord << 2) ? 32u : 0u);
 }
 
 // One stage of the lossless acoustic step: takes row r in x, leaves row r - 1 of the next time
@@ -271,7 +301,7 @@ __device__ __forceinline__ void fused_acoustic_stage(FuCarry<T> &c, FuRow<T> &x,
     if (any & 4u) fused_bound<T, KAHAN, 2>(E, m[2], s, w, vy, cvy);
   }
   if constexpr (EV) {
-    if (any & kRowRecord) fused_record<T, KAHAN>(E, s, r, x.p, x.cp, vx, cvx, vy, cvy);
+    if (any & kRowRecord) fused_record<T, KAHAN>(E, s, r, any, x.p, x.cp, vx, cvx, vy, cvy);
   }
   const T kvy = k.ky * vy;
   const T dy = (-c.kvy) + kvy;
@@ -310,7 +340,7 @@ __device__ __forceinline__ void fused_thermal_stage(FuCarry<T> &c, FuRow<T> &x, 
     if (any & 4u) fused_bound<T, false, 2>(E, m[2], s, w, fy, none);
   }
   if constexpr (EV) {
-    if (any & kRowRecord) fused_record<T, KAHAN>(E, s, r, x.p, x.cp, fx, T(0), fy, T(0));
+    if (any & kRowRecord) fused_record<T, KAHAN>(E, s, r, any, x.p, x.cp, fx, T(0), fy, T(0));
   }
   const T gqy = k.ky * fy;
   const T dy = (-c.kvy) + gqy;

@@ -64,8 +64,8 @@ __device__ __forceinline__ void fused_lossy_stage(LfCarry<T> &c, FuRow<T> &x, co
     fused_terms(E, s, wa, fa & 1u, ma);
     fused_terms(E, s, wc, fc & 6u, mc);
     if (fa & 1u) fused_bound<T, KAHAN, 0>(E, ma[0], s, wa, x.p, x.cp);
-    if (fa & kRowRecord)
-      fused_record<T, KAHAN, 0, 1>(E, s, r, x.p, x.cp, T(0), T(0), T(0), T(0));
+    if (fa & 8u)
+      fused_record<T, KAHAN, 0, 1>(E, s, r, fa, x.p, x.cp, T(0), T(0), T(0), T(0));
   }
   // ---- row r
   const T bpx = ka.bx * x.p;
@@ -112,8 +112,8 @@ __device__ __forceinline__ void fused_lossy_stage(LfCarry<T> &c, FuRow<T> &x, co
   }
   if constexpr (EV) {
     if (fc & 4u) fused_bound<T, KAHAN, 2>(E, mc[2], s, wc, vy, cvy);
-    if (fc & kRowRecord)
-      fused_record<T, KAHAN, 1, 3>(E, s, r - 1, T(0), T(0), vx, cvx, vy, cvy);
+    if (fc & kRowRecord & ~8u)
+      fused_record<T, KAHAN, 1, 3>(E, s, r - 1, fc, T(0), T(0), vx, cvx, vy, cvy);
   }
   const T kvy = ky * vy;
   // ---- row r - 2: its pressure
