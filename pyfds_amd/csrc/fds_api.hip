@@ -241,6 +241,9 @@ struct fds_ctx {
   const uint16_t *lbc_w1 = nullptr, *lbc_w2 = nullptr;
   int lbc_layer = 0;
   float lbc_cs[3] = {1.f, 1.f, 1.f};
+  bool lbc_ring = false;      // several steps per launch (fds_lbc_ring.hip)
+  DevBuf lbc_rec, lbc_cells, lbc_packed;   // recorded points of its band, its cells, its weights
+  int lbc_nrec = 0;
   // non-finite detection: scans in every graph chunk and after every run; the result
   // (dyn[kDynNonfinite]) is copied to nf_stage[slot] (slot kMaxFlights: synchronous runs)
   bool nf_check = false;
@@ -414,6 +417,32 @@ int line_variant(int64_t n, int cpt, int fam) {
   return -1;
 }
 
+// Depth of a cell from the rim of a square grid.
+int rim_depth(const fds_ctx *c, int64_t cell) {
+  const int64_t x = cell % c->nx, y = cell / c->nx;
+  return (int)std::min(std::min(x, c->nx - 1 - x), std::min(y, c->ny - 1 - y));
+}
+
+// Whether a learned boundary can take S steps per launch (fds_lbc_ring.hip): FP32, isotropic
+// lossless, no boundary cell where the frame is computed anew, no recorded point in the layer and
+// few in the band.  Any other field steps one by one (1056^2: 19.8 us a step then, 7.9 so).
+bool can_ring(const fds_ctx *c, int S) {
+  if (is_kahan(c) || c->lossy || c->flow || c->coupled || !c->iso_b || !c->iso_k ||
+      !fds::lbc_ring_fits(c->nx, S))
+    return false;
+  int records = 0;
+  for (int k = 0; k < 3; ++k) {
+    for (int64_t q : c->comp[k].cells)
+      if (rim_depth(c, q) < fds::kLbcDepth + fds::kLbcBand + S) return false;
+    for (int64_t q : c->comp[k].out_cells) {
+      const int d = rim_depth(c, q);
+      if (d < fds::kLbcDepth) return false;
+      if (d < fds::kLbcDepth + fds::kLbcBand) ++records;
+    }
+  }
+  return records <= fds::kRingRecords;
+}
+
 // Layout of the fused engine: stages per launch and strip height.
 //
 // Stages: a launch's time grows slowly with them (2048^2 FP64 acoustics: 36 us at 4, 42 us at 6),
@@ -431,13 +460,13 @@ int line_variant(int64_t n, int cpt, int fam) {
 // measured best or within 3 % of it (lossy 5 %) from 1024 x 1536 (4-6 rows) over 2048^2 (12) to
 // 4096 x 3000 (24-48).
 int choose_fused(fds_ctx *c) {
-  const bool each = c->lbc_w1 || c->flow || c->coupled;
   const bool lossy = c->lossy && c->family == kAcoustic;
   int S = c->n < (1 << 18) ? 4 : fds::kFusedMax;
   if (lossy && c->axi) S = c->n < (1 << 22) ? 2 : 3;
   else if (lossy) S = c->elem == 4 && c->n >= (1 << 20) ? fds::kFusedLossyMax : 3;
   if (c->fused_stages) S = c->fused_stages;
-  if (each) S = 1;
+  c->lbc_ring = c->lbc_w1 && can_ring(c, S);
+  if ((c->lbc_w1 && !c->lbc_ring) || c->flow || c->coupled) S = 1;
   const int64_t sx = 64 - 2 * S - (lossy ? 1 : 0), across = (c->nx + sx - 1) / sx;
   const int64_t strips = (lossy ? 16 : 24) * (int64_t)c->num_cu;
   const int64_t want = (across * c->ny + strips / 2) / strips;
@@ -465,6 +494,7 @@ int choose_fused(fds_ctx *c) {
 int choose_tiles(fds_ctx *c) {
   c->streaming = false;
   c->fused = false;
+  c->lbc_ring = false;
   c->line = false;
   c->fuse = 1;
   c->ghost = 0;
@@ -743,6 +773,24 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
       }
     }
     cls_ptr.push_back((int32_t)cls.size());
+  }
+  if (c->lbc_ring) {
+    std::vector<fds::LbcRec> rec;
+    for (int k = 0; k < 3; ++k)
+      for (size_t q = 0; q < c->comp[k].out_cells.size(); ++q)
+        if (rim_depth(c, c->comp[k].out_cells[q]) < fds::kLbcDepth + fds::kLbcBand)
+          rec.push_back(fds::LbcRec{(int32_t)c->comp[k].out_cells[q], k, (int32_t)q});
+    c->lbc_nrec = (int)rec.size();
+    HIP_TRY(upload(c->lbc_rec, rec, c->stream));
+    fds::LbcRing r{};
+    r.g = (int)c->nx;
+    r.depth = c->fuse;
+    r.rec = c->lbc_rec.as<const fds::LbcRec>();
+    r.nrec = c->lbc_nrec;
+    HIP_TRY(c->lbc_cells.ensure(fds::lbc_ring_cells_bytes(r)));
+    HIP_TRY(c->lbc_packed.ensure(fds::lbc_ring_packed_bytes()));
+    fds::launch_ring_cells(r, c->lbc_cells.p, c->stream);
+    HIP_TRY(hipGetLastError());
   }
   c->fev_rows = rows;
   c->fev_nslots = nslots;
@@ -1134,10 +1182,37 @@ void launch_lbc<float>(fds_ctx *c, const fds::StepArgs<float> &a) {
   fds::launch_lbc_step(st, c->stream);
 }
 
+template <typename T>
+void launch_ring(fds_ctx *, const fds::StepArgs<T> &, int) {}
+
+template <>
+void launch_ring<float>(fds_ctx *c, const fds::StepArgs<float> &a, int stages) {
+  fds::LbcRing r{};
+  for (int k = 0; k < 3; ++k) {
+    r.in[k] = a.in[k];
+    r.out[k] = a.out[k];
+    r.rows[k] = a.outp[k].buf;
+    r.m[k] = a.outp[k].m;
+    r.cs[k] = c->lbc_cs[k];
+  }
+  r.b = a.coef[FDS_C_BX];
+  r.k = a.coef[FDS_C_KX];
+  r.packed = c->lbc_packed.p;
+  r.cells = c->lbc_cells.p;
+  r.rec = c->lbc_rec.as<const fds::LbcRec>();
+  r.nrec = c->lbc_nrec;
+  r.dyn = a.dyn;
+  r.row = a.k;
+  r.g = (int)c->nx;
+  r.stages = stages;
+  r.depth = c->fuse;
+  fds::launch_lbc_ring(r, c->stream);
+}
+
 // Time steps per launch: the streaming shapes' fused stage count (one step per launch when a
 // per-step learned boundary follows the step kernel).
 int step_group(const fds_ctx *c) {
-  return (c->streaming && !c->lbc_w1 && !c->flow) ? c->fuse : 1;
+  return (c->streaming && (!c->lbc_w1 || c->lbc_ring) && !c->flow) ? c->fuse : 1;
 }
 
 // Launch `stages` fused steps (1 <= stages <= step_group(c)) starting at step k of the launch
@@ -1168,7 +1243,8 @@ int launch_step(fds_ctx *c, int parity, int k, bool store, int stages) {
     HIP_TRY(hipGetLastError());
   }
   if (c->lbc_w1) {
-    launch_lbc<T>(c, a);
+    if (stages > 1) launch_ring<T>(c, a, stages);
+    else launch_lbc<T>(c, a);
     HIP_TRY(hipGetLastError());
   }
   return 0;
@@ -1681,7 +1757,7 @@ int fds_set_boundaries(fds_ctx *c, int comp, int64_t ncell, const int64_t *cells
   HIP_TRY(upload(cp.d_off, cp.off, c->stream));
   HIP_TRY(upload(cp.d_stride, cp.stride, c->stream));
   HIP_TRY(upload(cp.d_table, cp.table, c->stream));
-  if (c->fused_over) {
+  if (c->fused_over || c->lbc_w1) {
     c->fused_over = false;
     if (int rc = choose_tiles(c)) return rc;
   }
@@ -1699,6 +1775,8 @@ int fds_set_outputs(fds_ctx *c, int comp, int64_t m, const int64_t *cells) {
       return fail(FDS_E_INDEX, "output cell %lld out of range", (long long)cells[k]);
   Comp &cp = c->comp[comp];
   cp.out_cells.assign(cells, cells + m);
+  if (c->lbc_w1)
+    if (int rc = choose_tiles(c)) return rc;
   c->events_dirty = true;
   touch(c);
   return 0;
@@ -1798,6 +1876,10 @@ int prepare_run(fds_ctx *c, int64_t start, int64_t nsteps) {
   }
   hipLaunchKernelGGL(k_set_dyn, dim3(1), dim3(64), 0, c->stream, c->dyn.as<int64_t>(), start);
   HIP_TRY(hipGetLastError());
+  if (c->lbc_ring) {       // the caller may have trained on since the last run
+    fds::launch_ring_pack(c->lbc_w1, c->lbc_w2, c->lbc_packed.p, c->stream);
+    HIP_TRY(hipGetLastError());
+  }
   if (c->nf_check) {
     hipLaunchKernelGGL(k_nonfinite_reset, dim3(1), dim3(64), 0, c->stream, c->dyn.as<int64_t>());
     HIP_TRY(hipGetLastError());

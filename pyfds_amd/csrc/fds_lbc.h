@@ -12,6 +12,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace fds {
@@ -48,5 +49,38 @@ struct LbcStep {
 
 // Launch the fused inference kernel for one step on stream s.
 void launch_lbc_step(const LbcStep &a, hipStream_t s);
+
+// Several steps per launch (fds_lbc_ring.hip): a recorded point of the band, and the launch after
+// the fused engine's of the same steps.
+constexpr int kRingSeg = 62;                 // positions a side segment owns
+constexpr int kRingRecords = 64;             // recorded points of the band, at most
+
+struct LbcRec {
+  int32_t cell, comp, id;
+};
+
+struct LbcRing {
+  const float *in[3];          // state before the launch
+  float *out[3];               // what the fused engine made of it: the frame is overwritten
+  const float *b, *k;          // coefficients (isotropic)
+  const void *packed, *cells;  // weights and cells (launch_ring_pack, launch_ring_cells)
+  const LbcRec *rec;
+  double *rows[3];             // recorded values [row][m]
+  int32_t m[3];
+  const int64_t *dyn;          // dyn[1] + row: output row of the first step
+  int nrec, row, g;
+  int stages, depth;           // steps of this launch, of a full one
+  int halo, segs;              // (set at launch)
+  float cs[3];
+};
+
+// Whether a grid of side g has room for the segments of `stages` steps (two at least).
+bool lbc_ring_fits(int64_t g, int stages);
+// The cells of a layout (g, depth and rec of `a`), the weights as they are now, the steps.
+size_t lbc_ring_cells_bytes(LbcRing a);
+size_t lbc_ring_packed_bytes();
+void launch_ring_cells(LbcRing a, void *cells, hipStream_t s);
+void launch_ring_pack(const uint16_t *w1, const uint16_t *w2, void *packed, hipStream_t s);
+void launch_lbc_ring(LbcRing a, hipStream_t s);
 
 }  // namespace fds

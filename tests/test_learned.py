@@ -354,6 +354,66 @@ def test_fused_inference_writes_oracle_layer():
     fld._runner().close()
 
 
+def _ring_field(torch, g, case, tile, steps):
+    import pyfds_amd as fds
+    from pyfds_amd.learned import LearnedBoundary, CIN, HIDDEN, COUT, TAPS
+    rng = np.random.default_rng(g)
+    lb = LearnedBoundary.__new__(LearnedBoundary)
+    lb.torch, lb.lib, lb.dev = torch, nat.load(), torch.device('cuda', 0)
+    lb.cs = np.array([1.0, 1.5e6, 1.5e6], np.float32)
+    lb.w1b = _bf16_tensor(torch, rng.standard_normal((4, HIDDEN, TAPS, CIN)) * 0.05)
+    lb.w2b = _bf16_tensor(torch, rng.standard_normal((4, COUT, TAPS, HIDDEN)) * 0.05)
+    dt = 1e-8
+    fld = fds.Acoustic2D(x_samples=g, x_delta=1e-4, y_samples=g,
+                         y_delta=1.25e-4 if case == 'anisotropic' else 1e-4, t_samples=steps,
+                         t_delta=dt, material=fds.AcousticMaterial(1500.0, 1000.0))
+    fld.form = 'fp32_kahan' if case == 'kahan' else 'fp32'
+    fld.tile = tile
+    cells = [x + g * y for x in range(3, g // 2) for y in range(g // 3, g // 2)]
+    fld.add_material_region(fds.regions.Region(cells), fds.AcousticMaterial(2500.0, 1800.0))
+    n = g * g
+    for comp, scale in ((fld.pressure, 1.0), (fld.velocity_x, 1e-6), (fld.velocity_y, 1e-6)):
+        comp.values = (rng.standard_normal(n) * scale).astype(np.float32).astype(np.float64)
+    src = 20 if case == 'source' else g // 2
+    fld.pressure.add_boundary(fds.regions.Region([src + g * (g // 2)]),
+                              value=np.sin(np.arange(steps + 1)), additive=True)
+    last = g - 1
+    at = {'layer': [(5, 40)], 'many': [(x, 18) for x in range(20, g - 20)] +
+          [(20, y) for y in range(20, g - 20)]}.get(case, [])
+    at = at + [(16, 16), (23, 16), (16, last - 16), (last - 17, last - 20), (last - 16, 33),
+               (33, 20), (g // 2, 16), (24, 24), (g // 2, g // 2), (g // 2, g // 2)]
+    for comp in (fld.pressure, fld.velocity_x, fld.velocity_y):
+        comp.add_output(fds.regions.Region([x + g * y for x, y in at]))
+    lb.attach(fld)
+    return fld, lb
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('g, case, stages', [
+    (66, '', 4), (67, '', 4), (127, '', 4), (129, '', 4), (256, '', 4), (511, '', 4),
+    (512, '', 6), (573, '', 6), (65, '', 1), (130, 'source', 1), (130, 'layer', 1),
+    (130, 'many', 1), (130, 'kahan', 1), (130, 'anisotropic', 1)])
+def test_steps_per_launch_with_the_layer_equal_single_steps(g, case, stages):
+    """The learned layer with several steps per launch against the LDS-tile engine with the
+    network after every step: the same bits.  Smallest grids, segments of every length, corners,
+    remainders of a run; and the fields that keep single steps."""
+    torch = _torch()
+    plan = (13, 1, 6)
+    got = []
+    for tile in (None, 0):
+        fld, lb = _ring_field(torch, g, case, tile, sum(plan))
+        assert lb.lib.fds_steps_per_launch(fld._runner().ctx) == (1 if tile == 0 else stages)
+        for n in plan:
+            fld.simulate(n)
+        comps = (fld.pressure, fld.velocity_x, fld.velocity_y)
+        got.append([np.array(c.values) for c in comps] +
+                   [np.array(c.outputs[0].signals) for c in comps])
+        fld._runner().close()
+    assert np.isfinite(got[0][0]).all() and np.abs(got[0][0]).max() > 0
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.fixture(scope='module')
 def trained_small():
     """A network trained at reduced size (interior 256, enlarged 768) on three recorded runs."""
