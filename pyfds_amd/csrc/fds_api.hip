@@ -197,9 +197,8 @@ struct fds_ctx {
   bool coupled = false;   // stepped one step per launch by a coupling (until the next commit)
   int fused_stages = 0, fused_rows = 0;   // layout a batch asked for (0: by the grid)
   bool fused_over = false;   // the event lists do not fit the fused engine's tile classes
-  DevBuf fev_slot, fev_words, fev_cls_ptr, fev_cls, fev_points,
-      fev_point_rows, fev_tiles;     // its event tables (fds::FusedEv)
-  int fev_rows = 0, fev_nslots = 0;
+  DevBuf fev_tables;         // its event tables, one after the other (`fused_ev` points into it)
+  fds::FusedEv fused_ev{};
   DevBuf pal_idx, pal;    // material classes of the cells and their coefficients
   int npal = 0;           // classes, the zero class included (0: none known)
   bool line = false;      // resident 1D engine in use (one workgroup, many steps per launch)
@@ -456,9 +455,12 @@ bool can_ring(const fds_ctx *c, int S) {
 // 2, 15.6 at 3, 301 x 901 5.4 and 5.7), three for large ones (3000^2 FP64 53 at 2, 46 at 3).
 //
 // Height: short strips make enough waves to fill the chip, tall ones waste fewer ghost rows
-// (2S a strip, lossy 3S).  About 24 strips a CU (lossy: 16) are two rounds of resident waves, and
-// measured best or within 3 % of it (lossy 5 %) from 1024 x 1536 (4-6 rows) over 2048^2 (12) to
-// 4096 x 3000 (24-48).
+// (2S a strip, lossy 3S).  Two rounds of resident waves: two a SIMD for FP64, lossy fields and
+// AXI (its stage's chain is the longest), so 16 strips a CU, three for the FP32 forms, 24.  us a
+// step at 16 and 24: FP64 1200 x 1100 3.70 and 4.14, 2048^2 7.0 and 7.0, 3000 x 2500 16.7 and
+// 16.3, thermal 1500^2 3.47 and 3.64, AXI 1024 x 1536 3.99 and 4.79, Kahan AXI 4.13 and 4.92;
+// Kahan 2048^2 7.45 and 7.29, thermal 1500^2 3.16 and 2.94; FP32 1500 x 1203 3.23 and 3.02,
+// 2500^2 5.8 and 5.3.  Rows beyond 64 or below 4 gained nothing at any size.
 int choose_fused(fds_ctx *c) {
   const bool lossy = c->lossy && c->family == kAcoustic;
   int S = c->n < (1 << 18) ? 4 : fds::kFusedMax;
@@ -468,7 +470,7 @@ int choose_fused(fds_ctx *c) {
   c->lbc_ring = c->lbc_w1 && can_ring(c, S);
   if ((c->lbc_w1 && !c->lbc_ring) || c->flow || c->coupled) S = 1;
   const int64_t sx = 64 - 2 * S - (lossy ? 1 : 0), across = (c->nx + sx - 1) / sx;
-  const int64_t strips = (lossy ? 16 : 24) * (int64_t)c->num_cu;
+  const int64_t strips = (lossy || c->axi || c->elem == 8 ? 16 : 24) * (int64_t)c->num_cu;
   const int64_t want = (across * c->ny + strips / 2) / strips;
   const int H = c->strip_rows > 0 ? std::min(c->strip_rows, fds::kFusedStrip)
                 : c->fused_rows   ? c->fused_rows
@@ -792,15 +794,25 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
     fds::launch_ring_cells(r, c->lbc_cells.p, c->stream);
     HIP_TRY(hipGetLastError());
   }
-  c->fev_rows = rows;
-  c->fev_nslots = nslots;
-  HIP_TRY(upload(c->fev_tiles, tiles, c->stream));
-  HIP_TRY(upload(c->fev_slot, slot, c->stream));
-  HIP_TRY(upload(c->fev_words, words, c->stream));
-  HIP_TRY(upload(c->fev_cls_ptr, cls_ptr, c->stream));
-  HIP_TRY(upload(c->fev_cls, cls, c->stream));
-  HIP_TRY(upload(c->fev_points, points, c->stream));
-  HIP_TRY(upload(c->fev_point_rows, point_rows, c->stream));
+  // one buffer and one copy: each costs more than what is in it
+  std::vector<uint8_t> blob;
+  const auto put = [&](const auto &v) {
+    const size_t at = blob.size(), n = v.size() * sizeof(v[0]);
+    blob.resize((at + n + 15) / 16 * 16);
+    if (n) std::memcpy(blob.data() + at, v.data(), n);
+    return at;
+  };
+  const size_t at[7] = {put(slot), put(tiles), put(words), put(cls_ptr), put(cls), put(points),
+                        put(point_rows)};
+  HIP_TRY(upload(c->fev_tables, blob, c->stream));
+  const uint8_t *base = c->fev_tables.as<const uint8_t>();
+  c->fused_ev = fds::FusedEv{reinterpret_cast<const int32_t *>(base + at[0]),
+                        reinterpret_cast<const int32_t *>(base + at[1]),
+                        reinterpret_cast<const uint32_t *>(base + at[2]),
+                        reinterpret_cast<const int32_t *>(base + at[3]),
+                        reinterpret_cast<const fds::FusedClass *>(base + at[4]),
+                        reinterpret_cast<const fds::FusedPoint *>(base + at[5]),
+                        reinterpret_cast<const int32_t *>(base + at[6]), rows, nslots};
   return 0;
 }
 
@@ -1041,12 +1053,7 @@ void fill_args(const fds_ctx *c, fds::StepArgs<T> &a, int parity) {
   a.ghost_rows = c->ghost_rows;
   a.sx = c->sx;
   if (c->fused) {
-    a.fev = fds::FusedEv{c->fev_slot.as<const int32_t>(), c->fev_tiles.as<const int32_t>(),
-                         c->fev_words.as<const uint32_t>(),
-                         c->fev_cls_ptr.as<const int32_t>(),
-                         c->fev_cls.as<const fds::FusedClass>(),
-                         c->fev_points.as<const fds::FusedPoint>(),
-                         c->fev_point_rows.as<const int32_t>(), c->fev_rows, c->fev_nslots};
+    a.fev = c->fused_ev;
     a.pal_idx = c->pal_idx.as<const uint8_t>();
     a.pal = c->pal.as<const T>();
     a.npal = c->npal;
@@ -1233,7 +1240,7 @@ int launch_step(fds_ctx *c, int parity, int k, bool store, int stages) {
       ring_ok = ring_ok && ((uintptr_t)a.in[k] & 15) == 0 && ((uintptr_t)a.cin[k] & 15) == 0;
     for (int q = 0; q < FDS_NUM_COEFF; ++q) ring_ok = ring_ok && ((uintptr_t)a.coef[q] & 15) == 0;
   }
-  const int nb = fds::xcd_grid(c->ntiles) + (c->fused ? fds::xcd_grid(c->fev_nslots) : 0);
+  const int nb = fds::xcd_grid(c->ntiles) + (c->fused ? fds::xcd_grid(c->fused_ev.nslots) : 0);
   pick_launch(c, stages, ring_ok)(&a, nb, lds_bytes(c), c->stream);
   HIP_TRY(hipGetLastError());
   if (c->flow) {
@@ -1413,6 +1420,12 @@ __global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uin
 }
 
 template <typename T>
+__global__ __launch_bounds__(256) void k_pal_init(T *pal, int coefs, unsigned *first, int slots) {
+  for (int i = threadIdx.x; i < coefs; i += 256) pal[i] = T(0);
+  for (int i = threadIdx.x; i < 2 * slots; i += 256) first[i] = i > 0 && i < slots ? ~0u : 0u;
+}
+
+template <typename T>
 int find_classes(fds_ctx *c) {
   const bool lossy = c->lossy && c->family == kAcoustic;
   const auto slot = [&](int k, int alias) {
@@ -1422,26 +1435,23 @@ int find_classes(fds_ctx *c) {
   // (thermal: Q, G in the places of B, K)
   const PalCoefs<T> pc{{slot(2, -1), slot(0, -1), slot(3, 2), slot(1, 0), slot(4, -1), slot(5, 4),
                         slot(6, -1), slot(7, -1)}};
-  DevBuf first;
+  constexpr int kSlots = fds::kPalMax + 1, kCoefs = fds::kPalMax * fds::kPalSlots;
+  unsigned f[2 * kSlots];                     // first cells, then counts of the cells left
   HIP_TRY(c->pal_idx.ensure(c->n));
-  HIP_TRY(c->pal.ensure(fds::kPalMax * fds::kPalSlots * sizeof(T)));
-  constexpr int kSlots = fds::kPalMax + 1;
-  std::vector<unsigned> f(2 * kSlots, ~0u);   // first cells, then counts of the cells left
-  f[0] = 0;
-  std::fill(f.begin() + kSlots, f.end(), 0u);
-  HIP_TRY(upload(first, f, c->stream));
-  HIP_TRY(hipMemsetAsync(c->pal.p, 0, fds::kPalMax * fds::kPalSlots * sizeof(T), c->stream));
+  HIP_TRY(c->pal.ensure(kCoefs * sizeof(T) + sizeof f));     // (f's device side behind the table)
+  unsigned *const first = reinterpret_cast<unsigned *>(c->pal.as<T>() + kCoefs);
+  hipLaunchKernelGGL(k_pal_init<T>, dim3(1), dim3(256), 0, c->stream, c->pal.as<T>(), kCoefs, first,
+                     kSlots);
   const unsigned nb = (unsigned)std::min<int64_t>((c->n + 1023) / 1024, 2048);
   const int most = fds::kPalMax - 1;
   for (int q = 0; q < most;) {
     const int q1 = std::min(q + 4, most);
     for (; q < q1; ++q)
       hipLaunchKernelGGL((lossy ? k_pal_pass<T, 8> : k_pal_pass<T, 4>), dim3(nb), dim3(256), 0,
-                         c->stream, pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(),
-                         first.as<unsigned>(), first.as<unsigned>() + kSlots, q);
+                         c->stream, pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(), first,
+                         first + kSlots, q);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(f.data(), first.p, f.size() * sizeof(unsigned), hipMemcpyDeviceToHost,
-                           c->stream));
+    HIP_TRY(hipMemcpyAsync(f, first, sizeof f, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (f[q] == ~0u) {
       while (q > 1 && f[q - 1] == ~0u) --q;
@@ -2191,6 +2201,11 @@ int fds_prepare_run(fds_ctx *c, int64_t start, int64_t nsteps, int chunk) {
   if (nsteps < 1 || start < 0) return fail(FDS_E_ARG, "a run needs steps");
   if (int rc = prepare_run(c, start, nsteps)) return rc;
   if (int rc = capture_run_graphs(c, nsteps, chunk, true)) return rc;
+  // the fused engines' stage counts are code objects of their own, loaded on their first launch
+  // (1.3 ms): those of the launches outside the graphs
+  if (c->fused)
+    for (const int st : {step_group(c), (int)(nsteps % step_group(c))})
+      if (st > 0) pick_launch(c, st)(nullptr, 0, 0, c->stream);
   // pinned staging and events of asynchronous runs of this length (both slots)
   for (int slot = 0; slot < kMaxFlights; ++slot) {
     if (int rc = ensure_events(c->fev[slot])) return rc;
@@ -2485,7 +2500,7 @@ int batch_build(fds_batch *b, int64_t nsteps) {
   if (b->fused) {
     std::vector<int32_t> inst, slot;
     for (int i = 0; i < ni; ++i)
-      for (int s = 0; s < b->ctxs[i]->fev_nslots; ++s) {
+      for (int s = 0; s < b->ctxs[i]->fused_ev.nslots; ++s) {
         inst.push_back(i);
         slot.push_back(s);
       }

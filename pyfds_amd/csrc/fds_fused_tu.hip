@@ -43,8 +43,16 @@ __global__ __launch_bounds__(64) void k_fused(StepArgs<T> a) {
   fused_tile<T, K, THERMAL, AXI, ISO, PAL, S, kRowsAhead>(a, a.dyn[0] + a.k, a.dyn[1] + a.k, L);
 }
 
+// (no workgroups: the kernel's code is loaded onto the device, which its first launch would do)
+template <typename F>
+void load_kernel(F *kernel) {
+  hipFuncAttributes attr;
+  (void)hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(kernel));
+}
+
 template <int S, bool THERMAL, bool AXI, bool ISO, bool PAL>
 void launch_fused(const void *args, int nblocks, size_t, hipStream_t s) {
+  if (nblocks == 0) return load_kernel(k_fused<S, THERMAL, AXI, ISO, PAL>);
   hipLaunchKernelGGL((k_fused<S, THERMAL, AXI, ISO, PAL>), dim3(nblocks), dim3(64), 0, s,
                      *static_cast<const StepArgs<T> *>(args));
 }
@@ -57,6 +65,7 @@ __global__ __launch_bounds__(64) void k_fused_lossy(StepArgs<T> a) {
 
 template <int S, bool AXI, bool ISO>
 void launch_fused_lossy(const void *args, int nblocks, size_t, hipStream_t s) {
+  if (nblocks == 0) return load_kernel(k_fused_lossy<S, AXI, ISO>);
   hipLaunchKernelGGL((k_fused_lossy<S, AXI, ISO>), dim3(nblocks), dim3(64), 0, s,
                      *static_cast<const StepArgs<T> *>(args));
 }
