@@ -14,7 +14,7 @@ Prints one JSON line.  ``value`` is the FP64 drop-in form (bit-identical to the 
 float64 arithmetic); the FP32 and FP32-Kahan forms are reported under ``forms`` with their
 relative L2 error against the FP64 result.  ``roofline`` uses the algorithmic bytes per cell
 update (FP64: p, vx, vy read + write and the two coefficients K, B = 8 words = 64 B) times the
-cell updates of one launch (a launch of the streaming engine advances 1-3 fused time steps), over
+cell updates of one launch (a launch of the fused engine advances up to 6 time steps), over
 the launch time from HIP events recorded on the library's stream around the timed launches.
 With fused steps the physical HBM traffic per launch (``traffic``, measured with rocprofv3) is
 below the algorithmic bytes, so ``frac`` can pass what one pass per step could reach.
@@ -24,14 +24,14 @@ number of steps of the same workload.
 Further sections (reported under ``lossy``, ``batched`` and ``thermal2d``):
 
 * lossy: the same Acoustic2D 2048^2 scene with absorbing materials (shear viscosity 1e-3 Pa s,
-  bulk viscosity 2.4e-3 Pa s everywhere), FP64 and FP32, autotuned (lossy acoustics stream one
-  step per launch); algorithmic bytes 72 / 36 B per cell update (the viscous factor M adds one
+  bulk viscosity 2.4e-3 Pa s everywhere), FP64 and FP32, autotuned (the fused lossy engine takes
+  2-4 steps per launch, a table shape one); algorithmic bytes 72 / 36 B per cell update (the viscous factor M adds one
   word).
 
 * batched: 256 Acoustic2D / Acoustic3DAxi instances, sides uniform in 128..1024 (seed 2),
   1-4 seeded inclusions each (c 1000-6000 m/s, rho 800-8000 kg/m^3), dt at CFL 0.5 on each
   instance's own c_max, a 1 MHz burst source at each centre and 16 recorded points, FP32 and
-  FP32-Kahan, one launch per step over all instances' tiles in HIP-graph chunks of 50; each
+  FP32-Kahan, each launch over all instances' tiles, in HIP-graph chunks of 50; each
   form's pressure after the run against the same sweep in FP64 (the oracle's bits):
   relative L2 per member (largest, median) and over all cells (``rel_l2_vs_fp64``).
 * learned_bc: Acoustic2D 1024x1024 FP32 interior + 16-cell learned layer (BF16-MFMA conv net,
@@ -136,13 +136,20 @@ def tuned(fld, fixed=None):
         fld.tile, fld.strip_height, fld.graph_chunk = fixed[0], fixed[1], 50
         tile, chunk, table = fixed[0], 50, None
     else:
-        tile, chunk, table = autotune.tune_field(fld, steps=40, use_cache=False)
+        tile, chunk, table = autotune.tune_field(fld, steps=40, use_cache=False,
+                                                 default_engine=True)
         table = {k: round(v, 2) for k, v in table.items()}
-    info = nat.tile_table()[tile]
-    # steps per launch as the context runs them (lossy fields: one, whatever the shape)
+    # steps per launch as the context runs them (lossy fields on a table shape: one)
     runner = fld._runner()
     runner.sync(fld)
     spl = nat.check(runner.lib.fds_steps_per_launch(runner.ctx))
+    if tile < 0:
+        strip = getattr(fld, 'strip_height', 0) or 0
+        return dict(tile=tile, strip=strip, chunk=chunk,
+                    shape='default engine, %s, %d step(s) per launch' % (
+                        'strips of %d rows' % strip if strip else 'strips by the grid', spl),
+                    steps_per_launch=spl, table=table)
+    info = nat.tile_table()[tile]
     return dict(tile=tile, strip=getattr(fld, 'strip_height', 0) or 0, chunk=chunk,
                 shape='%s %dx%d, %d step(s) per launch%s' % (
                     info['engine'], info['tx'], getattr(fld, 'strip_height', 0) or info['ty'],
@@ -181,7 +188,8 @@ def measure_traffic(kind, form, tile, strip, launches=20):
     prof = shutil.which('rocprofv3') or '/opt/rocm/bin/rocprofv3'
     if not os.path.exists(prof):
         return None
-    family = {'acoustic2d': 'k_stream_acoustic<', 'thermal': 'k_stream_thermal<'}[kind]
+    family = 'k_fused<' if tile < 0 else {'acoustic2d': 'k_stream_acoustic<',
+                                          'thermal': 'k_stream_thermal<'}[kind]
     out = {}
     for counter in ('FETCH_SIZE', 'WRITE_SIZE'):
         d = tempfile.mkdtemp(prefix='pyfds_pmc_', dir='/tmp')
@@ -251,8 +259,8 @@ def traffic_probe(spec):
     runner.sync(fld)
     spl = nat.check(lib.fds_steps_per_launch(runner.ctx))
     fld.simulate(spl * launches)
-    info = nat.tile_table()[tile]
-    if info['lds_ring'] and info['tx'] == 64 and spl in (2, 3) and form in ('fp64', 'fp32'):
+    info = None if tile < 0 else nat.tile_table()[tile]
+    if info and info['lds_ring'] and info['tx'] == 64 and spl in (2, 3) and form in ('fp64', 'fp32'):
         # the memory-only kernel of the same access pattern, for its own byte counters
         ms, b = ct.c_double(), ct.c_double()
         nat.check(lib.fds_stream_pattern_bench(
@@ -284,6 +292,8 @@ def pattern_floor(tune, nx, ny, elem, n_state, launch_us):
     launch time over it (1 = the kernel runs at the floor its memory traffic sets)."""
     import ctypes as ct
     from pyfds_amd import _native as nat
+    if tune['tile'] < 0:
+        return None
     info = nat.tile_table()[tune['tile']]
     spl = tune['steps_per_launch']
     if not info['lds_ring'] or info['tx'] != 64 or spl not in (2, 3):
@@ -408,7 +418,7 @@ def time_batched(ns, form, steps, warmup, chunk=50, fixed=None):
     table = None
     if fixed is None:
         tile, chunk, table = autotune.tune_batch(fields, steps=20, chunks=(chunk,),
-                                                 use_cache=False)
+                                                 use_cache=False, default_engine=True)
     else:
         tile = fixed[0]
         for f in fields:

@@ -78,23 +78,26 @@ def _restore(fields, snap):
 # register-path shapes did worst at powers of two, the LDS-ring shapes best at 8 or 12 rows;
 # on 4096^2 thermal the ring shapes at 16), so the tuner times each
 STRIP_HEIGHTS = {16: (6, 12, 20, 24), 32: (8, 12, 16, 20, 24)}
+# and for the default engine of the 2D models, whose own height the grid sets
+DEFAULT_HEIGHTS = (8, 12, 16, 24, 32, 48)
 
 
-def tune_field(fld, steps=40, chunks=(50,), use_cache=True):
+def tune_field(fld, steps=40, chunks=(50,), use_cache=True, default_engine=False):
     """Choose ``fld.tile`` / ``fld.strip_height`` / ``fld.graph_chunk`` for one field; returns
     (tile, chunk, table) where table maps 'tile,strip,chunk' -> microseconds per step (strip 0:
-    the shape's own height)."""
-    return _tune([fld], steps, chunks, use_cache, batch=False)
+    the shape's own height).  ``default_engine``: the engine a field without a tile runs is a
+    candidate too (tile -1), not only the shapes of the table."""
+    return _tune([fld], steps, chunks, use_cache, False, default_engine)
 
 
-def tune_batch(fields, steps=20, chunks=(50,), use_cache=True):
+def tune_batch(fields, steps=20, chunks=(50,), use_cache=True, default_engine=False):
     """Choose one tile shape and chunk for a ``BatchRunner`` over ``fields``."""
-    return _tune(fields, steps, chunks, use_cache, batch=True)
+    return _tune(fields, steps, chunks, use_cache, True, default_engine)
 
 
-def _tune(fields, steps, chunks, use_cache, batch):
+def _tune(fields, steps, chunks, use_cache, batch, default_engine):
     lib = nat.load()
-    key = _key(fields) + ('|batch' if batch else '')
+    key = _key(fields) + ('|batch' if batch else '') + ('|default' if default_engine else '')
     cache = _load_cache() if use_cache else {}
     if key in cache:
         tile, chunk = cache[key]['tile'], cache[key]['chunk']
@@ -109,6 +112,8 @@ def _tune(fields, steps, chunks, use_cache, batch):
     one_row = fields[0]._device_grid()[1] == 1
     lossy = any(getattr(x, '_coefs', {}).get(4) is not None for x in fields)
     cand = []
+    if default_engine:
+        cand = [(-1, h) for h in (0,) + (() if one_row else DEFAULT_HEIGHTS)]
     for i, (tx, ty) in enumerate(shapes):
         if (ty == 1) != one_row:
             continue
