@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kRingThreads) void k_ring_cells(LbcRing A, RingCell
 }
 
 // What bounds it: the issue rate and latency of one CU.  A step is four phases with a barrier
-// after each (velocities; pressure and the network's input; hidden layer; layer), and of the 76
+// after each (velocities; pressure and the network's input; hidden layer; layer), and of the 68
 // segments of a 1056^2 grid the corners take longest.  12 waves share a phase, each keeping its
 // weights in registers; a step's row tiles are those that still reach an owned cell.
 __global__ __launch_bounds__(kRingThreads) void k_lbc_ring(LbcRing A) {
