@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_gather(const float *__restrict__ frames
 // ---------------------------------------------------------------- fused training iteration
 // Three launches per iteration.  One kernel per operation, enqueued one by one with six sample
 // lists copied in between, was bound by the host and by those copies: 20 iterations of 32 samples
-// on 1056 positions 6.9 ms, so 1.6 ms.
+// on 1056 positions 6.9 ms, 1.0 ms so.
 //   k_train_grads    gather, both convolutions, loss and the gradient at the hidden layer of a
 //                    segment of a sample, in LDS;
 //   k_train_weights  the weight gradients of one sample, one 16 x 16 tile for all taps a wave;
@@ -262,7 +262,8 @@ __global__ __launch_bounds__(64) void k_train_pads(uint16_t *rows, int G, int pi
 // Bound by latency: a chain of loads, three products and three barriers; 64 positions a
 // workgroup give 544 of them for 32 samples of 1056 positions (two a CU), and the 12 rows
 // computed twice on the way cost a fifth.  The weights stay in registers: a wave keeps one
-// column of 16 output channels for all its rows.
+// column of 16 output channels for all its rows.  24.7 us at that size (26.9 with the input
+// cells dealt out by element, whose index arithmetic every lane did).
 __global__ __launch_bounds__(256) void k_train_grads(TrainStep A) {
   constexpr int R = kLbcTaps / 2;
   constexpr int NT = 5;                            // row tiles of the hidden layer and of dy
@@ -283,18 +284,22 @@ __global__ __launch_bounds__(256) void k_train_grads(TrainStep A) {
   constexpr int N1 = kLbcTaps * (kLbcCin / 16), N2 = kLbcTaps * (kLbcHidden / 16),
                 NB = kLbcTaps * (kLbcCout / 16);
 
-  // inputs, targets and the weights of both layers, all in flight together
-  constexpr int NI = kLbcCin * NXR, II = (NI + 255) / 256;
-  float rx[II];
+  // inputs, targets and the weights of both layers, all in flight together.  A wave takes 12
+  // input channels: of each the first 64 rows, then the other 20 rows of three at a time.
+  constexpr int WC = kLbcCin / 4, NL = NXR - 64, NP = 64 / NL;
+  static_assert(NL > 0 && WC % NP == 0, "the rows past a wave's lanes go by whole groups");
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const auto source = [&](int ci) {
+    const int h = ci / 24, c = (ci % 24) / kLbcBand, j = ci % kLbcBand;
+    return A.frames + ((((f0 - h) * 3 + c) * 4 + s) * A.D + L + j) * G;
+  };
+  const int al = a0 - 3 * R + l, row2 = 64 + l % NL, ah = a0 - 3 * R + row2, q2 = l / NL;
+  const bool in1 = al >= L && al < G - L, in2 = q2 < NP && ah >= L && ah < G - L;
+  float r1[WC], r2[WC / NP];
 #pragma unroll
-  for (int i = 0; i < II; ++i) {
-    const int e = tid + 256 * i, row = e % NXR, ci = e / NXR, a = a0 - 3 * R + row;
-    rx[i] = 0.f;
-    if (e < NI && a >= L && a < G - L) {
-      const int h = ci / 24, c = (ci % 24) / kLbcBand, j = ci % kLbcBand;
-      rx[i] = A.frames[((((f0 - h) * 3 + c) * 4 + s) * A.D + L + j) * G + a];
-    }
-  }
+  for (int i = 0; i < WC; ++i) r1[i] = in1 ? source(wv * WC + i)[al] : 0.f;
+#pragma unroll
+  for (int i = 0; i < WC / NP; ++i) r2[i] = in2 ? source(wv * WC + NP * i + q2)[ah] : 0.f;
   // layer 2: waves 0-2 take a column of channels each (a component), rows of tiles 0-3; wave 3
   // the last tile of all three
   float tg[4][4];
@@ -303,11 +308,14 @@ __global__ __launch_bounds__(256) void k_train_grads(TrainStep A) {
     const int nt = wave < 3 ? wave : i, mt = wave < 3 ? i : NT - 1;
     const int a = a0 - 2 * R + 16 * mt + 4 * g;
     const bool job = wave < 3 || i < 3;
+    const float *t = A.frames + (((f0 * 3 + nt) * 4 + s) * A.D + m) * G + a;
+    if (job && a >= 0 && a + 3 < G) {
+      typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
+      const f4a v = *reinterpret_cast<const f4a *>(t);
+      tg[i][0] = v[0], tg[i][1] = v[1], tg[i][2] = v[2], tg[i][3] = v[3];
+    } else {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      tg[i][v] = 0.f;
-      if (job && a + v >= 0 && a + v < G)
-        tg[i][v] = A.frames[(((f0 * 3 + nt) * 4 + s) * A.D + m) * G + a + v];
+      for (int v = 0; v < 4; ++v) tg[i][v] = job && a + v >= 0 && a + v < G ? t[v] : 0.f;
     }
   }
   s4 b1[N1], b2[N2];
@@ -323,15 +331,18 @@ __global__ __launch_bounds__(256) void k_train_grads(TrainStep A) {
     b1[i] = ld4(g1 + ((16 * (wave & 1) + m) * kLbcTaps + i / 3) * kLbcCin + 16 * (i % 3) + 4 * g);
   load2(wave < 3 ? wave : 0);
 
-#pragma unroll
-  for (int i = 0; i < II; ++i) {
-    const int e = tid + 256 * i, row = e % NXR, ci = e / NXR, a = a0 - 3 * R + row;
-    if (e >= NI) continue;
+  const auto input = [&](int ci, int row, int a, float v) {
     const int c = (ci % 24) / kLbcBand;
-    const uint16_t v = f2bf(rx[i] * (c == 0 ? A.cs[0] : c == 1 ? A.cs[1] : A.cs[2]) * sc);
-    xin[row * SX + ci] = v;
+    const uint16_t u = f2bf(v * (c == 0 ? A.cs[0] : c == 1 ? A.cs[1] : A.cs[2]) * sc);
+    xin[row * SX + ci] = u;
     if (a >= a0 && a < a0 + kTrainSeg && a < G)
-      A.x[((size_t)b * kLbcCin + ci) * A.pitch + kPad + a] = v;
+      A.x[((size_t)b * kLbcCin + ci) * A.pitch + kPad + a] = u;
+  };
+#pragma unroll
+  for (int i = 0; i < WC; ++i) input(wv * WC + i, l, al, r1[i]);
+  if (q2 < NP) {
+#pragma unroll
+    for (int i = 0; i < WC / NP; ++i) input(wv * WC + NP * i + q2, row2, ah, r2[i]);
   }
   for (int e = tid; e < R * SH; e += 256) {
     hid[e] = 0;

@@ -12,8 +12,9 @@ step instead:
   biases, so the map is linear and scale-equivariant like the wave equation it stands in for;
 * velocities enter in pressure units (times rho0 c0) so all channels have one scale;
 * weights are bf16, products accumulate in fp32 on the matrix cores
-  (``pyfds_amd/csrc/fds_lbc.hip``); inference runs as one fused kernel per step inside the
-  device step loop (``fds_set_learned_boundary``), captured in the same HIP graphs.
+  (``pyfds_amd/csrc/fds_lbc.hip``); inference runs inside the device step loop
+  (``fds_set_learned_boundary``), as one fused kernel per step or, where the field allows it, one
+  per up to six steps (``fds_lbc_ring.hip``), captured in the same HIP graphs.
 
 Training data come from the plain method on the enlarged grid (default 3072^2, the interior
 centred): the layer and band rows are recorded every step while waves from random sources and
