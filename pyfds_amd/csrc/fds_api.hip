@@ -444,15 +444,15 @@ bool can_ring(const fds_ctx *c, int S) {
 
 // Layout of the fused engine: stages per launch and strip height.
 //
-// Stages: a launch's time grows slowly with them (2048^2 FP64 acoustics: 36 us at 4, 42 us at 6),
+// Stages: a launch's time grows slowly with them (2048^2 FP64 acoustics: 38 us at 4, 42 us at 6),
 // so all kFusedMax, except on small grids, where a launch is bound by the latency of one strip
-// and the iterations it takes: 401 x 301 FP64 2.5 us a step at 4 stages, 2.6 at 6; from 800 x 600
+// and the iterations it takes: 401 x 301 FP64 2.3 us a step at 4 stages, 2.4 at 6; from 800 x 600
 // on 6 are ahead (FP64 3.0 and 2.9).  One where something follows every step.
 //
 // Lossy acoustics: a stage holds 15 values a column, so three stages (2000 x 1500 FP64 11 us a
 // step at 3, 14 at 2; 3000^2 38 at 3 and 4), four for large fields of the FP32 forms (3000^2 FP32
 // 13.4 at 4, 15.0 at 3), and with the radius' coefficients on top two (2000 x 1500 FP64 15.8 at
-// 2, 15.6 at 3, 301 x 901 5.4 and 5.7), three for large ones (3000^2 FP64 53 at 2, 46 at 3).
+// 2, 15.6 at 3, 301 x 901 5.3 and 5.4), three for large ones (3000^2 FP64 53 at 2, 46 at 3).
 //
 // Height: short strips make enough waves to fill the chip, tall ones waste fewer ghost rows
 // (2S a strip, lossy 3S).  Two rounds of resident waves: two a SIMD for FP64, lossy fields and
