@@ -2400,7 +2400,6 @@ int batch_layout(fds_batch *b, bool try_fused) {
   std::vector<int32_t> tinst, base;
   size_t lds = 0;
   b->member_tiles.clear();
-  b->fused_any = false;
   const int n = (int)b->ctxs.size();
   for (int i = 0; i < n; ++i) {
     fds_ctx *c = b->ctxs[i];
@@ -2411,7 +2410,6 @@ int batch_layout(fds_batch *b, bool try_fused) {
       touch(c);
       lds = std::max(lds, lds_bytes(c));
     }
-    b->fused_any = b->fused_any || c->family != kAcoustic || !(c->axi || (c->iso_b && c->iso_k));
     base.push_back((int32_t)tinst.size());
     b->member_tiles.push_back(c->ntiles);
     for (int k = 0; k < c->ntiles; ++k) tinst.push_back(i);
@@ -2498,12 +2496,17 @@ int batch_build(fds_batch *b, int64_t nsteps) {
       HIP_TRY(upload(b->descs[parity][store], d, b->stream));
     }
   if (b->fused) {
+    // (a member's new coefficients may be of another kind than those the batch was laid out for)
+    b->fused_any = false;
     std::vector<int32_t> inst, slot;
-    for (int i = 0; i < ni; ++i)
-      for (int s = 0; s < b->ctxs[i]->fused_ev.nslots; ++s) {
+    for (int i = 0; i < ni; ++i) {
+      const fds_ctx *c = b->ctxs[i];
+      b->fused_any = b->fused_any || c->family != kAcoustic || !(c->axi || (c->iso_b && c->iso_k));
+      for (int s = 0; s < c->fused_ev.nslots; ++s) {
         inst.push_back(i);
         slot.push_back(s);
       }
+    }
     b->nev = (int)inst.size();
     HIP_TRY(upload(b->ev_inst, inst, b->stream));
     HIP_TRY(upload(b->ev_slot, slot, b->stream));

@@ -281,3 +281,36 @@ def test_fp32_sweep_batch_within_tolerance_of_oracle(form, sweep_reference):
                                        '  '.join('%s %.3e' % kv for kv in errs.items())))
         worst = max([worst] + list(errs.values()))
     assert worst <= FP32_SWEEP_TOL, worst
+
+
+def test_fp64_batch_follows_a_member_made_anisotropic():
+    """A small batch of isotropic plane fields (the members' own layout is the batch's, so nothing
+    is laid out again): one member's y step changes and it is assembled anew between runs."""
+    members = []
+    for i, (nx, ny) in enumerate([(120, 61), (57, 80), (64, 64)]):
+        scene = dict(scenes.scene_a2d_main(), plan=[('simulate', 13), ('simulate', 10)])
+        n = nx * ny
+        rng = np.random.default_rng(i)
+        scene['kwargs'] = dict(scene['kwargs'], x_samples=nx, y_samples=ny)
+        scene['regions'] = [(np.flatnonzero(rng.random(n) < 0.3), scene['regions'][0][1])]
+        scene['init'] = {'pressure': rng.standard_normal(n)}
+        scene['boundaries'] = {}
+        scene['outputs'] = {'pressure': [[0, n // 2, n - 1]]}
+        members.append((scene, scenes.build_field(pyfds_amd, pyfds_amd.regions, scene)))
+    fields = [f for _, f in members]
+    batch = BatchRunner(fields)
+    batch.simulate(13)
+    fields[1].y.increment *= 1.25
+    fields[1].assemble_matrices()
+    batch.simulate(10)
+    assert batch.lib.fds_batch_steps_per_launch(batch.handle) == 4
+    for i, (scene, fld) in enumerate(members):
+        ref = scenes.build_oracle(scene)
+        ref.simulate(13)
+        if i == 1:
+            ref.dy *= 1.25
+            ref.assemble()
+        ref.simulate(10)
+        np.testing.assert_array_equal(fld.pressure.values, ref.components['pressure'])
+        np.testing.assert_array_equal(np.array(fld.pressure.outputs[0].signals),
+                                      np.array(ref.signals('pressure')[0]))
