@@ -714,7 +714,8 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
   std::vector<fds::FusedClass> cls;
   std::vector<fds::FusedPoint> points;
   std::vector<int32_t> point_rows;
-  // distinct programs of each component, by their entries
+  // distinct programs of each component, by their entries (-1: one without entries, which does
+  // nothing and has no class)
   std::vector<int32_t> prog[3];
   std::vector<std::pair<int32_t, int32_t>> first[3];   // entries of a distinct program
   for (int k = 0; k < 3; ++k) {
@@ -722,6 +723,10 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
     std::map<std::vector<int64_t>, int32_t> seen;
     std::vector<int64_t> key;
     for (size_t u = 0; u < cp.cells.size(); ++u) {
+      if (cp.ptr[u] == cp.ptr[u + 1]) {
+        prog[k].push_back(-1);
+        continue;
+      }
       key.clear();
       for (int32_t e = cp.ptr[u]; e < cp.ptr[u + 1]; ++e) {
         int64_t bits;
@@ -752,6 +757,7 @@ int build_fused_events(fds_ctx *c, const Events *bev, const Events *oev) {
         const int r = bev[k].pos[e] / R.w + R.rmin + g, col = bev[k].pos[e] % R.w + R.cmin;
         if (r < 0 || r >= rows || col < 0 || col >= 64) continue;
         const int32_t p = prog[k][bev[k].id[e]];
+        if (p < 0) continue;
         const auto it = local.emplace(std::make_pair(k, p), (int32_t)(cls.size() - base + 1));
         if (it.second) {
           const auto [e0, e1] = first[k][p];

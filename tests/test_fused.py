@@ -205,3 +205,42 @@ def test_fp64_batch_matches_oracle_bitwise(models):
                 np.testing.assert_array_equal(got['signals/%s/%d' % (comp, k)],
                                               np.array(out['signals'], dtype=float),
                                               err_msg='%d %s' % (i, comp))
+
+
+@pytest.mark.parametrize('mu', [0.0, 0.3])
+def test_boundary_cells_without_entries_do_nothing(mu):
+    """``fds_set_boundaries`` takes cells with no entry, first, between others and last of a tile,
+    of every component: the tile engine's bits."""
+    nat = pyfds_amd._native
+    nx, ny, steps = 90, 40, 11
+    signal = np.random.default_rng(5).standard_normal(steps)
+    table = np.concatenate([[0.5, -0.25], signal])
+    inf = np.iinfo(np.int64).max
+    entry = {'set': (0.0, 0, 0, inf), 'add': (1.0, 1, 0, inf), 'signal': (1.0, 2, 1, steps)}
+    programs = [  # component 0, 1, 2: (cell, entries)
+        [(3, []), (40, ['set']), (41, []), (nx + 7, ['signal', 'add']), (9 * nx + 2, []),
+         (30 * nx + 60, ['add']), (39 * nx + 89, [])],
+        [(5, ['add']), (nx + 6, []), (20 * nx + 61, [])],
+        [(0, []), (17 * nx, []), (39 * nx + 88, [])]]
+    res = []
+    for tile in (1, -1):
+        print('empty programs', mu, tile, flush=True)
+        fld = scenes.build_field(pyfds_amd, pyfds_amd.regions, _scene('Acoustic2D', nx, ny, mu=mu))
+        fld.tile = tile
+        fld.assemble_matrices()
+        run = fld._runner()
+        run.sync(fld)
+        for k, prog in enumerate(programs):
+            ents = [entry[e] for _, es in prog for e in es]
+            cells = nat.i64([c for c, _ in prog])
+            ptr = np.concatenate([[0], np.cumsum([len(es) for _, es in prog])]).astype(np.int32)
+            a = nat.f64([e[0] for e in ents])
+            off, stride, length = (nat.i64([e[i] for e in ents]) for i in (1, 2, 3))
+            nat.check(run.lib.fds_set_boundaries(
+                run.ctx, k, cells.size, nat.lptr(cells), nat.iptr(ptr), len(ents), nat.dptr(a),
+                nat.lptr(off), nat.lptr(stride), nat.lptr(length), table.size, nat.dptr(table)))
+        nat.check(run.lib.fds_run(run.ctx, 0, steps, 0))
+        res.append([run.download(k) for k in range(3)])
+        run.close()
+    for a, b in zip(*res):
+        np.testing.assert_array_equal(a, b)
