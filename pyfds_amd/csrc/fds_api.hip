@@ -249,6 +249,17 @@ struct fds_ctx {
   HostBuf nf_stage;
 };
 
+// What a batch's kernels and tables assume of a member.
+struct MemberLayout {
+  int shape, fuse, ghost, ghost_rows, tx, ty, ntiles;
+  bool fused, line, lossy;
+  bool operator==(const MemberLayout &o) const {
+    return shape == o.shape && fuse == o.fuse && ghost == o.ghost && ghost_rows == o.ghost_rows &&
+           tx == o.tx && ty == o.ty && ntiles == o.ntiles && fused == o.fused && line == o.line &&
+           lossy == o.lossy;
+  }
+};
+
 struct fds_batch {
   std::vector<fds_ctx *> ctxs;
   int device = 0, form = 0, tile = -1;
@@ -262,7 +273,7 @@ struct fds_batch {
   int nev = 0;
   int fuse = 1;
   int tx = 0, ty = 0, ntiles = 0;
-  std::vector<int> member_tiles;           // the members' tile counts the tables hold
+  std::vector<MemberLayout> layouts;       // the members as its tables and kernels take them
   size_t lds = 0;
   DevBuf descs[2][2];          // [parity][store]
   DevBuf tile_inst, inst_base, dyn;
@@ -2362,9 +2373,20 @@ void batch_drop_graphs(fds_batch *b) {
   b->graph_objs.clear();
 }
 
+MemberLayout layout_of(const fds_ctx *c) {
+  return MemberLayout{c->shape, c->fuse,   c->ghost, c->ghost_rows, c->tx,
+                      c->ty,    c->ntiles, c->fused, c->line,       c->lossy};
+}
+
 // Lay a batch out: every member on the fused engine (try_fused, where it covers them all) or on
 // one shape of the tile table, and the tables that map the launch's tiles to members.
 int batch_layout(fds_batch *b, bool try_fused) {
+  // (runs in flight elsewhere read the members' tables)
+  for (auto *c : b->ctxs)
+    if (!c->flights.empty() || c->batch_flights) {
+      HIP_TRY(hipDeviceSynchronize());
+      break;
+    }
   b->fused = false;
   if (try_fused && b->tile < 0 && b->schedule == 0) {
     int64_t cells = 0, across = 0;
@@ -2405,7 +2427,7 @@ int batch_layout(fds_batch *b, bool try_fused) {
                 fds::kStreamShapes[t - fds::kNumTiles][4]);
   std::vector<int32_t> tinst, base;
   size_t lds = 0;
-  b->member_tiles.clear();
+  b->layouts.clear();
   const int n = (int)b->ctxs.size();
   for (int i = 0; i < n; ++i) {
     fds_ctx *c = b->ctxs[i];
@@ -2417,7 +2439,7 @@ int batch_layout(fds_batch *b, bool try_fused) {
       lds = std::max(lds, lds_bytes(c));
     }
     base.push_back((int32_t)tinst.size());
-    b->member_tiles.push_back(c->ntiles);
+    b->layouts.push_back(layout_of(c));
     for (int k = 0; k < c->ntiles; ++k) tinst.push_back(i);
   }
   if (lds > 65536)
@@ -2452,12 +2474,12 @@ int batch_layout(fds_batch *b, bool try_fused) {
   return 0;
 }
 
-// Whether the members are still as the batch was laid out.
+// Whether the members are still as the batch was laid out (a member may have been given another
+// tile, strip height, or coefficients of another kind since).
 bool batch_laid_out(const fds_batch *b) {
   for (size_t i = 0; i < b->ctxs.size(); ++i) {
     const fds_ctx *c = b->ctxs[i];
-    if (c->ntiles != b->member_tiles[i] ||
-        (b->fused && !(c->fused && c->fuse == b->fuse && c->npal > 0 && !c->lossy)))
+    if (!(layout_of(c) == b->layouts[i]) || lds_bytes(c) > b->lds || (b->fused && !c->npal))
       return false;
   }
   return true;

@@ -314,3 +314,52 @@ def test_fp64_batch_follows_a_member_made_anisotropic():
         np.testing.assert_array_equal(fld.pressure.values, ref.components['pressure'])
         np.testing.assert_array_equal(np.array(fld.pressure.outputs[0].signals),
                                       np.array(ref.signals('pressure')[0]))
+
+
+@pytest.mark.parametrize('tile, change', [(None, 1), (-2, -1), (-2, -3), (0, -1), (0, 4),
+                                          (0, 'anisotropic'), (-2, 'lossy')])
+def test_fp64_batch_lays_out_again_after_a_member_changed(tile, change):
+    """A member is given another tile (of as many workgroups: 50 x 4 cells are one on any), or
+    coefficients of another kind, between two runs of a batch: the batch goes back to a layout that
+    holds for all.  ``tile`` and ``change`` -2, -3: two streaming shapes."""
+    stream = {-2: _stream_index(9), -3: _stream_index(14)}
+    members = []
+    for i, (nx, ny) in enumerate([(50, 4), (64, 9)]):
+        scene = dict(scenes.scene_a2d_main(), plan=[])
+        n = nx * ny
+        scene['kwargs'] = dict(scene['kwargs'], x_samples=nx, y_samples=ny)
+        scene['regions'] = [(np.arange(0, n, 3), scene['regions'][0][1])]
+        scene['init'] = {'pressure': np.random.default_rng(i).standard_normal(n)}
+        scene['boundaries'] = {'pressure': [dict(indices=[7, n - 1], value=0.5, additive=True)]}
+        scene['outputs'] = {'pressure': [[0, n // 2, n - 1]]}
+        members.append((scene, scenes.build_field(pyfds_amd, pyfds_amd.regions, scene)))
+    fields = [f for _, f in members]
+    batch = BatchRunner(fields, tile=stream.get(tile, tile), chunk=0)
+    batch.simulate(7)
+    fld, mu = fields[0], 0.3
+    if change == 'anisotropic':
+        fld.y.increment *= 1.25
+    elif change == 'lossy':
+        for r in fld.material_regions:
+            for m in r.materials:
+                m.absorption_coef = mu
+    else:
+        nat = pyfds_amd._native
+        nat.check(batch.lib.fds_set_tile(fld._runner().ctx, stream.get(change, change)))
+    if isinstance(change, str):
+        fld.assemble_matrices()
+    print('batch', tile, change, flush=True)
+    batch.simulate(5)
+    for i, (scene, f) in enumerate(members):
+        ref = scenes.build_oracle(scene)
+        ref.simulate(7)
+        if i == 0 and change == 'anisotropic':
+            ref.dy *= 1.25
+        if i == 0 and change == 'lossy':
+            for _, m in ref.materials:
+                m['absorption_coef'] = mu
+        ref.assemble()
+        ref.simulate(5)
+        np.testing.assert_array_equal(f.pressure.values, ref.components['pressure'])
+        np.testing.assert_array_equal(np.array(f.pressure.outputs[0].signals),
+                                      np.array(ref.signals('pressure')[0]))
