@@ -196,7 +196,8 @@ struct fds_ctx {
   bool fused = false;     // fused engine in use (a row-streaming engine: streaming is set too)
   bool coupled = false;   // stepped one step per launch by a coupling (until the next commit)
   int fused_stages = 0, fused_rows = 0;   // layout a batch asked for (0: by the grid)
-  bool fused_over = false;   // the event lists do not fit the fused engine's tile classes
+  // the layout (stages, strip height) whose tiles cannot hold the event lists (0: none known)
+  int over_stages = 0, over_rows = 0;
   DevBuf fev_tables;         // its event tables, one after the other (`fused_ev` points into it)
   fds::FusedEv fused_ev{};
   DevBuf pal_idx, pal;    // material classes of the cells and their coefficients
@@ -411,7 +412,7 @@ bool fuse_reach(const fds_ctx *c) {
 }
 
 bool can_fuse(const fds_ctx *c) {
-  return fuse_reach(c) && !c->fused_over && (!(c->lossy && c->family == kAcoustic) || c->npal > 0);
+  return fuse_reach(c) && (!(c->lossy && c->family == kAcoustic) || c->npal > 0);
 }
 
 // Resident 1D engine variant for n cells: `cpt` cells per thread if given, else the fewest
@@ -472,6 +473,8 @@ bool can_ring(const fds_ctx *c, int S) {
 // 16.3, thermal 1500^2 3.47 and 3.64, AXI 1024 x 1536 3.99 and 4.79, Kahan AXI 4.13 and 4.92;
 // Kahan 2048^2 7.45 and 7.29, thermal 1500^2 3.16 and 2.94; FP32 1500 x 1203 3.23 and 3.02,
 // 2500^2 5.8 and 5.3.  Rows beyond 64 or below 4 gained nothing at any size.
+//
+// 1: no such layout, the tiles of this one cannot hold the event lists.
 int choose_fused(fds_ctx *c) {
   const bool lossy = c->lossy && c->family == kAcoustic;
   int S = c->n < (1 << 18) ? 4 : fds::kFusedMax;
@@ -486,6 +489,10 @@ int choose_fused(fds_ctx *c) {
   const int H = c->strip_rows > 0 ? std::min(c->strip_rows, fds::kFusedStrip)
                 : c->fused_rows   ? c->fused_rows
                                   : (int)std::min<int64_t>(std::max<int64_t>(want, 4), 64);
+  if (S == c->over_stages && H == c->over_rows) {
+    c->lbc_ring = false;
+    return 1;
+  }
   c->fused = c->streaming = true;
   c->fuse = S;
   c->ghost = S;
@@ -568,7 +575,8 @@ int choose_tiles(fds_ctx *c) {
     c->ty = 1;
     c->shape = 0;
   } else {
-    if (c->tile < 0 && can_fuse(c)) return choose_fused(c);
+    if (c->tile < 0 && can_fuse(c))
+      if (const int rc = choose_fused(c); rc <= 0) return rc;
     int t = c->tile;
     if (t < 0) t = (c->ny == 1) ? fds::kTileRow : (c->lossy ? fds::kDefaultLossy2D
                                                              : fds::kDefaultLossless2D);
@@ -848,7 +856,8 @@ int rebuild_events(fds_ctx *c) {
       touch(c);
       return 0;
     }
-    c->fused_over = true;    // until the boundaries change
+    c->over_stages = c->fuse;    // until the boundaries change
+    c->over_rows = c->ty;
     if (int rc2 = choose_tiles(c)) return rc2;
   }
   if (!c->line) {
@@ -1784,8 +1793,8 @@ int fds_set_boundaries(fds_ctx *c, int comp, int64_t ncell, const int64_t *cells
   HIP_TRY(upload(cp.d_off, cp.off, c->stream));
   HIP_TRY(upload(cp.d_stride, cp.stride, c->stream));
   HIP_TRY(upload(cp.d_table, cp.table, c->stream));
-  if (c->fused_over || c->lbc_w1) {
-    c->fused_over = false;
+  if (c->over_stages || c->lbc_w1) {
+    c->over_stages = c->over_rows = 0;
     if (int rc = choose_tiles(c)) return rc;
   }
   c->events_dirty = true;
@@ -2393,7 +2402,7 @@ int batch_layout(fds_batch *b, bool try_fused) {
     bool ok = true;
     for (auto *c : b->ctxs) {
       c->tile = -1;
-      if (!(can_stream_batch(c) && fuse_reach(c)) || c->fused_over || c->coupled) ok = false;
+      if (!(can_stream_batch(c) && fuse_reach(c)) || c->coupled) ok = false;
       if (ok && !c->npal)
         if (int rc = ready_classes(c)) return rc;
       ok = ok && c->npal > 0;

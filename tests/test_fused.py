@@ -244,3 +244,51 @@ def test_boundary_cells_without_entries_do_nothing(mu):
         run.close()
     for a, b in zip(*res):
         np.testing.assert_array_equal(a, b)
+
+
+def _signals_scene(nx, ny, cells, seed=0):
+    """A signal of its own on each of ``cells``, on top of the plain scene."""
+    sc = _scene('Acoustic2D', nx, ny, seed=seed)
+    rng = np.random.default_rng(seed)
+    sc['boundaries']['pressure'] = [dict(indices=list(cells), additive=True,
+                                         value=[rng.standard_normal(STEPS) for _ in cells])]
+    return sc
+
+
+@pytest.mark.parametrize('count', [63, 64])
+def test_as_many_boundary_classes_as_a_tile_holds(count):
+    scene = _signals_scene(50, 8, range(3, 3 + 5 * count, 5))
+    print('classes', count, flush=True)
+    ref = scenes.run_oracle(scene)
+    got, group = _run(scene, strip_height=8)
+    assert group == (4 if count == 63 else 2)
+    for k in ref:
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+def test_strips_too_tall_for_the_classes_leave_other_heights_alone():
+    """Two signals a row: strips of 48 rows see more classes than a tile holds, strips of 8 and the
+    height of the grid's own choice do not, whatever was tried before."""
+    nx, ny = 130, 60
+    scene = _signals_scene(nx, ny, [r * nx + c for r in range(ny) for c in (20, 21)])
+    fld = scenes.build_field(pyfds_amd, pyfds_amd.regions, scene)
+    fld.assemble_matrices()
+    run = fld._runner()
+    run.sync(fld)
+    lib = run.lib
+
+    def go(n, strip=None, tile=None):
+        if tile is not None:
+            pyfds_amd._native.check(lib.fds_set_tile(run.ctx, tile))
+        if strip is not None:
+            pyfds_amd._native.check(lib.fds_set_strip_height(run.ctx, strip))
+        fld.simulate(n)
+        return lib.fds_steps_per_launch(run.ctx)
+
+    groups = [go(3, 48), go(3, 8), go(3, 48), go(2, 0), go(1, 48), go(2, 0, 1), go(2, 0, -1)]
+    fld.assemble_matrices()
+    groups += [go(2, 48), go(2, 8)]
+    assert groups == [2, 4, 2, 4, 2, 1, 4, 2, 4]
+    ref = scenes.build_oracle(scene)
+    ref.simulate(20)
+    np.testing.assert_array_equal(fld.pressure.values, ref.components['pressure'])
