@@ -752,6 +752,9 @@ def learned_section(no_cpu, runs=3, iters=1500):
                window_steps=list(res['window']), finite=res['finite'],
                learned_s=round(res['learned_s'], 4), enlarged_s=round(res['enlarged_s'], 4),
                speedup_vs_enlarged=round(res['speedup'], 3), timed_steps=steps,
+               default_engines=dict(learned_s=round(res['default_learned_s'], 4),
+                                    enlarged_s=round(res['default_enlarged_s'], 4),
+                                    speedup_vs_enlarged=round(res['default_speedup'], 3)),
                learned_gcells=round(lb.G ** 2 * steps / res['learned_s'] / 1e9, 3),
                enlarged_gcells=round(lb.big ** 2 * steps / res['enlarged_s'] / 1e9, 3),
                params=int(lb.n_params), net_gflop_per_step=round(2 * macs / 1e9, 4),

@@ -1,9 +1,10 @@
 """Autotuner: picks the step kernels' shape, strip height and HIP-graph chunk by timing.
 
-For a field (or a batch of fields) it times a few steps of every admissible shape of the
+For a field (or a batch of fields) it times a few steps of the engine a field runs by itself
+(tile -1, 2D models also at a few strip heights), of every admissible shape of the
 compiled shape table (``fds_tile_count``/``fds_tile_shape``/``fds_tile_engine``; streaming
-shapes also at a few strip heights, ``fds_set_strip_height``) and graph-chunk length with the
-GPU's own clock (HIP events around the launches, ``fds_last_run_ms`` /
+shapes also at a few strip heights, ``fds_set_strip_height``) and of each graph-chunk length
+with the GPU's own clock (HIP events around the launches, ``fds_last_run_ms`` /
 ``fds_batch_last_run_ms``), keeps the fastest and caches the choice in a JSON file keyed by
 device, model, form, grid and lossy/Axi variant.  Timing runs advance a scratch copy of the
 state: the caller's field is restored to its values before tuning.
@@ -50,7 +51,7 @@ def _key(fields):
     lossy = any(getattr(x, '_coefs', {}).get(4) is not None for x in fields)
     cells = sum(x.num_points for x in fields)
     return '|'.join(str(v) for v in (_device_name(), type(f).__name__, f.form, len(fields),
-                                     cells, f._device_grid(), lossy, 'v4'))
+                                     cells, f._device_grid(), lossy, 'v5'))
 
 
 def _snapshot(fields):
@@ -82,22 +83,23 @@ STRIP_HEIGHTS = {16: (6, 12, 20, 24), 32: (8, 12, 16, 20, 24)}
 DEFAULT_HEIGHTS = (8, 12, 16, 24, 32, 48)
 
 
-def tune_field(fld, steps=40, chunks=(50,), use_cache=True, default_engine=False):
+def tune_field(fld, steps=40, chunks=(50,), use_cache=True, default_engine=True):
     """Choose ``fld.tile`` / ``fld.strip_height`` / ``fld.graph_chunk`` for one field; returns
     (tile, chunk, table) where table maps 'tile,strip,chunk' -> microseconds per step (strip 0:
-    the shape's own height).  ``default_engine``: the engine a field without a tile runs is a
-    candidate too (tile -1), not only the shapes of the table."""
+    the shape's own height).  ``default_engine=False`` leaves the engine that a field without a
+    tile runs (tile -1) out: the best shape of the table, which is slower on every 2D model
+    (Acoustic2D 2048^2 FP64: 24.5 us a step on it, 7.0 on tile -1)."""
     return _tune([fld], steps, chunks, use_cache, False, default_engine)
 
 
-def tune_batch(fields, steps=20, chunks=(50,), use_cache=True, default_engine=False):
+def tune_batch(fields, steps=20, chunks=(50,), use_cache=True, default_engine=True):
     """Choose one tile shape and chunk for a ``BatchRunner`` over ``fields``."""
     return _tune(fields, steps, chunks, use_cache, True, default_engine)
 
 
 def _tune(fields, steps, chunks, use_cache, batch, default_engine):
     lib = nat.load()
-    key = _key(fields) + ('|batch' if batch else '') + ('|default' if default_engine else '')
+    key = _key(fields) + ('|batch' if batch else '') + ('' if default_engine else '|table')
     cache = _load_cache() if use_cache else {}
     if key in cache:
         tile, chunk = cache[key]['tile'], cache[key]['chunk']

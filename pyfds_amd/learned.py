@@ -301,24 +301,28 @@ class LearnedBoundary:
 
     def time_methods(self, scene, steps):
         """Wall-clock of the plain enlarged run and of the learned-boundary run (setup and
-        shape tuning excluded, both FP32 with HIP-graph chunks)."""
+        shape tuning excluded, both FP32 with HIP-graph chunks), each on its own best shape of
+        the kernel table (``speedup``) and on the engine that a field runs by default
+        (``default_speedup``)."""
         torch = self.torch
         out = {}
-        for key, make in (('enlarged', lambda: self.field(scene, self.big, self.off, steps)),
-                          ('learned', lambda: self.attach(self.field(scene, self.G, 0, steps)))):
-            f = make()
-            f.assemble_matrices()
-            # each method on its own best kernel shape (tuning restores the field's state)
-            autotune.tune_field(f, steps=20, use_cache=False)
-            f.simulate(min(20, steps))           # warm-up (graph capture, first launches)
-            torch.cuda.synchronize()
-            t0 = time.perf_counter()
-            f.simulate(steps - f.step)
-            torch.cuda.synchronize()
-            out[key + '_s'] = time.perf_counter() - t0
-            out[key + '_steps'] = steps - 20
-            f._runner().close()
-        out['speedup'] = out['enlarged_s'] / out['learned_s']
+        for prefix in ('', 'default_'):
+            for key, make in (('enlarged', lambda: self.field(scene, self.big, self.off, steps)),
+                              ('learned', lambda: self.attach(self.field(scene, self.G, 0,
+                                                                         steps)))):
+                f = make()
+                f.assemble_matrices()
+                if not prefix:       # (tuning restores the field's state)
+                    autotune.tune_field(f, steps=20, use_cache=False, default_engine=False)
+                f.simulate(min(20, steps))           # warm-up (graph capture, first launches)
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                f.simulate(steps - f.step)
+                torch.cuda.synchronize()
+                out[prefix + key + '_s'] = time.perf_counter() - t0
+                out[prefix + key + '_steps'] = steps - 20
+                f._runner().close()
+            out[prefix + 'speedup'] = out[prefix + 'enlarged_s'] / out[prefix + 'learned_s']
         return out
 
     def validate(self, scene, tolerance=0.01, **kw):

@@ -292,3 +292,23 @@ def test_strips_too_tall_for_the_classes_leave_other_heights_alone():
     ref = scenes.build_oracle(scene)
     ref.simulate(20)
     np.testing.assert_array_equal(fld.pressure.values, ref.components['pressure'])
+
+
+def test_autotuner_times_the_engine_a_field_runs_by_itself(tmp_path, monkeypatch):
+    """By default tile -1 is among the candidates, of single fields and batches, and picks stored
+    before it was one are not applied."""
+    from pyfds_amd import autotune
+    monkeypatch.setattr(autotune, 'CACHE', str(tmp_path / 'tune.json'))
+    fields = [scenes.build_field(pyfds_amd, pyfds_amd.regions, _scene('Acoustic2D', 90, 40, seed=i))
+              for i in range(2)]
+    for f in fields:
+        f.assemble_matrices()
+    old = autotune._key(fields[:1]).rsplit('|', 1)[0] + '|v4'
+    autotune._save_cache({old: dict(tile=0, strip=0, chunk=50, table={'0,0,50': 1.0})})
+    tile, _, table = autotune.tune_field(fields[0], steps=6)
+    assert '-1,0,50' in table and '-1,8,50' in table and '0,0,50' in table
+    assert fields[0].tile == tile
+    _, _, table = autotune.tune_batch(fields, steps=6, use_cache=False)
+    assert '-1,0,50' in table
+    tile, _, table = autotune.tune_field(fields[0], steps=6, default_engine=False)
+    assert tile >= 0 and '-1,0,50' not in table
