@@ -194,7 +194,7 @@ struct fds_ctx {
   int ghost_rows = 0;     // ghost rows per side of a streaming strip (fuse - 1; lossy: 0)
   int sx = 0;             // x stride of the tiles (tx - 2*ghost)
   bool fused = false;     // fused engine in use (a row-streaming engine: streaming is set too)
-  bool coupled = false;   // stepped one step per launch by a coupling (until the next commit)
+  bool coupled = false;   // stepped one step per launch by a coupling (until it runs alone again)
   int fused_stages = 0, fused_rows = 0;   // layout a batch asked for (0: by the grid)
   // the layout (stages, strip height) whose tiles cannot hold the event lists (0: none known)
   int over_stages = 0, over_rows = 0;
@@ -1498,6 +1498,19 @@ int ready_classes(fds_ctx *c) {
   return c->elem == 8 ? find_classes<double>(c) : find_classes<float>(c);
 }
 
+// A field that a coupling stepped last (one step per launch, coefficients cell by cell) runs by
+// itself again: the layout and classes of its coefficients as the coupling left them.
+int leave_coupling(fds_ctx *c) {
+  if (!c->coupled) return 0;
+  c->coupled = false;
+  if (c->tile >= 0 || !fuse_reach(c)) return 0;      // (its engine is the same either way)
+  if (!c->npal)
+    if (int rc = ready_classes(c)) return rc;
+  if (int rc = choose_tiles(c)) return rc;
+  touch(c);
+  return 0;
+}
+
 int check_ctx(fds_ctx *c) {
   if (!c) return fail(FDS_E_ARG, "null context");
   hipError_t e = hipSetDevice(c->device);
@@ -2211,6 +2224,7 @@ int fds_run(fds_ctx *c, int64_t start, int64_t nsteps, int chunk) {
   if (!c->committed) return fail(FDS_E_STATE, "coefficients not committed");
   if (nsteps < 0 || start < 0) return fail(FDS_E_ARG, "negative step count");
   if (nsteps == 0) return 0;
+  if (int rc = leave_coupling(c)) return rc;
   if (int rc = prepare_run(c, start, nsteps)) return rc;
   if (int rc = enqueue_steps(c, nsteps, chunk, c->ev0, c->ev1)) return rc;
   if (int rc = stage_nonfinite(c, kMaxFlights, c->stream)) return rc;
@@ -2225,6 +2239,7 @@ int fds_prepare_run(fds_ctx *c, int64_t start, int64_t nsteps, int chunk) {
   if (int rc = check_idle(c)) return rc;
   if (!c->committed) return fail(FDS_E_STATE, "coefficients not committed");
   if (nsteps < 1 || start < 0) return fail(FDS_E_ARG, "a run needs steps");
+  if (int rc = leave_coupling(c)) return rc;
   if (int rc = prepare_run(c, start, nsteps)) return rc;
   if (int rc = capture_run_graphs(c, nsteps, chunk, true)) return rc;
   // the fused engines' stage counts are code objects of their own, loaded on their first launch
@@ -2251,6 +2266,7 @@ int fds_run_async(fds_ctx *c, int64_t start, int64_t nsteps, int chunk) {
   if (c->batch_flights) return fail(FDS_E_STATE, "a batch run of this context is in flight");
   if ((int)c->flights.size() >= kMaxFlights)
     return fail(FDS_E_STATE, "%d runs in flight: take the oldest first", kMaxFlights);
+  if (int rc = leave_coupling(c)) return rc;     // (a coupled run left none in flight)
   // a run that rebuilds tables or grows the output rows frees device memory the runs in
   // flight may read: let them finish first
   if (!run_steady(c, nsteps)) HIP_TRY(hipStreamSynchronize(c->stream));
@@ -2402,7 +2418,8 @@ int batch_layout(fds_batch *b, bool try_fused) {
     bool ok = true;
     for (auto *c : b->ctxs) {
       c->tile = -1;
-      if (!(can_stream_batch(c) && fuse_reach(c)) || c->coupled) ok = false;
+      if (int rc = leave_coupling(c)) return rc;
+      if (!(can_stream_batch(c) && fuse_reach(c))) ok = false;
       if (ok && !c->npal)
         if (int rc = ready_classes(c)) return rc;
       ok = ok && c->npal > 0;
@@ -2641,6 +2658,7 @@ int batch_prepare(fds_batch *b, int64_t start, int64_t nsteps) {
           return fail(FDS_E_INDEX, "boundary signal too short for step %lld",
                       (long long)(start + nsteps - 1));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    if (int rc = leave_coupling(c)) return rc;
   }
   int rc = b->elem == 8 ? batch_build<double>(b, nsteps) : batch_build<float>(b, nsteps);
   if (rc) return rc;

@@ -401,3 +401,41 @@ def test_device_power_law_paths(monkeypatch, caplog, power):
                                        err_msg=k)
         else:
             np.testing.assert_array_equal(dev[k], host[k], err_msg=k)
+
+
+@pytest.mark.gpu
+def test_fields_leave_a_coupling_for_their_own_engine():
+    """Plane fields coupled, run alone, and coupled again: alone they take the steps per launch of a
+    field that was never coupled (lossless and lossy), with the LDS-tile engine's bits."""
+    nx, ny, dx = 90, 60, 1e-4
+    res = []
+    for tile in (1, -1):
+        ac = fds.Acoustic2D(x_samples=nx, x_delta=dx, y_samples=ny, y_delta=dx, t_samples=100,
+                            t_delta=0.3 * dx / 1500,
+                            material=fds.AcousticMaterial(1500.0, 1000.0, absorption_coef=1e-3))
+        th = fds.Thermal2D(x_samples=nx, x_delta=dx, y_samples=ny, y_delta=dx, t_samples=100,
+                           t_delta=0.3 * dx / 1500, material=fds.ThermalMaterial(4000.0, 1000.0, 0.6))
+        rng = np.random.default_rng(0)
+        ac.pressure.values = rng.standard_normal(nx * ny)
+        th.temperature.values = rng.standard_normal(nx * ny)
+        ac.pressure.add_output(fds.regions.Region([5, nx * 30 + 40]))
+        ac.tile = th.tile = tile
+        # the thermal field feeds the acoustic one's density in a step-wise way: few classes
+        dens = fds.MaterialCouplingPowerLaw(th.temperature, ac, 'density', power=0, factor=1e-4)
+        fld = fds.SynchronizedFields([ac, th], [dens])
+        groups = []
+        for n in (5, 9):
+            fld.simulate(n)
+            for f in (ac, th):
+                step = f.step
+                f.simulate(n + 2)
+                f.step = step
+                lib = f._runner().lib
+                groups.append(lib.fds_steps_per_launch(f._runner().ctx))
+        print('coupled, alone', tile, groups, flush=True)
+        assert groups == ([1, 1] * 2 if tile == 1 else [3, 4] * 2)
+        res.append([np.array(c.values) for c in (ac.pressure, ac.velocity_x, ac.velocity_y,
+                                                 th.temperature)]
+                   + [np.array(ac.pressure.outputs[0].signals)])
+    for a, b in zip(*res):
+        np.testing.assert_array_equal(a, b)
