@@ -215,10 +215,6 @@ struct fds_ctx {
   DevBuf zero_ptr;        // ntiles+1 zeros: empty event lists
   const fds::KernelSet *ks = nullptr;
   size_t elem = 8;
-  // host transfers: conversion scratch, pinned chunks and the events after their copies
-  DevBuf conv;
-  HostBuf pinned;
-  hipEvent_t xev[8] = {};
   // graphs: key (chunk, parity) -> exec
   std::map<std::pair<int, int>, hipGraphExec_t> graphs;
   int graph_chunk = 0;              // steps of a full graph chunk (other graphs: run tails)
@@ -967,17 +963,98 @@ int transfer_small(fds_ctx *c, bool up, double *host, void *dev, void *comp, int
 // of Thermal2D 4096^2 FP32-Kahan with the state there and back: 87.7 ms before, 22.8 ms so (16.5
 // in the kernels); below 2^20 values a pass got up to 9 % slower.
 constexpr int64_t kXferChunk = 1 << 18;      // values (2 MB)
-constexpr int kXferThreads = 4;              // two chunks each: 16 MB pinned per large context
+constexpr int kXferThreads = 4;              // two chunks each
+constexpr int kXferSlots = 2 * kXferThreads;
 constexpr int64_t kXferLarge = 1 << 20;      // values from which an array takes this path
+constexpr size_t kXferKept = 2;              // idle workspaces a device keeps
+
+// What one large transfer works in: pinned chunks (16 MB), conversion scratch (FP32 forms, 16 MB)
+// and the events after the chunks' copies.
+struct Xfer {
+  HostBuf pinned;
+  DevBuf conv;
+  hipEvent_t ev[kXferSlots] = {};
+  ~Xfer() {
+    for (auto e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
+  hipError_t ready(bool convert) {
+    constexpr size_t bytes = kXferSlots * kXferChunk * 8;
+    hipError_t e = pinned.ensure(bytes);
+    if (e == hipSuccess && convert) e = conv.ensure(bytes);
+    for (auto &v : ev)
+      if (e == hipSuccess && !v) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    return e;
+  }
+};
+
+// The workspaces between transfers.  A sweep of many large fields transfers one or two of them at
+// a time, so they belong to the device and not to each field, and are freed with its last context.
+// (The pool itself is never destroyed: the runtime may be gone when the process ends.)
+struct XferPool {
+  struct PerDevice {
+    int contexts = 0;
+    std::vector<Xfer *> idle;
+  };
+  std::mutex mu;
+  std::map<int, PerDevice> devices;
+};
+
+XferPool &xfer_pool() {
+  static XferPool *pool = new XferPool;
+  return *pool;
+}
+
+void count_context(int device, int by) {
+  std::vector<Xfer *> gone;
+  XferPool &pool = xfer_pool();
+  {
+    std::lock_guard<std::mutex> lock(pool.mu);
+    XferPool::PerDevice &d = pool.devices[device];
+    d.idle.reserve(kXferKept);
+    d.contexts += by;
+    if (d.contexts == 0) gone.swap(d.idle);
+  }
+  for (auto *x : gone) delete x;
+}
+
+// A workspace, or null where its memory is not to be had.
+Xfer *take_xfer(const fds_ctx *c) {
+  Xfer *x = nullptr;
+  XferPool &pool = xfer_pool();
+  {
+    std::lock_guard<std::mutex> lock(pool.mu);
+    auto &idle = pool.devices[c->device].idle;
+    if (!idle.empty()) {
+      x = idle.back();
+      idle.pop_back();
+    }
+  }
+  if (!x) x = new Xfer;
+  if (x->ready(c->elem == 4) == hipSuccess) return x;
+  (void)hipGetLastError();
+  delete x;
+  return nullptr;
+}
+
+void give_xfer(const fds_ctx *c, Xfer *x) {
+  XferPool &pool = xfer_pool();
+  {
+    std::lock_guard<std::mutex> lock(pool.mu);
+    auto &idle = pool.devices[c->device].idle;
+    if (idle.size() < kXferKept) {
+      idle.push_back(x);
+      return;
+    }
+  }
+  delete x;
+}
 
 int transfer(fds_ctx *c, bool up, double *host, void *dev, void *comp, int64_t n) {
   if (n < kXferLarge) return transfer_small(c, up, host, dev, comp, n);
-  constexpr int kSlots = 2 * kXferThreads;
-  static_assert(kSlots == sizeof(fds_ctx::xev) / sizeof(hipEvent_t), "one event a chunk");
-  HIP_TRY(c->pinned.ensure(kSlots * kXferChunk * 8));
-  if (c->elem == 4) HIP_TRY(c->conv.ensure(kSlots * kXferChunk * 8));
-  for (auto &e : c->xev)
-    if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  Xfer *const ws = take_xfer(c);
+  if (!ws) return transfer_small(c, up, host, dev, comp, n);
+  double *const pinned = static_cast<double *>(ws->pinned.p), *const conv = ws->conv.as<double>();
   const int64_t chunks = (n + kXferChunk - 1) / kXferChunk;
   std::atomic<int> err{(int)hipSuccess};
   const auto worker = [&](int w) {
@@ -987,22 +1064,20 @@ int transfer(fds_ctx *c, bool up, double *host, void *dev, void *comp, int64_t n
     const auto count = [&](int64_t k) { return std::min(kXferChunk, n - k * kXferChunk); };
     const auto finish = [&]() {     // (down) the chunk in flight to the caller's array
       if (prev < 0 || e != hipSuccess) return;
-      e = hipEventSynchronize(c->xev[before]);
+      e = hipEventSynchronize(ws->ev[before]);
       if (e == hipSuccess)
-        std::memcpy(host + prev * kXferChunk,
-                    static_cast<double *>(c->pinned.p) + before * kXferChunk, count(prev) * 8);
+        std::memcpy(host + prev * kXferChunk, pinned + before * kXferChunk, count(prev) * 8);
     };
     for (int64_t k = w; k < chunks && e == hipSuccess; k += kXferThreads, ++i) {
       const int slot = 2 * w + (i & 1);
-      double *pin = static_cast<double *>(c->pinned.p) + slot * kXferChunk;
+      double *pin = pinned + slot * kXferChunk;
       if (up) {
-        if (i >= 2) e = hipEventSynchronize(c->xev[slot]);
+        if (i >= 2) e = hipEventSynchronize(ws->ev[slot]);
         std::memcpy(pin, host + k * kXferChunk, count(k) * 8);
       }
       if (e == hipSuccess)
-        e = move_piece(c, up, pin, dev, comp, c->conv.as<double>() + slot * kXferChunk,
-                       k * kXferChunk, count(k));
-      if (e == hipSuccess) e = hipEventRecord(c->xev[slot], c->stream);
+        e = move_piece(c, up, pin, dev, comp, conv + slot * kXferChunk, k * kXferChunk, count(k));
+      if (e == hipSuccess) e = hipEventRecord(ws->ev[slot], c->stream);
       if (!up) finish();
       prev = k;
       before = slot;
@@ -1020,8 +1095,10 @@ int transfer(fds_ctx *c, bool up, double *host, void *dev, void *comp, int64_t n
   worker(0);
   for (int w = started; w < kXferThreads; ++w) worker(w);
   for (auto &t : extra) t.join();
+  const hipError_t done = hipStreamSynchronize(c->stream);     // (the workspace is in use until then)
+  give_xfer(c, ws);
   HIP_TRY((hipError_t)err.load());
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(done);
   return 0;
 }
 
@@ -1628,6 +1705,7 @@ int fds_create(fds_ctx **out, int model, int form, int64_t nx, int64_t ny, int d
     delete c;
     return fail(FDS_E_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
   }
+  count_context(device, 1);
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess &&
       cus > 0)
@@ -1684,9 +1762,10 @@ int fds_destroy(fds_ctx *c) {
   for (auto &set : c->fev)
     for (auto e : set)
       if (e) (void)hipEventDestroy(e);
-  for (auto e : c->xev)
-    if (e) (void)hipEventDestroy(e);
-  if (c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->stream) {
+    (void)hipStreamDestroy(c->stream);
+    count_context(c->device, -1);
+  }
   delete c;
   return 0;
 }

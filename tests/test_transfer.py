@@ -50,3 +50,65 @@ def test_state_round_trip_rounds_like_ieee(form, nx, ny):
             np.testing.assert_array_equal(np.signbit(got[want == 0]), np.signbit(want[want == 0]))
     finally:
         lib.fds_destroy(ctx)
+
+
+def test_large_contexts_share_the_transfer_workspace():
+    """A context's first large transfer takes no device memory of its own once another's has been,
+    and the last context's end gives the workspace back.  (The first round loads the kernels, which
+    the runtime keeps.)"""
+    import torch
+    lib = nat.load()
+    nx = ny = 1 << 10
+    v = np.random.default_rng(0).standard_normal(nx * ny)
+    got = np.empty_like(v)
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    for _ in range(2):
+        ctxs, before = [], free()
+        try:
+            for i in range(4):
+                ctx = ct.c_void_p()
+                nat.check(lib.fds_create(ct.byref(ctx), nat.ACOUSTIC2D, nat.FORMS['fp32'], nx, ny,
+                                         0))
+                ctxs.append(ctx)
+                held = free()
+                nat.check(lib.fds_set_state(ctx, 0, v.ctypes.data_as(DP), v.size))
+                nat.check(lib.fds_get_state(ctx, 0, got.ctypes.data_as(DP), v.size))
+                np.testing.assert_array_equal(got, v.astype(np.float32))
+                if i:
+                    assert held - free() < 4 << 20
+        finally:
+            for ctx in ctxs:
+                lib.fds_destroy(ctx)
+    assert before - free() < 4 << 20
+
+
+def test_large_transfers_of_several_threads():
+    import threading
+    lib = nat.load()
+    nx, ny = 1031, 1021
+    errors = []
+
+    def work(seed, form):
+        try:
+            v = np.random.default_rng(seed).standard_normal(nx * ny)
+            got = np.empty_like(v)
+            ctx = ct.c_void_p()
+            nat.check(lib.fds_create(ct.byref(ctx), nat.ACOUSTIC2D, nat.FORMS[form], nx, ny, 0))
+            for _ in range(3):
+                nat.check(lib.fds_set_state(ctx, 0, v.ctypes.data_as(DP), v.size))
+                nat.check(lib.fds_get_state(ctx, 0, got.ctypes.data_as(DP), v.size))
+                np.testing.assert_array_equal(got, v if form == 'fp64' else v.astype(np.float32))
+            lib.fds_destroy(ctx)
+        except BaseException as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i, ('fp64', 'fp32')[i % 2])) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
