@@ -1477,55 +1477,104 @@ int get_graph(fds_ctx *c, int chunk, int parity, hipGraphExec_t *out) {
 
 // Material classes.  Cells with the same coefficients (by their bits) are one class; a field whose
 // cells form fewer than kPalMax classes gets an array of class numbers, one byte a cell, and a
-// table of the classes' coefficients.  Pass q compares every cell without a class to the first
-// such cell (`first[q]`, found by the pass before), gives the equal ones class q + 1 and finds
-// the first cell left.
+// table of the classes' coefficients.  The table is a hash table of the classes' first cells found:
+// a wave looks the coefficients of its first cell without a class up, gives the class to all its
+// cells that have them, and goes on with the next such cell.  A class that finds no slot ends the
+// search: the field has too many.
+//
+// One pass over the coefficients, and one launch whatever the number of classes (a pass a class
+// costs a field of 80 materials 0.65 ms at each commit, at any size).
 template <typename T>
 struct PalCoefs {
   const T *c[fds::kPalSlots];   // in the table's order
 };
 
+constexpr int kPalClasses = fds::kPalMax - 1;     // slots; tab[kPalClasses]: too many classes
+
+__device__ __forceinline__ uint32_t lane_bits(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ uint64_t lane_bits(uint64_t v, int lane) {
+  return (uint64_t)lane_bits((uint32_t)(v >> 32), lane) << 32 | lane_bits((uint32_t)v, lane);
+}
+
 template <typename T, int NC>
-__global__ __launch_bounds__(256) void k_pal_pass(PalCoefs<T> pc, int64_t n, uint8_t *idx, T *pal,
-                                                  unsigned *first, unsigned *count, int q) {
+__global__ __launch_bounds__(256) void k_classes(PalCoefs<T> pc, int64_t n, uint8_t *idx, T *pal,
+                                                 unsigned *tab) {
   using B = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
-  const unsigned f = first[q];
-  if (f == ~0u) return;
-  B b[NC];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) {
-    b[k] = __builtin_bit_cast(B, pc.c[k][f]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) pal[(q + 1) * fds::kPalSlots + k] = pc.c[k][f];
-  }
+  const int lane = threadIdx.x & 63;
   const int64_t stride = (int64_t)gridDim.x * 256;
-  unsigned left = ~0u, rest = 0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-    if (q > 0 && idx[i]) continue;
-    bool eq = true;
+  B last[NC] = {};       // the class looked up last (0: none)
+  int cls = 0;
+  for (int64_t i0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63); i0 < n; i0 += stride) {
+    if (__hip_atomic_load(tab + kPalClasses, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    const int64_t i = i0 + lane;
+    const bool in = i < n;
+    B own[NC];
 #pragma unroll
-    for (int k = 0; k < NC; ++k) eq = eq && __builtin_bit_cast(B, pc.c[k][i]) == b[k];
-    if (eq) {
-      idx[i] = (uint8_t)(q + 1);
-    } else {
-      if (q == 0) idx[i] = 0;
-      ++rest;
-      if (left == ~0u) left = (unsigned)i;
+    for (int k = 0; k < NC; ++k) own[k] = in ? __builtin_bit_cast(B, pc.c[k][i]) : B(0);
+    int mine = 0;
+    for (uint64_t left = __ballot(in); left;) {
+      const int lead = __builtin_ctzll(left);
+      B key[NC];
+      bool same = cls != 0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        key[k] = lane_bits(own[k], lead);
+        same = same && key[k] == last[k];
+      }
+      if (!same) {
+        uint64_t h = 0;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+          h = (h ^ key[k]) * 0x9e3779b97f4a7c15ull;      // (the golden ratio's bits, odd)
+          h ^= h >> 29;
+          last[k] = key[k];
+        }
+        unsigned s = (unsigned)(((h >> 32) * kPalClasses) >> 32);
+        cls = 0;
+        for (int t = 0; t < kPalClasses && !cls; ++t) {
+          unsigned f = __hip_atomic_load(tab + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (f == 0) {
+            if (lane == lead) f = atomicCAS(tab + s, 0u, (unsigned)i + 1);
+            f = lane_bits(f, lead);
+            if (f == 0) {        // the slot is this class's
+              cls = (int)s + 1;
+              if (lane == lead) {
+#pragma unroll
+                for (int k = 0; k < NC; ++k)
+                  pal[cls * fds::kPalSlots + k] = __builtin_bit_cast(T, own[k]);
+              }
+              break;
+            }
+          }
+          bool eq = true;
+#pragma unroll
+          for (int k = 0; k < NC; ++k)
+            eq = eq && __builtin_bit_cast(B, pc.c[k][f - 1]) == key[k];
+          if (eq) cls = (int)s + 1;
+          s = s + 1 == kPalClasses ? 0 : s + 1;
+        }
+        if (!cls) {
+          if (lane == lead)
+            __hip_atomic_store(tab + kPalClasses, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          return;
+        }
+      }
+      bool eq = in;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) eq = eq && own[k] == key[k];
+      if (eq) mine = cls;
+      left &= ~__ballot(eq);
     }
-  }
-  for (int d = 32; d > 0; d >>= 1) {
-    left = min(left, (unsigned)__shfl_xor((int)left, d));
-    rest += (unsigned)__shfl_xor((int)rest, d);
-  }
-  if ((threadIdx.x & 63) == 0 && left != ~0u) {
-    atomicMin(first + q + 1, left);
-    atomicAdd(count + q + 1, rest);
+    if (in) idx[i] = (uint8_t)mine;
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_pal_init(T *pal, int coefs, unsigned *first, int slots) {
+__global__ __launch_bounds__(256) void k_pal_init(T *pal, int coefs, unsigned *tab, int slots) {
   for (int i = threadIdx.x; i < coefs; i += 256) pal[i] = T(0);
-  for (int i = threadIdx.x; i < 2 * slots; i += 256) first[i] = i > 0 && i < slots ? ~0u : 0u;
+  for (int i = threadIdx.x; i < slots; i += 256) tab[i] = 0u;
 }
 
 template <typename T>
@@ -1538,33 +1587,20 @@ int find_classes(fds_ctx *c) {
   // (thermal: Q, G in the places of B, K)
   const PalCoefs<T> pc{{slot(2, -1), slot(0, -1), slot(3, 2), slot(1, 0), slot(4, -1), slot(5, 4),
                         slot(6, -1), slot(7, -1)}};
-  constexpr int kSlots = fds::kPalMax + 1, kCoefs = fds::kPalMax * fds::kPalSlots;
-  unsigned f[2 * kSlots];                     // first cells, then counts of the cells left
+  constexpr int kCoefs = fds::kPalMax * fds::kPalSlots;
   HIP_TRY(c->pal_idx.ensure(c->n));
-  HIP_TRY(c->pal.ensure(kCoefs * sizeof(T) + sizeof f));     // (f's device side behind the table)
-  unsigned *const first = reinterpret_cast<unsigned *>(c->pal.as<T>() + kCoefs);
-  hipLaunchKernelGGL(k_pal_init<T>, dim3(1), dim3(256), 0, c->stream, c->pal.as<T>(), kCoefs, first,
-                     kSlots);
+  HIP_TRY(c->pal.ensure(kCoefs * sizeof(T) + (kPalClasses + 1) * sizeof(unsigned)));
+  unsigned *const tab = reinterpret_cast<unsigned *>(c->pal.as<T>() + kCoefs);
+  hipLaunchKernelGGL(k_pal_init<T>, dim3(1), dim3(256), 0, c->stream, c->pal.as<T>(), kCoefs, tab,
+                     kPalClasses + 1);
   const unsigned nb = (unsigned)std::min<int64_t>((c->n + 1023) / 1024, 2048);
-  const int most = fds::kPalMax - 1;
-  for (int q = 0; q < most;) {
-    const int q1 = std::min(q + 4, most);
-    for (; q < q1; ++q)
-      hipLaunchKernelGGL((lossy ? k_pal_pass<T, 8> : k_pal_pass<T, 4>), dim3(nb), dim3(256), 0,
-                         c->stream, pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(), first,
-                         first + kSlots, q);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(f, first, sizeof f, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (f[q] == ~0u) {
-      while (q > 1 && f[q - 1] == ~0u) --q;
-      c->npal = q + 1;
-      return 0;
-    }
-    // graded media (a lossless field runs without classes): the first eight hold less than an
-    // eighth of the cells, so 63 are unlikely to hold all
-    if (!lossy && q == 8 && f[kSlots + q] > c->n / 8 * 7) return 0;
-  }
+  hipLaunchKernelGGL((lossy ? k_classes<T, 8> : k_classes<T, 4>), dim3(nb), dim3(256), 0, c->stream,
+                     pc, c->n, c->pal_idx.as<uint8_t>(), c->pal.as<T>(), tab);
+  HIP_TRY(hipGetLastError());
+  unsigned over = 0;
+  HIP_TRY(hipMemcpyAsync(&over, tab + kPalClasses, sizeof over, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (!over) c->npal = fds::kPalMax;
   return 0;
 }
 

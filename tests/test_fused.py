@@ -312,3 +312,32 @@ def test_autotuner_times_the_engine_a_field_runs_by_itself(tmp_path, monkeypatch
     assert '-1,0,50' in table
     tile, _, table = autotune.tune_field(fields[0], steps=6, default_engine=False)
     assert tile >= 0 and '-1,0,50' not in table
+
+
+@pytest.mark.parametrize('mu', [0.0, 0.3])
+@pytest.mark.parametrize('rows', [62, 63, 64])
+def test_as_many_materials_as_the_table_holds(rows, mu):
+    """A material a row; the class table holds 63.  Lossy fields of more take one step a launch."""
+    scene = _scene('Acoustic2D', 71, rows, medium='rows', mu=mu)
+    print('materials', rows, mu, flush=True)
+    ref = scenes.run_oracle(scene)
+    got, group = _run(scene)
+    assert group == (4 if not mu else 3 if rows <= 63 else 1)
+    for k in ref:
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+@pytest.mark.parametrize('form', ['fp64', 'fp32'])
+def test_classes_of_scattered_materials(form):
+    """50 materials cell by cell at random, a few of them equal in all but one coefficient."""
+    scene = _scene('Acoustic2D', 301, 97, seed=9)
+    rng = np.random.default_rng(9)
+    of = rng.integers(0, 50, 301 * 97)
+    base = dict(scenes.WATER)
+    scene['regions'] = [(np.flatnonzero(of == i), ('AcousticMaterial', dict(
+        base, sound_velocity=1000.0 + 40.0 * (i // 2), density=900.0 + (i % 2)))) for i in range(50)]
+    a, _ = _run(scene, form=form, tile=1)
+    b, group = _run(scene, form=form)
+    assert group == 4
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
