@@ -1482,14 +1482,17 @@ int get_graph(fds_ctx *c, int chunk, int parity, hipGraphExec_t *out) {
 // cells that have them, and goes on with the next such cell.  A class that finds no slot ends the
 // search: the field has too many.
 //
-// One pass over the coefficients, and one launch whatever the number of classes (a pass a class
-// costs a field of 80 materials 0.65 ms at each commit, at any size).
+// One pass over the coefficients, and one launch whatever the number of classes: bound by the
+// latency of its lookups on small fields.  A commit takes 39 us with it, 50000 cells of one
+// material or of 200 (0.7 ms for the latter with a pass a class; 65 us with the slots of a lookup
+// tried one after the other).
 template <typename T>
 struct PalCoefs {
   const T *c[fds::kPalSlots];   // in the table's order
 };
 
 constexpr int kPalClasses = fds::kPalMax - 1;     // slots; tab[kPalClasses]: too many classes
+static_assert(kPalClasses == 63, "a slot a lane");
 
 __device__ __forceinline__ uint32_t lane_bits(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
@@ -1507,7 +1510,6 @@ __global__ __launch_bounds__(256) void k_classes(PalCoefs<T> pc, int64_t n, uint
   B last[NC] = {};       // the class looked up last (0: none)
   int cls = 0;
   for (int64_t i0 = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63); i0 < n; i0 += stride) {
-    if (__hip_atomic_load(tab + kPalClasses, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
     const int64_t i = i0 + lane;
     const bool in = i < n;
     B own[NC];
@@ -1531,34 +1533,42 @@ __global__ __launch_bounds__(256) void k_classes(PalCoefs<T> pc, int64_t n, uint
           h ^= h >> 29;
           last[k] = key[k];
         }
-        unsigned s = (unsigned)(((h >> 32) * kPalClasses) >> 32);
+        const int home = (int)(((h >> 32) * kPalClasses) >> 32);
+        // all slots at a time, one a lane (the last lane: too many); a slot another wave took
+        // meanwhile shows next time
         cls = 0;
-        for (int t = 0; t < kPalClasses && !cls; ++t) {
-          unsigned f = __hip_atomic_load(tab + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (f == 0) {
-            if (lane == lead) f = atomicCAS(tab + s, 0u, (unsigned)i + 1);
-            f = lane_bits(f, lead);
-            if (f == 0) {        // the slot is this class's
-              cls = (int)s + 1;
-              if (lane == lead) {
+        while (!cls) {
+          const unsigned f = __hip_atomic_load(tab + lane, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+          if (lane_bits(f, kPalClasses)) return;
+          bool eq = f != 0 && lane < kPalClasses;
+          if (eq) {
 #pragma unroll
-                for (int k = 0; k < NC; ++k)
-                  pal[cls * fds::kPalSlots + k] = __builtin_bit_cast(T, own[k]);
-              }
-              break;
+            for (int k = 0; k < NC; ++k)
+              eq = eq && __builtin_bit_cast(B, pc.c[k][f - 1]) == key[k];
+          }
+          const uint64_t hit = __ballot(eq), empty = __ballot(f == 0 && lane < kPalClasses);
+          if (hit) {
+            cls = __builtin_ctzll(hit) + 1;
+          } else if (!empty) {
+            if (lane == lead)
+              __hip_atomic_store(tab + kPalClasses, 1u, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+            return;
+          } else {
+            // the first empty slot from the key's own on: waves with one key try one slot
+            const uint64_t after = empty >> home << home;
+            const int s = __builtin_ctzll(after ? after : empty);
+            unsigned was = 1;
+            if (lane == lead) was = atomicCAS(tab + s, 0u, (unsigned)i + 1);
+            if (lane_bits(was, lead)) continue;
+            cls = s + 1;
+            if (lane == lead) {
+#pragma unroll
+              for (int k = 0; k < NC; ++k)
+                pal[cls * fds::kPalSlots + k] = __builtin_bit_cast(T, own[k]);
             }
           }
-          bool eq = true;
-#pragma unroll
-          for (int k = 0; k < NC; ++k)
-            eq = eq && __builtin_bit_cast(B, pc.c[k][f - 1]) == key[k];
-          if (eq) cls = (int)s + 1;
-          s = s + 1 == kPalClasses ? 0 : s + 1;
-        }
-        if (!cls) {
-          if (lane == lead)
-            __hip_atomic_store(tab + kPalClasses, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          return;
         }
       }
       bool eq = in;
