@@ -341,3 +341,23 @@ def test_classes_of_scattered_materials(form):
     assert group == 4
     for k in a:
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+@pytest.mark.parametrize('nx, ny', [(130, 60), (5, 90)])
+def test_boundary_and_output_cells_in_any_order(nx, ny):
+    """Cells handed over in descending and in random order (the event lists are sorted by tile and
+    place), rows shorter than a strip among them: the oracle's bits."""
+    scene = _scene('Acoustic2D', nx, ny, boundaries='walls', seed=2)
+    rng = np.random.default_rng(2)
+    n = nx * ny
+    scene['boundaries']['velocity_x'].append(dict(
+        indices=[int(v) for v in rng.permutation(n)[:n // 3]], value=0.125, additive=False))
+    scene['boundaries']['velocity_y'].append(dict(
+        indices=list(range(n - 1, 0, -7)), value=-0.5, additive=True))
+    scene['outputs']['pressure'].append([int(v) for v in rng.permutation(n)[:400]])
+    scene['outputs']['velocity_y'].append(list(range(n - 1, 0, -11)))
+    ref = scenes.run_oracle(scene)
+    got, group = _run(scene)
+    assert group == 4
+    for k in ref:
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
