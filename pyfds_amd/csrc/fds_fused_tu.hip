@@ -126,9 +126,12 @@ void FDS_CAT(fill_fused_, FDS_STAGES)(KernelSet &ks) {
   ks.fused_batch[0][S - 1] = launch_fused_batch<S, false>;
   ks.fused_batch[1][S - 1] = launch_fused_batch<S, true>;
   if constexpr (S <= kFusedLossyMax) {
-    ks.fused_lossy[0][S - 1] = launch_fused_lossy<S, false, false>;
-    ks.fused_lossy[1][S - 1] = launch_fused_lossy<S, true, false>;
-    ks.fused_lossy[2][S - 1] = launch_fused_lossy<S, false, true>;
+    // (four stages: the FP32 forms' plane fields only, see choose_fused)
+    if constexpr (S < kFusedLossyMax) ks.fused_lossy[1][S - 1] = launch_fused_lossy<S, true, false>;
+    if constexpr (S < kFusedLossyMax || sizeof(T) == 4) {
+      ks.fused_lossy[0][S - 1] = launch_fused_lossy<S, false, false>;
+      ks.fused_lossy[2][S - 1] = launch_fused_lossy<S, false, true>;
+    }
   }
 }
 

@@ -361,3 +361,18 @@ def test_boundary_and_output_cells_in_any_order(nx, ny):
     assert group == 4
     for k in ref:
         np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+@pytest.mark.parametrize('model, form, nx, ny, group', [
+    ('Acoustic2D', 'fp32', 1031, 1021, 4), ('Acoustic2D', 'fp32_kahan', 1033, 1019, 4),
+    ('Acoustic2D', 'fp64', 1031, 1021, 3), ('Acoustic3DAxi', 'fp64', 2053, 2047, 3)])
+def test_large_lossy_fields_equal_tile_engine(model, form, nx, ny, group):
+    """The stage counts that only large lossy fields take, with remainder launches."""
+    scene = _scene(model, nx, ny, boundaries='walls', mu=0.3, seed=6)
+    scene['plan'] = [('simulate', 9), ('simulate', 6)]
+    print('large lossy', model, form, flush=True)
+    a, _ = _run(scene, form=form, tile=1)
+    b, got = _run(scene, form=form)
+    assert got == group
+    for k in a:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
