@@ -10,7 +10,9 @@ burst as an additive pressure point source at the centre, dt at CFL 0.5 on the s
 velocity, 64 recorded pressure points; everything is set up through the pyfds-compatible API
 of pyfds_amd and timed through ``Field.simulate`` (device run + output download).
 
-Prints one JSON line.  ``value`` is the FP64 drop-in form (bit-identical to the reference's
+Prints one JSON line of the headline figures, under 2 KB, and writes the full record (autotuner
+tables, traffic, every layout timed) to the file of ``--detail``, whose path the line names.
+``value`` is the FP64 drop-in form (bit-identical to the reference's
 float64 arithmetic); the FP32 and FP32-Kahan forms are reported under ``forms`` with their
 relative L2 error against the FP64 result.  ``roofline`` uses the algorithmic bytes per cell
 update (FP64: p, vx, vy read + write and the two coefficients K, B = 8 words = 64 B) times the
@@ -55,6 +57,7 @@ import argparse
 import json
 import os
 import sys
+import tempfile
 import time
 
 import numpy as np
@@ -862,6 +865,34 @@ def cpu_baseline(wl, steps, rate=True):
     return n * steps / wall / 1e9 if rate else (n * steps, wall)
 
 
+def summary(line, detail):
+    """The headline figures of the full record ``line``, short enough for one line of output."""
+    def pick(d, *keys):
+        return {k: float('%.4g' % d[k]) if isinstance(d[k], float) else d[k]
+                for k in keys if k in d}
+
+    out = {k: v for k, v in line.items() if not isinstance(v, dict)}
+    out['config'] = line['config']
+    out['roofline'] = pick(line['roofline'], 'bound', 'achieved', 'peak', 'unit', 'frac', 'traffic')
+    if line['cpu_baseline']:
+        out['cpu_baseline'] = pick(line['cpu_baseline'], 'value', 'unit', 'cores', 'kind')
+        out['cpu_baseline']['sample'] = 'scipy oracle, same scene, few steps'
+    for name in ('forms', 'lossy', 'batched', 'thermal2d'):
+        if name in line:
+            out[name] = {f: pick(r, 'value', 'ms_per_step') for f, r in line[name].items()
+                         if isinstance(r, dict) and 'ms_per_step' in r}
+    for f, r in line['forms'].items():
+        out['forms'][f].update(pick(r, 'rel_l2_vs_fp64'))
+    if 'acoustic1d' in line:
+        out['acoustic1d'] = pick(line['acoustic1d']['fp64'], 'us_per_step')
+    if 'learned_bc' in line:
+        out['learned_bc'] = pick(line['learned_bc'], 'reflected_energy', 'learned_s', 'enlarged_s',
+                                 'speedup_vs_enlarged')
+        out['learned_bc']['default_engines'] = line['learned_bc']['default_engines']
+    out['detail'] = detail
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument('--gpus', type=int, default=1)
@@ -893,6 +924,9 @@ def main():
     ap.add_argument('--batch-strip', type=int, default=0)
     ap.add_argument('--no-traffic', action='store_true',
                     help='skip the rocprofv3 HBM traffic measurement of the chosen shapes')
+    ap.add_argument('--detail', default=os.path.join(tempfile.gettempdir(),
+                                                     'pyfds_amd_bench_detail.json'),
+                    help='file for the full record')
     ap.add_argument('--traffic-probe', default=None, help=argparse.SUPPRESS)
     args = ap.parse_args()
     if args.traffic_probe:
@@ -1070,7 +1104,13 @@ def main():
         line['thermal2d'] = th
     if 'learned' in sections:
         line['learned_bc'] = learned_section(args.no_cpu, iters=args.learned_iters)
-    print(json.dumps(line), flush=True)
+    try:
+        with open(args.detail, 'w') as f:
+            json.dump(line, f, indent=1)
+    except OSError as e:
+        print('no full record: %s' % e, file=sys.stderr)
+        args.detail = None
+    print(json.dumps(summary(line, args.detail)), flush=True)
 
 
 if __name__ == '__main__':
