@@ -2575,16 +2575,10 @@ int batch_layout(fds_batch *b, bool try_fused) {
       ok = ok && c->npal > 0;
       cells += c->n;
     }
-    // The stages by the rule of one field (choose_fused) on the whole batch; the height for 16
-    // strips a CU whatever the form: the kernel's registers are those of its largest member model.
-    // us a step at 16 and 24: 40 plane and axial members, 128 to 640 cells a side, FP64 12.8 and
-    // 12.6, FP32 6.2 and 6.3, Kahan 13.8 and 13.7; 12 of 500 x 480 FP64 6.2 and 6.6, FP32 4.3 and
-    // 4.5, Kahan 6.5 and 7.0; 100 of 100 to 200 FP64 5.8 and 6.2, Kahan 6.1 and 6.6; 4 of
-    // 1500 x 1400 FP64 17.9 and 20.1, FP32 7.9 and 8.3, thermal FP64 7.2 and 8.2.  (12: 12.4 of
-    // the first, but 18.8 and 8.8 of the last.)
+    // stages and height by the rules of one field (choose_fused) on the whole batch
     const int S = cells < (1 << 18) ? 4 : fds::kFusedMax, sx = 64 - 2 * S;
     for (auto *c : b->ctxs) across += (c->nx + sx - 1) / sx * c->ny;
-    const int64_t strips = 16 * (int64_t)b->ctxs[0]->num_cu;
+    const int64_t strips = 24 * (int64_t)b->ctxs[0]->num_cu;
     const int64_t want = (across + strips / 2) / strips;
     for (auto *c : b->ctxs) {
       if (!ok) break;
