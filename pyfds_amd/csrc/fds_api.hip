@@ -2575,7 +2575,14 @@ int batch_layout(fds_batch *b, bool try_fused) {
       ok = ok && c->npal > 0;
       cells += c->n;
     }
-    // stages and height by the rules of one field (choose_fused) on the whole batch
+    // The stages by the rule of one field (choose_fused) on the whole batch; the height for 24
+    // strips a CU in every form: a launch ends with the tiles that hold sources and recorded points,
+    // which every member has, and short strips shorten those.  us a step at 16, 20, 24 and 28, with
+    // a source line and 8 points a member: 40 plane and axial members, 128 to 640 cells a side,
+    // FP64 13.7, 13.3, 13.8, 13.8, FP32 8.4, 8.0, 7.0, 6.9, Kahan 14.5, 14.1, 14.3, 14.3; 12 of
+    // 500 x 480 FP64 7.1, 6.5, 6.2, 6.3, FP32 5.6, 5.3, 4.9, 4.8; 60 of 100 to 200 FP64 5.9, 5.7,
+    // 6.0, 6.4, Kahan 6.1, 6.1, 6.3, 6.8; 4 of 1500 x 1400 FP64 19.7, 19.2, 20.1, 19.6, FP32 11.1,
+    // 9.9, 9.3, 9.2; 64 of 128 to 1024 level.  (Without any source or point 16 is 3 to 10 % ahead.)
     const int S = cells < (1 << 18) ? 4 : fds::kFusedMax, sx = 64 - 2 * S;
     for (auto *c : b->ctxs) across += (c->nx + sx - 1) / sx * c->ny;
     const int64_t strips = 24 * (int64_t)b->ctxs[0]->num_cu;
