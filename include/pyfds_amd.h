@@ -158,16 +158,18 @@ int fds_run_take(fds_ctx *ctx, double *dst0, double *dst1, double *dst2);
 int fds_prepare_run(fds_ctx *ctx, int64_t start_step, int64_t nsteps, int chunk);
 
 /* Tile shape of the 2D step kernels (autotuner hook): index into the compiled shape table,
- * or -1 for the default: lossless 2D fields run the fused engine (one-wave strips, up to six
- * steps per launch, height by fds_set_strip_height), which has no entry in the table.  fds_tile_count reports the table size, fds_tile_shape its entries
+ * or -1 for the default: 2D fields run the fused engines (one-wave strips, up to six steps per
+ * launch for lossless models, two to four for lossy ones of up to 63 materials, height by
+ * fds_set_strip_height), which have no entry in the table; lossy fields of more materials stream
+ * one step per launch.  fds_tile_count reports the table size, fds_tile_shape its entries
  * (tx columns x ty rows).  fds_tile_engine returns 0 for an LDS-tile shape and 1 for a
  * row-streaming shape (a workgroup of tx threads marching down a strip of ty rows); streaming
  * shapes serve the 2D models (lossy acoustics one time step per launch on any of them).
  * 1D models (Acoustic1D, Thermal1D, IdealGas1D, Acoustic2ndOrder1D) of up to 2^24 cells
  * default (-1) to the resident 1D engine: workgroups keep the line in registers for many steps
  * per launch (one wave up to 64 cells, one-wave segments beyond; see fds_set_line_shape); any tile
- * index (and longer lines) puts them on the LDS-tile kernels (one launch per step; nonlinear models on their 256-cell tiles
- * whatever the index). */
+ * index (and longer lines) puts them on the LDS-tile kernels (one launch per step; nonlinear
+ * models on their 256-cell tiles whatever the index). */
 int fds_set_tile(fds_ctx *ctx, int tile_index);
 int fds_tile_count(void);
 int fds_tile_shape(int tile_index, int *tx, int *ty);
@@ -191,11 +193,11 @@ int fds_set_strip_height(fds_ctx *ctx, int rows);
  * blocking).  Lines of up to 2^24 cells; longer ones ignore the layout and step on the
  * LDS-tile kernels. */
 int fds_set_line_shape(fds_ctx *ctx, int cells_per_thread, int threads, int ghost);
-/* Engine that runs a context's steps: 0 LDS tiles, 1 row streaming, 2 resident 1D,
+/* Engine that runs a context's steps: 0 LDS tiles, 1 row streaming or fused, 2 resident 1D,
  * 3 nonlinear 1D tiles (no reference counterpart; for tests and benchmarks). */
 int fds_engine(fds_ctx *ctx);
-/* Time steps one launch of the context's 2D step kernel advances (the streaming shape's fused
- * stage count, else 1; no reference counterpart): runs whose length is a multiple of it use
+/* Time steps one launch of the context's 2D step kernel advances (the fused engines' or the
+ * streaming shape's stage count, else 1; no reference counterpart): runs whose length is a multiple of it use
  * fused launches only. */
 int fds_steps_per_launch(fds_ctx *ctx);
 

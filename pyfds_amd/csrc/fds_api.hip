@@ -489,7 +489,8 @@ bool can_ring(const fds_ctx *c, int S) {
 // step at 16 and 24: FP64 1200 x 1100 3.70 and 4.14, 2048^2 7.0 and 7.0, 3000 x 2500 16.7 and
 // 16.3, thermal 1500^2 3.47 and 3.64, AXI 1024 x 1536 3.99 and 4.79, Kahan AXI 4.13 and 4.92;
 // Kahan 2048^2 7.45 and 7.29, thermal 1500^2 3.16 and 2.94; FP32 1500 x 1203 3.23 and 3.02,
-// 2500^2 5.8 and 5.3.  Rows beyond 64 or below 4 gained nothing at any size.
+// 2500^2 5.8 and 5.3.  Rows beyond 64 or below 4 gained nothing at any size.  (Not the best at
+// every size: 2048^2 FP64 takes 43.7 us a launch at the rule's height, 40.5 in strips of 12.)
 //
 // 1: no such layout, the tiles of this one cannot hold the event lists.
 int choose_fused(fds_ctx *c) {
