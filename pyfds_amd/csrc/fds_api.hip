@@ -1560,12 +1560,13 @@ __global__ __launch_bounds__(256) void k_classes(PalCoefs<T> pc, int64_t n, uint
           last[k] = key[k];
         }
         const int home = (int)(((h >> 32) * kPalClasses) >> 32);
-        // all slots at a time, one a lane (the last lane: too many); a slot another wave took
-        // meanwhile shows next time
+        // all slots at a time, one a lane (the last lane: too many); each turn without a class has
+        // at least one slot more to compare, which another wave took meanwhile
         cls = 0;
+        unsigned f = 0;
         while (!cls) {
-          const unsigned f = __hip_atomic_load(tab + lane, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
+          if (f == 0)
+            f = __hip_atomic_load(tab + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           if (lane_bits(f, kPalClasses)) return;
           bool eq = f != 0 && lane < kPalClasses;
           if (eq) {
@@ -1585,9 +1586,13 @@ __global__ __launch_bounds__(256) void k_classes(PalCoefs<T> pc, int64_t n, uint
             // the first empty slot from the key's own on: waves with one key try one slot
             const uint64_t after = empty >> home << home;
             const int s = __builtin_ctzll(after ? after : empty);
-            unsigned was = 1;
+            unsigned was = 0;
             if (lane == lead) was = atomicCAS(tab + s, 0u, (unsigned)i + 1);
-            if (lane_bits(was, lead)) continue;
+            was = lane_bits(was, lead);
+            if (was) {
+              if (lane == s) f = was;
+              continue;
+            }
             cls = s + 1;
             if (lane == lead) {
 #pragma unroll
