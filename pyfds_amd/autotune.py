@@ -171,6 +171,8 @@ def _tune(fields, steps, chunks, use_cache, batch, default_engine):
 def _set_strip(fields, strip):
     lib = nat.load()
     for f in fields:
+        if f._device_grid()[1] == 1:      # 1D: a layout of the line (line_shape), not a strip
+            continue
         f.strip_height = strip
         r = f.__dict__.get('_device_runner')
         if r is not None:

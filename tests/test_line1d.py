@@ -306,3 +306,17 @@ def test_ideal_gas_long_run_matches_cr_oracle_bitwise(engine):
     assert eng == engine
     for k in ref:
         np.testing.assert_array_equal(res[k], ref[k], err_msg='%s %s' % (engine, k))
+
+
+def test_autotuner_leaves_a_line_its_layout():
+    """Tuning times the engine a line runs by itself (tile -1) with the layout it was given: the
+    resident engine, which one launch a step does not beat."""
+    import pyfds_amd
+    from pyfds_amd import autotune
+    fld = pyfds_amd.Acoustic1D(x_samples=700, x_delta=1e-4, t_samples=100, t_delta=0.3e-7,
+                               material=pyfds_amd.AcousticMaterial(1500.0, 1000.0))
+    fld.pressure.values = np.exp(-0.01 * (np.arange(700) - 300.0) ** 2)
+    fld.line_shape = (2, 64, 16)
+    tile, _, table = autotune.tune_field(fld, steps=60, use_cache=False)
+    run = fld._runner()
+    assert '-1,0,50' in table and tile == -1 and run.lib.fds_engine(run.ctx) == 2
