@@ -90,7 +90,7 @@ class ThermoAcoustic1D(cp.SynchronizedFields):
         for f in (acoustic, thermal):
             if not f._device_loop_ok() or 'material_vector' in vars(f):
                 return None
-            if getattr(f, 'tile', None) is not None or getattr(f, 'strip_height', None):
+            if getattr(f, 'tile', None) not in (None, -1) or getattr(f, 'strip_height', None):
                 return None
         if getattr(acoustic, 'form', 'fp64') != getattr(thermal, 'form', 'fp64'):
             return None

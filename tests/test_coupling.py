@@ -439,3 +439,15 @@ def test_fields_leave_a_coupling_for_their_own_engine():
                    + [np.array(ac.pressure.outputs[0].signals)])
     for a, b in zip(*res):
         np.testing.assert_array_equal(a, b)
+
+
+def test_thermoacoustic_fields_on_tile_minus_one_stay_device_coupled():
+    """Tile -1 is the default engine, which the device-coupled loop runs on (a tuned field has it
+    set); a tile of the table takes the host protocol."""
+    fld, _, _, _ = cs.ta1d(fds, 1)
+    assert fld._device_coupling() is not None
+    for f in fld.fields:
+        f.tile = -1
+    assert fld._device_coupling() is not None
+    fld.fields[0].tile = 5
+    assert fld._device_coupling() is None
