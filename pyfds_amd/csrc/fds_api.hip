@@ -544,7 +544,8 @@ int choose_tiles(fds_ctx *c) {
       cfg_threads = 0;
       if (c->strip_rows <= 0 && c->n > fds::kLineWave) {
         const fds::LineLayout l = fds::line_layout(
-            c->n, c->lossy && c->family == kAcoustic, c->family == kNonlinear);
+            c->n, c->lossy && c->family == kAcoustic, c->family == kNonlinear,
+            c->family == kThermal, is_kahan(c));
         cfg_threads = fds::kLineWave;
         cfg_ghost = l.ghost;
         cpt_req = l.cpt;
